@@ -112,6 +112,8 @@ struct sld_ctx {
         bool ready = false;
         double theta[sld::kNParam] = {};
         sld::ModelTab tab{};
+        std::shared_ptr<const sld::ModelBridge> bridge;
+        double* d_bridge = nullptr;
         double *d_r = nullptr, *d_rd = nullptr, *d_h = nullptr;
         double *d_rho = nullptr, *d_fp = nullptr, *d_Q = nullptr;
         double *d_F = nullptr, *d_H = nullptr, *d_gE = nullptr, *d_gF = nullptr, *d_gH = nullptr;
@@ -1879,6 +1881,8 @@ int sld_model_set_params(sld_ctx* c, const double* theta) {
     auto& m = c->model;
     const int N = c->D.N;
     if (!m.d_r) {
+        m.bridge = model_bridge(c->prm.rcut_max);
+        TRY(upload_vec(c, &m.d_bridge, m.bridge->q));
         TRY(dalloc(c, &m.d_r, (size_t)kNInput * kMRStride));
         TRY(dalloc(c, &m.d_rd, (size_t)kNInput * kMRDStride));
         TRY(dalloc(c, &m.d_h, (size_t)kNInput * kMHStride));
@@ -1897,17 +1901,16 @@ int sld_model_set_params(sld_ctx* c, const double* theta) {
         TRY(dalloc(c, &m.d_grad, kNParam));
         TRY(dalloc(c, &m.d_part, (size_t)nblk(N, 256) * kNParam));
     }
-    ModelHostTables t;
-    build_model_tables(theta, c->prm.rcut_max, t);
-    HIPCHK(c, hipMemcpyAsync(m.d_r, t.r.data(), t.r.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(m.d_rd, t.rd.data(), t.rd.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(m.d_h, t.h.data(), t.h.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    const ModelCoef mc = model_coef(theta, c->prm.rcut_max, *m.bridge);
+    LAUNCH(c, k_model_tab_r, nblk(kNInput - 1, 255), 256, mc, (const double*)m.d_bridge, m.d_r);
+    LAUNCH(c, k_model_tab_rd, nblk(kNInput, 64), 64, mc, (const double*)m.d_bridge, m.d_rd);
+    LAUNCH(c, k_model_tab_h, nblk(kNInput, 256), 256, mc, m.d_h);
     HIPCHK(c, hipStreamSynchronize(c->stream));
     m.tab.r = m.d_r;
     m.tab.rd = m.d_rd;
     m.tab.h = m.d_h;
-    m.tab.in_over_rmax = t.in_over_rmax;
-    m.tab.in_over_rhomax = t.in_over_rhomax;
+    m.tab.in_over_rmax = (double)kNInput / mc.rmax;
+    m.tab.in_over_rhomax = (double)kNInput / mc.rhomax;
     for (int k = 0; k < 4; ++k) m.tab.L[k] = theta[P_LA + k];
     std::copy(theta, theta + kNParam, m.theta);
     m.ready = true;

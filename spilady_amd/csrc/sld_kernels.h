@@ -156,6 +156,9 @@ struct ModelTab {
     double in_over_rmax, in_over_rhomax;
     double L[4];        // Landau A B C D
 };
+__global__ void k_model_tab_r(ModelCoef m, const double* bridge, double* out);
+__global__ void k_model_tab_rd(ModelCoef m, const double* bridge, double* out);
+__global__ void k_model_tab_h(ModelCoef m, double* out);
 __global__ void k_model_rho(ModelTab M, Phys P, Dev D, double* rho_out, double* fp_out);
 __global__ void k_model_forward(ModelTab M, Phys P, Dev D, const double* rho, const double* fp, const int* coff,
                                 double* F, double* H, double* partials);

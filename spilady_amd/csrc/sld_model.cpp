@@ -1,10 +1,11 @@
-// Tables of the parametric potential model (sld_model.h): the forms of
+// Host side of the parametric potential model (sld_model.h): the forms of
 // DD05.cpp:6-164 and JijFe.cpp:5-43 with their coefficients taken from the
 // parameter vector, sampled like potential_CPU.cpp:61-170 (10^6 points, the
-// 6-point central-difference derivative). Every parameter except the exchange
-// cutoff rc enters a table linearly, so the derivative of a table with respect
-// to it is the table of its basis function, built the same way; the rc
-// derivative is the table of dJ/drc at the current parameters.
+// 6-point central-difference derivative) by the device (sld_model_tab.hip).
+// Every parameter except the exchange cutoff rc enters a table linearly, so
+// the derivative of a table with respect to it is the table of its basis
+// function, built the same way; the rc derivative is the table of dJ/drc at
+// the current parameters.
 //
 // The pair term's quintic bridge (1.8 < r <= 2 A) is evaluated as the bridge
 // of the ZBL end alone plus sum_k V_k times the bridge of knot k alone. This
@@ -12,9 +13,13 @@
 // is linear in its six end values), but the closed form cancels large terms
 // and carries rounding noise of about 1e-9 of V (1e-7 of V' after the
 // 6-point derivative) that varies with V; split, the noise sits in the
-// V-independent ZBL part and the model is smooth in V_k.
+// V-independent ZBL part and the model is smooth in V_k. The nine
+// polynomials' values do not depend on theta and are made here once.
+#include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "sld_common.h"
@@ -24,20 +29,9 @@
 namespace sld {
 namespace {
 
-// knots of the density and pair splines (DD05.cpp:26-37,70-85)
+// knots of the density and pair splines (DD05.cpp:26-37,70-85), as in sld_model_tab.hip
 const double kFR[6] = {3.0, 2.8666666666666666, 2.7333333333333333, 2.6, 2.4, 2.3};
 const double kVR[8] = {4.1, 3.8, 3.5, 3.2, 2.9, 2.6, 2.4, 2.3};
-
-template <class F>
-double deriv6(F fn, double x) {
-    double dx = x / 1000e0;
-    double vp = fn(x + dx), vm = fn(x - dx);
-    double v2p = fn(x + 2 * dx), v2m = fn(x - 2 * dx);
-    double v3p = fn(x + 3 * dx), v3m = fn(x - 3 * dx);
-    return (45e0 * (vp - vm) - 9e0 * (v2p - v2m) + (v3p - v3m)) / (60e0 * dx);
-}
-
-double cube_knot(double R, double r) { return r < R ? std::pow(R - r, 3) : 0e0; }
 
 double quintic(const Bridge& b, double r) {
     using std::pow;
@@ -45,23 +39,9 @@ double quintic(const Bridge& b, double r) {
     return a[5] * pow(r, 5) + a[4] * pow(r, 4) + a[3] * pow(r, 3) + a[2] * pow(r, 2) + a[1] * r + a[0];
 }
 
-struct Model {
-    double a[6], V[8], aa, bb, JA, Jrc;
-    Bridge zbridge;           // bridge of the ZBL end alone, zero spline end
-    Bridge vbasis[8];         // bridge of each V_k alone, zero ZBL ends
-    double rhomax;
-};
-
-Model make_model(const double* th) {
-    Model m;
-    for (int k = 0; k < 6; ++k) m.a[k] = th[P_A0 + k];
-    for (int k = 0; k < 8; ++k) m.V[k] = th[P_V0 + k];
-    m.aa = th[P_AA];
-    m.bb = th[P_BB];
-    m.JA = th[P_JA];
-    m.Jrc = th[P_JRC];
+void bridge_polynomials(Bridge (&q)[9]) {
     const double x2 = 2.0;
-    m.zbridge = bridge_from_ends(zbl_ends(), 0e0, 0e0, 0e0);
+    q[0] = bridge_from_ends(zbl_ends(), 0e0, 0e0, 0e0);
     const ZblEnds zero = {0e0, 0e0, 0e0};
     for (int k = 0; k < 8; ++k) {
         double g = 0e0, dg = 0e0, d2g = 0e0;
@@ -70,58 +50,51 @@ Model make_model(const double* th) {
             dg = -3e0 * std::pow(kVR[k] - x2, 2);
             d2g = 6e0 * (kVR[k] - x2);
         }
-        m.vbasis[k] = bridge_from_ends(zero, g, dg, d2g);
+        q[1 + k] = bridge_from_ends(zero, g, dg, d2g);
     }
-    double f1 = 0e0;
-    for (int i = 0; i < 6; ++i) f1 += m.a[i] * cube_knot(kFR[i], 1e0);
-    m.rhomax = 2e0 * f1 < 1000e0 ? 1000e0 : 2e0 * f1;
-    return m;
 }
 
-double f_of(const Model& m, double r) {
-    double f = 0e0;
-    for (int i = 0; i < 6; ++i)
-        if (r < kFR[i]) f += m.a[i] * std::pow(kFR[i] - r, 3);
-    return f;
-}
+// the r of table entry n, as the device computes it
+double entry_r(double rmax, int n) { return rmax / (double)kNInput * (double)(n + 1); }
 
-double v_of(const Model& m, double r) {
-    if (r <= 1.8) return zbl_pair(r);
-    if (r <= 2.0) {
-        double v = quintic(m.zbridge, r);
-        for (int k = 0; k < 8; ++k) v += m.V[k] * quintic(m.vbasis[k], r);
-        return v;
-    }
-    double v = 0e0;
-    for (int i = 0; i < 8; ++i)
-        if (r < kVR[i]) v += m.V[i] * std::pow((kVR[i] - r), 3);
-    return v;
-}
-
-// dV/dV_k: the knot term above 2, its share of the bridge between 1.8 and 2
-double v_basis(const Model& m, int k, double r) {
-    if (r <= 1.8) return 0e0;
-    if (r <= 2.0) return quintic(m.vbasis[k], r);
-    return cube_knot(kVR[k], r);
-}
-
-double j_of(const Model& m, double r) { return r < m.Jrc ? m.JA * std::pow(1.0 - r / m.Jrc, 3) : 0e0; }
-double j_basis_a(const Model& m, double r) { return r < m.Jrc ? std::pow(1.0 - r / m.Jrc, 3) : 0e0; }
-double j_basis_rc(const Model& m, double r) {
-    return r < m.Jrc ? m.JA * 3.0 * std::pow(1.0 - r / m.Jrc, 2) * r / (m.Jrc * m.Jrc) : 0e0;
-}
-
-double bigf_of(const Model& m, double rho) {
-    if (rho >= 1e0) return -m.aa * std::sqrt(rho);
-    return -m.aa * std::sqrt(rho) - m.bb / std::log(2e0) * (1e0 - std::sqrt(rho)) * std::log(2e0 - rho);
-}
-double bigf_basis_aa(double rho) { return -std::sqrt(rho); }
-double bigf_basis_bb(double rho) {
-    if (rho >= 1e0) return 0e0;
-    return -(1e0 - std::sqrt(rho)) * std::log(2e0 - rho) / std::log(2e0);
+void fill_bridge(double rmax, ModelBridge& t) {
+    Bridge q[9];
+    bridge_polynomials(q);
+    // rows whose stencil (x +- 3x/1000) can reach (1.8, 2.0], with a margin
+    const double per = kNInput / rmax;
+    t.row0 = std::max(0, std::min(kNInput, (int)(1.8 / 1.003 * per) - 4));
+    t.nrow = std::max(0, std::min(kNInput, (int)(2.0 / 0.997 * per) + 4) - t.row0);
+    t.q.assign((size_t)std::max(t.nrow, 1) * kModelBridgeRow, 0.0);
+    auto work = [&](int a, int b) {
+        for (int k = a; k < b; ++k) {
+            const double r = entry_r(rmax, t.row0 + k);
+            const double dx = r / 1000e0;
+            const double x[7] = {r, r + dx, r - dx, r + 2 * dx, r - 2 * dx, r + 3 * dx, r - 3 * dx};
+            for (int s = 0; s < 7; ++s)
+                if (x[s] > 1.8 && x[s] <= 2.0)
+                    for (int p = 0; p < 9; ++p) t.q[((size_t)k * 7 + s) * 9 + p] = quintic(q[p], x[s]);
+        }
+    };
+    unsigned nt = std::min(std::max(std::thread::hardware_concurrency(), 1u), 16u);
+    std::vector<std::thread> th;
+    const int chunk = (t.nrow + (int)nt - 1) / (int)nt;
+    for (int a = 0; a < t.nrow; a += chunk) th.emplace_back(work, a, std::min(a + chunk, t.nrow));
+    for (auto& x : th) x.join();
 }
 
 }  // namespace
+
+std::shared_ptr<const ModelBridge> model_bridge(double rcut_max) {
+    static std::mutex mu;
+    static std::vector<std::pair<double, std::shared_ptr<const ModelBridge>>> cache;
+    std::lock_guard<std::mutex> lock(mu);
+    for (auto& e : cache)
+        if (e.first == rcut_max) return e.second;
+    auto t = std::make_shared<ModelBridge>();
+    fill_bridge(rcut_max, *t);
+    cache.emplace_back(rcut_max, t);
+    return t;
+}
 
 void model_default_params(double* th) {
     const double a[6] = {0.9332056681088162, -1.162558782567700, -0.3502026949249225,
@@ -140,59 +113,22 @@ void model_default_params(double* th) {
     th[P_LA + 3] = 0e0;
 }
 
-void build_model_tables(const double* theta, double rcut_max, ModelHostTables& t) {
-    const Model m = make_model(theta);
-    t.rmax = rcut_max;
-    t.rhomax = m.rhomax;
-    const double finput = (double)kNInput;
-    t.in_over_rmax = finput / t.rmax;
-    t.in_over_rhomax = finput / t.rhomax;
-    t.r.assign((size_t)kNInput * kMRStride, 0.0);
-    t.rd.assign((size_t)kNInput * kMRDStride, 0.0);
-    t.h.assign((size_t)kNInput * kMHStride, 0.0);
-    auto work = [&](int n0, int n1) {
-        for (int n = n0; n < n1; ++n) {
-            const double r = t.rmax / finput * (double)(n + 1);
-            const double rho = t.rhomax / finput * (double)(n + 1);
-            double* R = &t.r[(size_t)n * kMRStride];
-            R[MR_F] = f_of(m, r);
-            R[MR_DF] = deriv6([&](double x) { return f_of(m, x); }, r);
-            R[MR_V] = v_of(m, r);
-            R[MR_DV] = deriv6([&](double x) { return v_of(m, x); }, r);
-            R[MR_J] = j_of(m, r);
-            R[MR_DJ] = deriv6([&](double x) { return j_of(m, x); }, r);
-            double* D = &t.rd[(size_t)n * kMRDStride];
-            for (int k = 0; k < 6; ++k) {
-                D[2 * k] = cube_knot(kFR[k], r);
-                D[2 * k + 1] = deriv6([&](double x) { return cube_knot(kFR[k], x); }, r);
-            }
-            for (int k = 0; k < 8; ++k) {
-                D[12 + 2 * k] = v_basis(m, k, r);
-                D[12 + 2 * k + 1] = deriv6([&](double x) { return v_basis(m, k, x); }, r);
-            }
-            D[28] = j_basis_a(m, r);
-            D[29] = deriv6([&](double x) { return j_basis_a(m, x); }, r);
-            D[30] = j_basis_rc(m, r);
-            D[31] = deriv6([&](double x) { return j_basis_rc(m, x); }, r);
-            double* H = &t.h[(size_t)n * kMHStride];
-            H[MH_F] = bigf_of(m, rho);
-            H[MH_DF] = deriv6([&](double x) { return bigf_of(m, x); }, rho);
-            H[MH_AA] = bigf_basis_aa(rho);
-            H[MH_DAA] = deriv6(bigf_basis_aa, rho);
-            H[MH_BB] = bigf_basis_bb(rho);
-            H[MH_DBB] = deriv6(bigf_basis_bb, rho);
-        }
-    };
-    unsigned nt = std::thread::hardware_concurrency();
-    if (nt == 0) nt = 1;
-    if (nt > 16) nt = 16;
-    std::vector<std::thread> th;
-    int chunk = (kNInput + nt - 1) / nt;
-    for (unsigned k = 0; k < nt; ++k) {
-        int a = k * chunk, b = a + chunk < kNInput ? a + chunk : kNInput;
-        if (a < b) th.emplace_back(work, a, b);
-    }
-    for (auto& x : th) x.join();
+ModelCoef model_coef(const double* th, double rcut_max, const ModelBridge& bridge) {
+    ModelCoef m;
+    for (int k = 0; k < 6; ++k) m.a[k] = th[P_A0 + k];
+    for (int k = 0; k < 8; ++k) m.V[k] = th[P_V0 + k];
+    m.aa = th[P_AA];
+    m.bb = th[P_BB];
+    m.JA = th[P_JA];
+    m.Jrc = th[P_JRC];
+    m.as = 0.88535e0 * 0.52917720859e0 / (2e0 * std::pow(26e0, 0.23));  // DD05.cpp:45-62
+    m.ln2 = std::log(2e0);
+    double f1 = 0e0;
+    for (int i = 0; i < 6; ++i) f1 += m.a[i] * std::pow(kFR[i] - 1e0, 3);
+    m.rmax = rcut_max;
+    m.rhomax = 2e0 * f1 < 1000e0 ? 1000e0 : 2e0 * f1;
+    m.row0 = bridge.row0;
+    return m;
 }
 
 }  // namespace sld

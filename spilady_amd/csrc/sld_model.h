@@ -19,24 +19,40 @@ enum ParamIndex { P_A0 = 0, P_V0 = 6, P_AA = 14, P_BB = 15, P_JA = 16, P_JRC = 1
 
 // Columns of the model tables (10^6 entries each, the reference's sampling
 // and 6-point derivative stencil):
-//   r value table   [N][8]:  f f' V V' J J' - -
+//   r value table   [N][16]: the interpolation pair (t[n-1], t[n]) of each of f f' V V' J J', then padding:
+//                            a lookup touches one 128-byte line
 //   r derivative    [N][32]: df/da_k, df'/da_k (k<6, interleaved), dV/dV_k, dV'/dV_k (k<8),
 //                            dJ/dA dJ'/dA dJ/drc dJ'/drc
 //   rho table       [N][8]:  F F' dF/daa dF'/daa dF/dbb dF'/dbb - -
-constexpr int kMRStride = 8;
+constexpr int kMRStride = 16;
 constexpr int kMRDStride = 32;
 constexpr int kMHStride = 8;
 enum MRCol { MR_F = 0, MR_DF, MR_V, MR_DV, MR_J, MR_DJ };
 enum MHCol { MH_F = 0, MH_DF, MH_AA, MH_DAA, MH_BB, MH_DBB };
 
-struct ModelHostTables {
-    double rmax = 0, rhomax = 0, in_over_rmax = 0, in_over_rhomax = 0;
-    std::vector<double> r, rd, h;
+// The quintic bridge of the pair term at the stencil points of the rows that
+// reach it, theta-independent: row n, point s (x, x + dx, x - dx, x + 2dx, ...)
+// holds the bridge of the ZBL end alone, then that of each knot alone. Rows
+// [row0, row0 + nrow) of the r tables; points outside the bridge hold 0.
+constexpr int kModelBridgeRow = 7 * 9;
+struct ModelBridge {
+    int row0 = 0, nrow = 0;
+    std::vector<double> q;  // [nrow][7][9]
+};
+// Built on the host (16 threads) once per cutoff and process.
+std::shared_ptr<const ModelBridge> model_bridge(double rcut_max);
+
+// What the device needs to fill the tables at theta.
+struct ModelCoef {
+    double a[6], V[8], aa, bb, JA, Jrc;
+    double as, ln2;        // ZBL screening length, log 2
+    double rmax, rhomax;
+    int row0;              // first row of the bridge values
 };
 
 // The reference's parameter values (DD05.cpp, JijFe.cpp).
 void model_default_params(double* theta);
-// Tables of the model at theta, sampled on [0, rcut_max] and [0, rhomax].
-void build_model_tables(const double* theta, double rcut_max, ModelHostTables& t);
+// The coefficients of the tables at theta, sampled on [0, rcut_max] and [0, rhomax].
+ModelCoef model_coef(const double* theta, double rcut_max, const ModelBridge& bridge);
 
 }  // namespace sld

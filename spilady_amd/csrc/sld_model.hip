@@ -42,6 +42,12 @@ __device__ __forceinline__ void model_partials(const double (&v)[NK], double* pa
     }
 }
 
+// column k of the r value table at lookup n: the row holds the interpolation pair
+__device__ __forceinline__ double lerp_pair(const double* row, int k, double ratio) {
+    const double2 t = reinterpret_cast<const double2*>(row)[k];
+    return t.x * ratio + t.y * (1.0 - ratio);
+}
+
 // density and F'(rho) of every atom (calculate_rho_CPU.cpp:33-92,
 // calculate_force_energy_CPU.cpp:98-107; the Fe Landau coefficients do not
 // depend on rho)
@@ -64,7 +70,7 @@ __global__ __launch_bounds__(256) void k_model_rho(ModelTab M, Phys P, Dev D, do
             int n;
             double ratio;
             interp_index(sqrt(rsq), M.in_over_rmax, n, ratio);
-            rho += lerp_tab(M.r, kMRStride, MR_F, n, ratio);
+            rho += lerp_pair(M.r + (size_t)n * kMRStride, MR_F, ratio);
         }
     }
     int n;
@@ -101,20 +107,18 @@ __global__ __launch_bounds__(256) void k_model_forward(ModelTab M, Phys P, Dev D
             int n;
             double ratio;
             interp_index(r, M.in_over_rmax, n, ratio);
-            const double* t0 = M.r + (size_t)(n - 1) * kMRStride;
-            const double* t1 = t0 + kMRStride;
-            const double wr = 1.0 - ratio;
+            const double* row = M.r + (size_t)n * kMRStride;
             double dudr = 0.0;
             if (r < P.rcut_pot) {
-                dudr = (fpi + fp[j]) * (t0[MR_DF] * ratio + t1[MR_DF] * wr) + (t0[MR_DV] * ratio + t1[MR_DV] * wr);
-                e += 0.5 * (t0[MR_V] * ratio + t1[MR_V] * wr);
+                dudr = (fpi + fp[j]) * lerp_pair(row, MR_DF, ratio) + lerp_pair(row, MR_DV, ratio);
+                e += 0.5 * lerp_pair(row, MR_V, ratio);
             }
             if (r < P.rcut_mag) {
                 const double4 sj4 = D.s[j];
                 const double3 sj = d3(sj4);
                 const double X = dot3(si, sj) - sqrt(si_sq * sq3(sj));
-                const double J = t0[MR_J] * ratio + t1[MR_J] * wr;
-                dudr += -(t0[MR_DJ] * ratio + t1[MR_DJ] * wr) * X;
+                const double J = lerp_pair(row, MR_J, ratio);
+                dudr += -lerp_pair(row, MR_DJ, ratio) * X;
                 e += -0.5 * J * X;
                 h = add3(h, mul3(J, sj));
                 S += J * sj4.w;
@@ -167,7 +171,7 @@ __global__ __launch_bounds__(256) void k_model_q(ModelTab M, Phys P, Dev D, cons
         int n;
         double ratio;
         interp_index(r, M.in_over_rmax, n, ratio);
-        q += -dot3(sub3(gi, gj), rij) / r * lerp_tab(M.r, kMRStride, MR_DF, n, ratio);
+        q += -dot3(sub3(gi, gj), rij) / r * lerp_pair(M.r + (size_t)n * kMRStride, MR_DF, ratio);
     }
     Q[i] = q;
 }
