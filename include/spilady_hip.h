@@ -268,13 +268,13 @@ int sld_kernel_timing(sld_ctx* ctx, int* launches, double* total_ms);
  * bitwise the same under any valid shapes. */
 typedef struct {
     int spin_block;        /* core_ds sweep level: threads (one per cell) per block; 32, 64 or 128 */
-    int sweep_block;       /* core_dTe diffusion level: threads per block; 64, 128 or 256 */
+    int sweep_block;       /* core_dTe diffusion: threads of a tile's workgroup (twice as many on meshes of
+                              up to 512 tiles); 64, 128 or 256 */
     int force_block;       /* force/energy: threads (one per atom) per block; 64, 128 or 256 */
     int nbuild_cells;      /* neighbour build: link cells (one wave each) per block; 1, 2 or 4 */
     int temperature_block; /* calculate_temperature: threads (32 per cell) per block; 64, 128 or 256 */
-    int sweep_tail;        /* core_dTe diffusion: the trailing levels of each sweep with at most this many
-                              cells run in one workgroup, level after level (0: every level its own
-                              launch); 0, 2048 or 8192 */
+    int sweep_tail;        /* kept for the layout: every level of a sweep runs inside its tile's workgroup;
+                              0, 2048 or 8192 */
     int spin_lanes;        /* core_ds sweep level: lanes that share one cell's walk (the neighbour
                               gathers and field sums split among them); 1, 2 or 4 */
 } sld_shapes;

@@ -211,7 +211,41 @@ __device__ __forceinline__ double horner(const double (&c)[N], double t) {
     for (int k = N - 2; k >= 0; --k) a = fma(a, t, c[k]);
     return a;
 }
+// The same in two interleaved chains (even and odd powers), for a kernel whose
+// time is the length of its dependent chain: half the steps, one multiply more.
+template <int N>
+__device__ __forceinline__ double horner2(const double (&c)[N], double t) {
+    const double t2 = t * t;
+    double e = c[(N - 1) & ~1], o = c[(N - 2) | 1];
+#pragma unroll
+    for (int k = ((N - 1) & ~1) - 2; k >= 0; k -= 2) e = fma(e, t2, c[k]);
+#pragma unroll
+    for (int k = ((N - 2) | 1) - 2; k >= 1; k -= 2) o = fma(o, t2, c[k]);
+    return fma(o, t, e);
+}
 constexpr double kCeB = 2e-4 / kBoltz;
+
+// T(E) = sqrt(2y) G(y) / b with y = bE/3 written in E itself, the three
+// constant factors folded into the coefficients: sqrt(E) P(E)
+constexpr double const_sqrt(double x) {
+    double g = x > 1.0 ? x : 1.0;
+    for (int k = 0; k < 64; ++k) g = 0.5 * (g + x / g);
+    return g;
+}
+struct EeToTe {
+    double c[13];
+};
+constexpr EeToTe make_ee_to_te() {
+    EeToTe p{};
+    double f = const_sqrt(2.0 * kCeB / 3.0) / kCeB;
+    for (int k = 0; k < 13; ++k) {
+        p.c[k] = kAcoshExpG[k] * f;
+        f *= kCeB / 3.0;
+    }
+    return p;
+}
+constexpr EeToTe kEeToTe = make_ee_to_te();
+constexpr double kPolyEMax = 3.0 * kPolyYMax / kCeB;
 
 // tanh(x), x = bT, for the heat capacity 3 tanh(x)
 __device__ __forceinline__ double tanh_bt(double x) {
@@ -226,8 +260,20 @@ __device__ __forceinline__ double te_to_ee(double te) {
     const double e = exp(x);
     return 3.0 / kCeB * log(0.5 * (e + 1.0 / e));
 }
+// sqrt(x) for normal x far from the ends of the exponent range, to about an
+// ulp: the hardware's reciprocal square root (2^-23 or better) and two
+// Newton steps, without the library's scaling and final rounding step
+__device__ __forceinline__ double sqrt_normal(double x) {
+    const double r = __builtin_amdgcn_rsq(x);
+    double g = x * r, h = 0.5 * r;
+    const double d = fma(-h, g, 0.5);
+    g = fma(g, d, g);
+    h = fma(h, d, h);
+    return fma(fma(-g, g, x), h, g);
+}
 // T(E); outside the fitted range acosh(e^y) = y + log1p(sqrt(-expm1(-2y)))
 __device__ __forceinline__ double ee_to_te(double ee) {
+    if (ee <= kPolyEMax && ee >= 1e-200) return sqrt_normal(ee) * horner2(kEeToTe.c, ee);
     const double y = kCeB / 3.0 * ee;
     if (y <= kPolyYMax) return sqrt(2.0 * y) * horner(kAcoshExpG, y) * (1.0 / kCeB);
     return (y + log1p(sqrt(-expm1(-2.0 * y)))) / kCeB;

@@ -74,7 +74,13 @@ struct sld_ctx {
     uint64_t step_npass = 0;        // noise passes of one step
     bool capturing = false;
     int device = 0;
-    LevelSet spin_fwd, spin_bwd, dte_fwd, dte_bwd;  // over all replicas
+    LevelSet spin_fwd, spin_bwd;  // over all replicas
+    // electron diffusion: tile schedules of the forward and the backward
+    // sweep, or one of both together, and the second copy of the mesh
+    int dte_n = 0;
+    DteTiles dte[2] = {};
+    size_t dte_lds[2] = {0, 0};
+    double *d_te2 = nullptr, *d_ee2 = nullptr;
     // buffers
     double *d_prow = nullptr, *d_rhotab = nullptr;
     int *d_cl2 = nullptr, *d_cn2 = nullptr;  // second cell-list buffer
@@ -106,7 +112,7 @@ struct sld_ctx {
     std::vector<size_t> alloc_bytes;  // size of each entry of allocs
     // launch shapes of the kernels whose results do not depend on them
     // (defaults: the autotuner's choice on the 2M-atom step on MI355X)
-    sld_shapes shapes{64, 64, 256, 2, 256, 2048, 4};
+    sld_shapes shapes{64, 256, 256, 2, 256, 2048, 4};
     // parametric potential model over the replicas' frozen configurations
     struct Model {
         bool ready = false;
@@ -432,6 +438,19 @@ int do_temperature(sld_ctx* c) {
     return SLD_OK;
 }
 
+constexpr int kDteEnds = 1024;       // final-energy partials that every block of the next kernel may add
+constexpr size_t kDteLds = 60 << 10;  // dynamic LDS of a tile at most
+
+// Edge of the tiles of a sweep: even, so that tiles inside the mesh see the
+// same colouring and share their lists, and the smallest that leaves at most
+// `most` tiles: with fewer than two a compute unit the longest tile sets the
+// time, with more the closures are computed more often.
+int dte_tile_edge(const HostCells& h, int most) {
+    for (int e = 4; e < 10; e += 2)
+        if (((h.nx + e - 1) / e) * ((h.ny + e - 1) / e) * ((h.nz + e - 1) / e) <= most) return e;
+    return 10;
+}
+
 // core_dTe_CPU.cpp:47-217 with nloop = 50
 int do_dTe_launches(sld_ctx* c, double dt);
 
@@ -463,17 +482,6 @@ int do_dTe(sld_ctx* c, double dt) {
     return SLD_OK;
 }
 
-// first level of a sweep's trailing run of levels that have at most `cap`
-// cells each, worth running in one workgroup (two levels or more, at most
-// kTailMaxLev); nlev when there is none or cap is 0
-int tail_start(const LevelSet& L, int cap) {
-    const int nl = L.nlev();
-    if (cap <= 0) return nl;
-    int lt = nl;
-    while (lt > 0 && nl - lt < kTailMaxLev && L.off[lt] - L.off[lt - 1] <= cap) --lt;
-    return nl - lt >= 2 ? lt : nl;
-}
-
 int do_dTe_launches(sld_ctx* c, double dt) {
     const int nloop = 50;
     double dtl = dt / nloop;
@@ -490,61 +498,56 @@ int do_dTe_launches(sld_ctx* c, double dt) {
                  c->phys.spinlang};
     LAUNCH(c, k_dte_ab, nb, 256, h, M, c->d_part);
     // block partials: [0, nb) starting energies (k_dte_ab / k_dte_finish_ab),
-    // then the final energies of each backward level in turn
+    // then the final energies of the backward sweep's tiles
+    double* start = c->d_scal + 8;
+    double* ends = c->d_part + nb;
+    const double px = pref / h0.dx2, py = pref / h0.dy2, pz = pref / h0.dz2;
     for (int it = 0; it < nloop; ++it) {
-        int npb = 0;
-        // the sweep levels are a few microseconds each: time them as one span
+        // the sub-step's sweeps timed as one span
         hipEvent_t* ev = timing_slot(c, "k_dte_sweep");
         if (ev) {
             (void)hipEventRecord(ev[0], c->stream);
             c->ev_span = true;
         }
-        int nlaunch = 0;
-        bool reduced = false;
-        const Box& bx = c->reps[0].box;
-        const double ix2 = 1.0 / h0.dx2, iy2 = 1.0 / h0.dy2, iz2 = 1.0 / h0.dz2;
-        for (int dir = 0; dir < 2; ++dir) {
-            LevelSet& L = dir == 0 ? c->dte_fwd : c->dte_bwd;
-            const int lt = tail_start(L, c->shapes.sweep_tail);
-            for (int l = 0; l < lt; ++l) {
-                int n = L.off[l + 1] - L.off[l];
-                double* part = dir == 1 ? c->d_part + (size_t)nb + npb : nullptr;
-                const int bs = c->shapes.sweep_block;
-                LAUNCH(c, k_dte_sweep, nblk(n, bs), bs, L.d_cells + L.off[l], n, pref, ix2, iy2, iz2, bx.nx,
-                       bx.ny, bx.nz, c->D.Te, c->D.Ee, part);
-                if (dir == 1) npb += nblk(n, 64);  // one partial per wave
-                nlaunch += n > 0;
-            }
-            if (lt < L.nlev()) {
-                // the small trailing levels in one workgroup; after the
-                // backward sweep's, the same block adds the sub-step's totals
-                SweepTail T{};
-                T.nlev = L.nlev() - lt;
-                for (int l = lt; l <= L.nlev(); ++l) T.off[l - lt] = L.off[l];
-                for (int l = lt; l < L.nlev(); ++l) {
-                    T.poff[l - lt] = npb;
-                    if (dir == 1) npb += nblk(L.off[l + 1] - L.off[l], 64);
-                }
-                double* part = dir == 1 ? c->d_part + (size_t)nb : nullptr;
-                LAUNCH(c, k_dte_tail, 1, 1024, L.d_cells, T, pref, ix2, iy2, iz2, bx.nx, bx.ny, bx.nz, c->D.Te,
-                       c->D.Ee, part, (const double*)c->d_part, nb, (const double*)(c->d_part + nb),
-                       dir == 1 ? npb : 0, dir == 1 ? c->d_scal + 8 : nullptr);
-                reduced = dir == 1;
-                nlaunch += 1;
-            }
+        for (int k = 0; k < c->dte_n; ++k) {
+            const DteTiles& S = c->dte[k];
+            const bool first = k == 0, last = k == c->dte_n - 1;
+            // with at most two tiles a compute unit a tile gets twice the waves
+            // (41^3 cells: 28.5 us a sub-step against 29.9; 69^3 in 729 tiles: 50.5 against 45.0)
+            const int bs = c->shapes.sweep_block * (S.ntile <= 512 ? 2 : 1);
+            DteSweepArgs A{px, py, pz, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr};
+            A.Tin = first ? c->D.Te : c->d_te2;
+            A.Ein = first ? c->D.Ee : c->d_ee2;
+            // the sub-step's end needs the energies only
+            A.Tout = last ? nullptr : c->d_te2;
+            A.Eout = first ? c->d_ee2 : c->D.Ee;
+            A.ends = last ? ends : nullptr;
+            A.pa = c->d_part;
+            A.na = nb;
+            A.start = first ? start : nullptr;
+            hipLaunchKernelGGL(k_dte_sweep, dim3(xcd_grid(S.ntile) + (first ? 1 : 0)), dim3(bs), c->dte_lds[k], c->stream, S,
+                               A);
+            HIPCHK(c, hipGetLastError());
         }
+        const double* Eswept = c->dte_n == 1 ? c->d_ee2 : c->D.Ee;
         if (ev) {
             c->ev_span = false;
             (void)hipEventRecord(ev[1], c->stream);
-            c->ev_launches[(ev - c->ev_pool.data()) / 2] = nlaunch;
+            c->ev_launches[(ev - c->ev_pool.data()) / 2] = c->dte_n;
         }
-        if (!reduced)
-            LAUNCH(c, k_reduce2, 1, 1024, (const double*)c->d_part, nb, (const double*)(c->d_part + nb), npb,
-                   c->d_scal + 8);
+        // up to kDteEnds partials every block of the next kernel adds them
+        // itself (at most four loads a thread); more are reduced first
+        const double* ep = ends;
+        int ne = c->dte[c->dte_n - 1].ntile;
+        if (ne > kDteEnds) {
+            TRY(reduce(c, ne, 1, c->d_scal + 9, nb));
+            ep = c->d_scal + 9;
+            ne = 1;
+        }
         if (it + 1 < nloop)
-            LAUNCH(c, k_dte_finish_ab, nb, 256, h, M, (const double*)(c->d_scal + 8), 1, c->d_part);
+            LAUNCH(c, k_dte_finish_ab, nb, 256, h, M, Eswept, (const double*)start, ep, ne, c->d_part);
         else
-            LAUNCH(c, k_dte_finish, nb, 256, h, M, (const double*)(c->d_scal + 8), 1);
+            LAUNCH(c, k_dte_finish, nb, 256, h, M, Eswept, (const double*)start, ep, ne);
     }
     return SLD_OK;
 }
@@ -939,26 +942,50 @@ int upload_levels(sld_ctx* c, LevelSet& L) {
     return SLD_OK;
 }
 
-// The electron sweep reads its cells as packed coordinates ix | iy << 10 |
-// iz << 20, which spares the stencil three integer divisions. The electron
-// mesh exists on single-system contexts only; batched ones upload plain
-// indices, which no sweep reads.
-int upload_dte_levels(sld_ctx* c, LevelSet& L) {
-    if (c->R == 1) {
-        const HostCells& hc = c->rh[0].hc;
-        if (hc.nx > 1023 || hc.ny > 1023 || hc.nz > 1023)
-            return set_err(c, SLD_ERR_CAPACITY, "the electron mesh needs at most 1023 link cells per side");
-        std::vector<int> packed(L.cells.size());
-        for (size_t k = 0; k < L.cells.size(); ++k) {
-            const int cell = L.cells[k];
-            const int ix = cell % hc.nx, iy = (cell / hc.nx) % hc.ny, iz = cell / (hc.nx * hc.ny);
-            packed[k] = ix | (iy << 10) | (iz << 20);
+// The tile schedules of the electron diffusion (single-system contexts).
+int upload_dte_schedules(sld_ctx* c) {
+    const HostCells& hc = c->rh[0].hc;
+    if (hc.nx > 1023 || hc.ny > 1023 || hc.nz > 1023)
+        return set_err(c, SLD_ERR_CAPACITY, "the electron mesh needs at most 1023 link cells per side");
+    if (!c->phys.eltemp) return SLD_OK;
+    std::vector<int> group(hc.C);
+    const ReplicaHost& h = c->rh[0];
+    for (size_t g = 0, k = 0; g < h.group_size.size(); ++g)
+        for (int q = 0; q < h.group_size[g]; ++q) group[h.group_cells[k++]] = (int)g;
+    // Both sweeps in one launch save a launch's latency and a pass over the
+    // mesh and compute the larger closure: kept where that is small, on meshes
+    // of few levels (40^3 cells, 8 levels: 17.4 us a sub-step against 20.0;
+    // 100^3: 70 against 74) and on small ones (7^3: 22.7 against 25.7;
+    // 33 x 25 x 10: 22.8 against 23.6). 41^3 cells, 36 levels: 31.9 against 28.5.
+    constexpr int kFewLevels = 16, kSmallMesh = 10000;
+    auto make = [&](DteSweeps sw, int e, int most_levels, DteSchedule& S) {
+        return dte_schedule(hc.nx, hc.ny, hc.nz, group, sw, e, e, e, most_levels, S) &&
+               8 * ((size_t)S.max_slot + S.max_upd) <= kDteLds;
+    };
+    std::vector<DteSchedule> sch(1);
+    if (!make(kDteBoth, dte_tile_edge(hc, 512), hc.C <= kSmallMesh ? kDteMaxLev : kFewLevels, sch[0])) {
+        sch.resize(2);
+        int e = dte_tile_edge(hc, 768);
+        while (!(make(kDteForward, e, kDteMaxLev, sch[0]) && make(kDteBackward, e, kDteMaxLev, sch[1]))) {
+            if (e == 1) return set_err(c, SLD_ERR_CAPACITY, "the electron mesh has no tile schedule");
+            --e;
         }
-        TRY(upload_vec(c, &L.d_cells, packed));
-    } else {
-        TRY(upload_vec(c, &L.d_cells, L.cells));
     }
-    TRY(upload_vec(c, &L.d_off, L.off));
+    c->dte_n = (int)sch.size();
+    for (int k = 0; k < c->dte_n; ++k) {
+        const DteSchedule& S = sch[k];
+        DteTile* tile = nullptr;
+        DteUpdate* upd = nullptr;
+        int32_t *slot = nullptr, *lev = nullptr;
+        TRY(upload_vec(c, &tile, S.tile));
+        TRY(upload_vec(c, &upd, S.upd));
+        TRY(upload_vec(c, &slot, S.slot));
+        TRY(upload_vec(c, &lev, S.lev));
+        c->dte[k] = DteTiles{tile, (const uint4*)upd, slot, lev, (int)S.tile.size(), S.max_slot};
+        c->dte_lds[k] = 8 * ((size_t)S.max_slot + S.max_upd);
+    }
+    TRY(dalloc(c, &c->d_te2, hc.C));
+    TRY(dalloc(c, &c->d_ee2, hc.C));
     return SLD_OK;
 }
 
@@ -1212,7 +1239,7 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
     // (links_CPU.cpp:37-50); initial lists with each atom pushed at the head in
     // ascending index, so a list holds its atoms in descending index (:53-81)
     std::vector<int> cell(N, 0), cn(C, 0), cl((size_t)C * kCellCap, 0), cslot(N, 0);
-    std::vector<LevelSet> sf(nrep), sb(nrep), tf(nrep), tb(nrep);
+    std::vector<LevelSet> sf(nrep), sb(nrep);
     for (int r = 0; r < nrep; ++r) {
         const Rep& R = c->reps[r];
         ReplicaHost& h = c->rh[r];
@@ -1270,11 +1297,8 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
         greedy_groups(hc, h.group_size, h.group_cells, group_of);
         int all26[26];
         for (int k = 0; k < 26; ++k) all26[k] = k;
-        const int faces[6] = {0, 13, 2, 14, 12, 15};
         make_levels(hc, h.group_size, h.group_cells, group_of, all26, 26, false, sf[r]);
         make_levels(hc, h.group_size, h.group_cells, group_of, all26, 26, true, sb[r]);
-        make_levels(hc, h.group_size, h.group_cells, group_of, faces, 6, false, tf[r]);
-        make_levels(hc, h.group_size, h.group_cells, group_of, faces, 6, true, tb[r]);
     }
     for (int cc = 0; cc < C; ++cc)
         for (int q = 0; q < cn[cc]; ++q) cslot[cl[(size_t)cc * kCellCap + q]] = cc * kCellCap + q;
@@ -1286,8 +1310,6 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
     HIPCHK(c, hipStreamSynchronize(c->stream));
     merge_levels(sf, c->reps, c->spin_fwd);
     merge_levels(sb, c->reps, c->spin_bwd);
-    merge_levels(tf, c->reps, c->dte_fwd);
-    merge_levels(tb, c->reps, c->dte_bwd);
     // A wave of the spin sweep walks as many atoms as its fullest cell holds,
     // and the cells of one level are independent, so each level lists its
     // cells by descending starting atom count (stable: neighbouring cells stay
@@ -1299,8 +1321,7 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
                              [&](int a, int b) { return cn[a] > cn[b]; });
     TRY(upload_levels(c, c->spin_fwd));
     TRY(upload_levels(c, c->spin_bwd));
-    TRY(upload_dte_levels(c, c->dte_fwd));
-    TRY(upload_dte_levels(c, c->dte_bwd));
+    if (nrep == 1) TRY(upload_dte_schedules(c));
 
     // electron temperatures (map_cells.cpp:128-159)
     if (P0.eltemp) {
@@ -1697,7 +1718,7 @@ namespace {
 constexpr int kNShape = 7;
 const int kShapeCand[kNShape][3] = {{32, 64, 128}, {64, 128, 256}, {64, 128, 256}, {1, 2, 4}, {64, 128, 256},
                                     {0, 2048, 8192}, {1, 2, 4}};
-// the kernel each shape is timed on (the sweep span covers the tail launches)
+// the kernel each shape is timed on
 const char* kShapeKernel[kNShape] = {"k_spin_phase", "k_dte_sweep", "k_force", "k_nbuild", "k_temperature",
                                      "k_dte_sweep", "k_spin_phase"};
 

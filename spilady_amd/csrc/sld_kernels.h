@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "sld_device.h"
+#include "sld_dte_plan.h"
 #include "sld_model.h"
 
 namespace sld {
@@ -61,8 +62,7 @@ struct Dev {
     int* err;                  // error flag bits
 };
 
-// The electron mesh as the core_dTe sub-step kernels read it: only what they
-// use, since a 2M-atom step launches about 100 of them and 3,600 sweeps.
+// The electron mesh as the core_dTe sub-step kernels read it.
 struct Mesh {
     double *Te, *Ee;
     const double *Gel, *Ges, *Tl, *TsL;
@@ -118,28 +118,32 @@ __global__ void k_dp_scale(Phys P, Dev D, const double* scal);
 __global__ void k_dr(double dt, Phys P, Dev D);
 __global__ void k_temperature(Tables T, Phys P, Dev D);
 __global__ void k_dte_ab(double h, Mesh M, double* partials);
-// the arguments are the few the stencil reads: one of these launches per
-// level and sub-step, 3,600 per 2M-atom step
-// cells: the level's cells as packed coordinates ix | iy << 10 | iz << 20;
-// idx2, idy2, idz2: reciprocals of the squared cell edges (the stencil
-// multiplies by them where the reference divides)
-__global__ void k_dte_sweep(const int* cells, int ncell, double pref, double idx2, double idy2,
-                            double idz2, int nx, int ny, int nz, double* Te, double* Ee, double* partials);
-__global__ void k_reduce2(const double* pa, int na, const double* pb, int nb, double* out);
-// the trailing small levels of a C sweep, run by one workgroup: level l of
-// the run holds entries [off[l], off[l + 1]) of the sweep's level list, and
-// its backward-sweep partials start at poff[l]
-constexpr int kTailMaxLev = 32;
-struct SweepTail {
-    int nlev;
-    int off[kTailMaxLev + 1];
-    int poff[kTailMaxLev];
+// the C diffusion sweeps over the tiles of a schedule. Tout (may be null),
+// Eout: the tile's own cells; ends (may be null): their final energies, one
+// partial per tile; start (may be null): receives the sum of the na
+// starting-energy partials pa, made by a block past the tiles.
+// px, py, pz: the step's prefactor over the squared cell edges
+struct DteTiles {
+    const DteTile* tile;
+    const uint4* upd;        // DteUpdate
+    const int32_t* slot;
+    const int32_t* lev;
+    int ntile, max_slot;
 };
-__global__ void k_dte_tail(const int* cells, SweepTail T, double pref, double idx2, double idy2, double idz2,
-                           int nx, int ny, int nz, double* Te, double* Ee, double* partials, const double* pa,
-                           int na, const double* pb, int nb, double* out);
-__global__ void k_dte_finish(double h, Mesh M, const double* xp, int nxp);
-__global__ void k_dte_finish_ab(double h, Mesh M, const double* xp, int nxp, double* partials);
+struct DteSweepArgs {
+    double px, py, pz;
+    const double *Tin, *Ein;
+    double *Tout, *Eout, *ends;
+    const double* pa;
+    int na;
+    double* start;
+};
+__global__ void k_dte_sweep(DteTiles S, DteSweepArgs A);
+// E: the energies the sweeps left; start: the sub-step's starting energy;
+// ends: nend partials of its final one
+__global__ void k_dte_finish(double h, Mesh M, const double* E, const double* start, const double* ends, int nend);
+__global__ void k_dte_finish_ab(double h, Mesh M, const double* E, const double* start, const double* ends, int nend,
+                                double* partials);
 __global__ void k_obs_atoms(Tables T, Phys P, Dev D, double* partials, int scan_spin);
 __global__ void k_obs_cells(Dev D, double* partials);
 __global__ void k_renorm(Dev D, const double* err, double* partials);

@@ -4,8 +4,9 @@
 // build + density, force), one thread per link cell for everything that the
 // reference runs as a sequential walk down a cell's list (spin sweeps,
 // Langevin momentum with local collective motion, cell temperatures).
-// Group-ordered sweeps are launched one dependency level at a time by the
-// host; within a launch no two cells interact.
+// The spin sweeps are launched one dependency level at a time by the host;
+// within a launch no two cells interact. The electron diffusion sweeps run all
+// their levels inside tiles of the mesh.
 #include <hip/hip_runtime.h>
 
 #include "../../include/spilady_hip.h"
@@ -1296,134 +1297,132 @@ __global__ __launch_bounds__(256) void k_dte_ab(double h, Mesh M, double* partia
     block_partials<1>(acc, partials);
 }
 
-// one dependency level of the C diffusion sweep (core_dTe_CPU.cpp:155-197).
-// The reference recomputes E(Te) of the cell first; the stored Ee of the
-// cell's last update is that value up to one rounding. The six face
-// neighbours (map_cells.cpp slots 0/13, 2/14, 12/15) come from the cell index.
-// In the backward sweep every cell is updated exactly once, last, so the
-// launch also leaves partials of the final energies (partials != null), one
-// per wave of 64 level entries: the sums do not depend on the block size.
-// the update of one cell of a C-sweep level, given as packed coordinates
-// ix | iy << 10 | iz << 20; returns its new Ee
-__device__ __forceinline__ double dte_cell_update(int pk, double pref, double idx2, double idy2, double idz2, int nx,
-                                                  int ny, int nz, double* Te, double* Ee) {
-    const int sl = nx * ny;
-    const int ix = pk & 1023, iy = (pk >> 10) & 1023, iz = pk >> 20;
-    const int c = ix + iy * nx + iz * sl;
-    const int xm = ix == 0 ? nx - 1 : ix - 1, xp = ix + 1 == nx ? 0 : ix + 1;
-    const int ym = iy == 0 ? ny - 1 : iy - 1, yp = iy + 1 == ny ? 0 : iy + 1;
-    const int zm = iz == 0 ? nz - 1 : iz - 1, zp = iz + 1 == nz ? 0 : iz + 1;
-    const int row = iy * nx + iz * sl;
-    const double tc = Te[c];
-    const double txm = Te[xm + row], txp = Te[xp + row];
-    const double tym = Te[ix + ym * nx + iz * sl], typ = Te[ix + yp * nx + iz * sl];
-    const double tzm = Te[ix + iy * nx + zm * sl], tzp = Te[ix + iy * nx + zp * sl];
-    double ee = Ee[c];
-    ee += pref * ((txp + txm - 2.0 * tc) * idx2 + (typ + tym - 2.0 * tc) * idy2 + (tzp + tzm - 2.0 * tc) * idz2);
-    Ee[c] = ee;
-    Te[c] = ee_to_te(ee);
-    return ee;
-}
-
-__global__ __launch_bounds__(256) void k_dte_sweep(const int* cells, int ncell, double pref, double idx2,
-                                                   double idy2, double idz2, int nx, int ny, int nz, double* Te,
-                                                   double* Ee, double* partials) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    double acc[1] = {0.0};
-    if (t < ncell) acc[0] = dte_cell_update(cells[t], pref, idx2, idy2, idz2, nx, ny, nz, Te, Ee);
-    if (partials) {
-        const double v = wave_sum(acc[0]);
-        if ((threadIdx.x & 63) == 0) partials[t >> 6] = v;
-    }
-}
-
-// the two totals of a sub-step (see k_reduce2) by one block of 1024 threads
-__device__ __forceinline__ void reduce2_block(const double* pa, int na, const double* pb, int nb, double* out) {
-    __shared__ double sh[2][16];
-    const int t = threadIdx.x;
-    double a = 0.0, e = 0.0;
-    // both arrays' loads in flight together; each array's terms are added in
-    // the order t, t + 1024, ...
-    const int nmax = na > nb ? na : nb;
-    for (int k0 = t; k0 < nmax; k0 += 8 * 1024) {
-        double v[8], w[8];
+// The C diffusion sweeps (core_dTe_CPU.cpp:155-197), one workgroup per tile of
+// the mesh (sld_dte_plan.h): the temperatures of the tile's cells, of their
+// closure and of what those read come into LDS, the levels of the schedule
+// run there with a workgroup barrier between them, and the tile writes its
+// own cells to the other copy of the mesh, which no tile of the launch reads.
+// The reference recomputes E(Te) of a cell first; the stored Ee of the cell's
+// last update is that value up to one rounding.
+//
+// A sweep is a chain of up to 20 dependent cell updates whatever the mesh
+// size. A launch per level cost 3.5 us each; here a level costs one LDS round
+// trip, the update's FP64 chain and a barrier, 0.2 us.
+// The energy partials are one per tile: its cells in slot order, 64 at a
+// time, so the sum does not depend on the block size.
+__global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
+    extern __shared__ double sT[];
+    __shared__ double sp[kDteMaxSlot / 64 + 1];
+    const int t = threadIdx.x, B = blockDim.x, lane = t & 63;
+    if ((int)blockIdx.x == ((S.ntile + 7) & ~7)) {  // the block past the tiles adds the starting energies
+        if (t < 64) {
+            double a = 0.0;
+            for (int k0 = t; k0 < A.na; k0 += 8 * 64) {
+                double v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            v[u] = k0 + u * 1024 < na ? pa[k0 + u * 1024] : 0.0;
-            w[u] = k0 + u * 1024 < nb ? pb[k0 + u * 1024] : 0.0;
-        }
+                for (int u = 0; u < 8; ++u) v[u] = k0 + u * 64 < A.na ? A.pa[k0 + u * 64] : 0.0;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            a += v[u];
-            e += w[u];
-        }
-    }
-    a = wave_sum(a);
-    e = wave_sum(e);
-    if ((t & 63) == 0) {
-        sh[0][t >> 6] = a;
-        sh[1][t >> 6] = e;
-    }
-    __syncthreads();
-    if (t == 0) {
-        double A = 0.0, E = 0.0;
-        for (int w = 0; w < 16; ++w) {
-            A += sh[0][w];
-            E += sh[1][w];
-        }
-        out[0] = A;
-        out[1] = E;
-    }
-}
-
-// The trailing small levels of a C sweep in one workgroup of 1024 threads:
-// level after level, separated by workgroup barriers (all of the block's
-// waves share one compute unit and its write-through L1, so a barrier makes
-// one level's stores visible to the next level's loads). Each cell update
-// and each backward-sweep partial (one per 64 entries of a level, at
-// T.poff[level] + entry / 64) is exactly what a k_dte_sweep launch per level
-// would produce. With out != null the block then adds the sub-step's two
-// totals from pa[0, na) and pb[0, nb), as k_reduce2 does.
-__global__ __launch_bounds__(1024) void k_dte_tail(const int* cells, SweepTail T, double pref, double idx2,
-                                                   double idy2, double idz2, int nx, int ny, int nz, double* Te,
-                                                   double* Ee, double* partials, const double* pa, int na,
-                                                   const double* pb, int nb, double* out) {
-    const int t = threadIdx.x;
-    for (int l = 0; l < T.nlev; ++l) {
-        const int o = T.off[l], n = T.off[l + 1] - o;
-        for (int e0 = 0; e0 < n; e0 += 1024) {
-            const int e = e0 + t;
-            double acc = 0.0;
-            if (e < n) acc = dte_cell_update(cells[o + e], pref, idx2, idy2, idz2, nx, ny, nz, Te, Ee);
-            if (partials) {
-                const double v = wave_sum(acc);
-                if ((t & 63) == 0 && e < n) partials[T.poff[l] + (e >> 6)] = v;
+                for (int u = 0; u < 8; ++u) a += v[u];
             }
+            a = wave_sum(a);
+            if (t == 0) A.start[0] = a;
         }
+        return;
+    }
+    const int tl = (int)(blockIdx.x & 7) * ((S.ntile + 7) >> 3) + (int)(blockIdx.x >> 3);  // see xcd_block
+    if (tl >= S.ntile) return;
+    const DteTile T = S.tile[tl];
+    const uint4* upd = S.upd + T.upd0;
+    const int32_t* slot = S.slot + T.slot0;
+    const int bound = S.lev[T.lev0 + lane];  // lane l: first update of level l
+    double* sE = sT + S.max_slot;
+    constexpr int U = 4;  // slots of a thread in flight
+    for (int s0 = t; s0 < T.nslot; s0 += U * B) {
+        int c[U];
+        double a[U], e[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) c[u] = T.origin + (slot[min(s0 + u * B, T.nslot - 1)] >> 1);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            a[u] = A.Tin[c[u]];
+            e[u] = s0 + u * B < T.nupd ? A.Ein[c[u]] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (s0 + u * B < T.nslot) sT[s0 + u * B] = a[u];
+            if (s0 + u * B < T.nupd) sE[s0 + u * B] = e[u];
+        }
+    }
+    // one update (core_dTe_CPU.cpp:161-190)
+    auto update = [&](const uint4 d) {
+        char* q = reinterpret_cast<char*>(sT);
+        auto at = [&](uint32_t o) -> double& { return *reinterpret_cast<double*>(q + o); };
+        const uint32_t self = d.x & 0xffffu;
+        const double txp = at(d.x >> 16), txm = at(d.y & 0xffffu);
+        const double typ = at(d.y >> 16), tym = at(d.z & 0xffffu);
+        const double tzp = at(d.z >> 16), tzm = at(d.w & 0xffffu);
+        const double tc = at(self);
+        double& E = *reinterpret_cast<double*>(reinterpret_cast<char*>(sE) + self);
+        double ee = E;
+        ee = fma(fma(-2.0, tc, txp + txm), A.px, ee);
+        ee = fma(fma(-2.0, tc, typ + tym), A.py, ee);
+        ee = fma(fma(-2.0, tc, tzp + tzm), A.pz, ee);
+        E = ee;
+        at(self) = ee_to_te(ee);
+    };
+    // a thread's first update of the next level is requested one level ahead
+    // (straight-line code: the wait before an update leaves the request in
+    // flight)
+    uint4 d = upd[min(t, T.nent - 1)];
+    __syncthreads();
+    int lo = 0;
+    for (int l = 0; l < T.nlev; ++l) {
+        const int hi = __builtin_amdgcn_readlane(bound, l + 1);
+        const uint4 nx = upd[min(hi + t, T.nent - 1)];
+        if (lo + t < hi) update(d);
+        if (hi - lo > B)
+            for (int k = lo + B + t; k < hi; k += B) update(upd[k]);
+        d = nx;
+        lo = hi;
         __syncthreads();
     }
-    if (out) reduce2_block(pa, na, pb, nb, out);
-}
-
-// the two totals of a sub-step: out[0] = sum of the starting-energy partials,
-// out[1] = sum of the final-energy partials; one block of 1024 threads in a
-// fixed order, independent of how the partials were produced. Each thread
-// keeps eight loads of each array in flight, a wave sums by shuffles and
-// thread 0 adds the 16 wave sums in order.
-__global__ __launch_bounds__(1024) void k_reduce2(const double* pa, int na, const double* pb, int nb,
-                                                  double* out) {
-    reduce2_block(pa, na, pb, nb, out);
-}
-
-// starting and final totals of a sub-step from n partial pairs (xp[0..n):
-// start, xp[n..2n): end), summed in a fixed order by every thread
-__device__ __forceinline__ double dte_factor(const double* xp, int n) {
-    double st = 0.0, en = 0.0;
-    for (int k = 0; k < n; ++k) {
-        st += xp[k];
-        en += xp[n + k];
+    const int nch = (T.nupd + 63) >> 6;
+    for (int q = t >> 6; q < nch; q += B >> 6) {
+        const int s = q * 64 + lane;
+        const int32_t c = s < T.nupd ? slot[s] : 0;
+        const bool own = (c & 1) != 0;
+        const double ee = own ? sE[s] : 0.0;
+        if (own) {
+            A.Eout[T.origin + (c >> 1)] = ee;
+            if (A.Tout) A.Tout[T.origin + (c >> 1)] = sT[s];
+        }
+        if (A.ends) {
+            const double v = wave_sum(ee);
+            if (lane == 0) sp[q] = v;
+        }
     }
-    return st / en;
+    if (A.ends) {
+        __syncthreads();
+        if (t < 64) {
+            double a = 0.0;
+            for (int k = t; k < nch; k += 64) a += sp[k];
+            a = wave_sum(a);
+            if (t == 0) A.ends[tl] = a;
+        }
+    }
+}
+
+// the final energy of a sub-step from its n partials, by every block of 256
+// threads for itself in the same fixed order
+__device__ __forceinline__ double dte_end_total(const double* p, int n) {
+    __shared__ double sh[4];
+    const int t = threadIdx.x;
+    double a = 0.0;
+    for (int k = t; k < n; k += 256) a += p[k];
+    a = wave_sum(a);
+    if ((t & 63) == 0) sh[t >> 6] = a;
+    __syncthreads();
+    return (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
 // end of one sub-step and start of the next: renormalise (core_dTe_CPU.cpp:199-216),
@@ -1431,15 +1430,17 @@ __device__ __forceinline__ double dte_factor(const double* xp, int n) {
 // In registers: the Te and Ee that the first A(h) leaves are overwritten by
 // the second before anything reads them, so only the final values are
 // computed and stored (same arithmetic as B, A, A, B applied in turn).
-__global__ __launch_bounds__(256) void k_dte_finish_ab(double h, Mesh M, const double* xp, int nxp,
-                                                       double* partials) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_dte_finish_ab(double h, Mesh M, const double* E, const double* start,
+                                                       const double* ends, int nend, double* partials) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    const int cc = c < M.C ? c : M.C - 1;
+    const double G = dte_G(cc, h, M);
+    const double dE = dte_dE(M, cc);
+    const double e0 = E[cc];
+    const double f = start[0] / dte_end_total(ends, nend);
     double acc[1] = {0.0};
     if (c < M.C) {
-        const double f = dte_factor(xp, nxp);
-        const double G = dte_G(c, h, M);
-        const double dE = dte_dE(M, c);
-        double T = ee_to_te(M.Ee[c] * f);
+        double T = ee_to_te(e0 * f);
         T = dte_rk4(T, G);                  // B(h) ends the sub-step
         double ee = te_to_ee(T) + h * dE;      // A(h) ends it
         ee += h * dE;                          // A(h) starts the next
@@ -1453,13 +1454,12 @@ __global__ __launch_bounds__(256) void k_dte_finish_ab(double h, Mesh M, const d
 }
 
 // renormalise to the starting total (core_dTe_CPU.cpp:199-216), then B(h), A(h)
-__global__ __launch_bounds__(256) void k_dte_finish(double h, Mesh M, const double* xp, int nxp) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_dte_finish(double h, Mesh M, const double* E, const double* start,
+                                                    const double* ends, int nend) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    const double f = start[0] / dte_end_total(ends, nend);
     if (c >= M.C) return;
-    double f = dte_factor(xp, nxp);
-    double ee = M.Ee[c] * f;
-    M.Ee[c] = ee;
-    M.Te[c] = ee_to_te(ee);
+    M.Te[c] = ee_to_te(E[c] * f);
     dte_B(c, h, M);
     dte_A(c, h, M);
 }
