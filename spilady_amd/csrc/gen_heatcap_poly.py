@@ -6,6 +6,7 @@ mesh normally holds, for use instead of exp/log/acosh in the dTe kernels.
 With x = bT and y = bE/3 = log cosh x:
   log cosh x   = x^2 * Q(x^2)          Q analytic, nearest singularity x^2 = -pi^2/4
   tanh x       = x   * R(x^2)          R likewise
+  x coth x     = K(x^2)                K analytic, nearest singularity x^2 = -pi^2: 1/C(T) without a division
   acosh(e^y)   = sqrt(2y) * Gy(y)      Gy analytic, nearest singularities y = +-i pi
 Each factor is fitted by Chebyshev interpolation in 60-digit arithmetic
 (mpmath.chebyfit) on [0, S]; the degree is the smallest whose fit is below
@@ -37,6 +38,13 @@ def r_fn(s):                      # tanh(x) / x at s = x^2
         return mp.mpf(1)
     x = mp.sqrt(s)
     return mp.tanh(x) / x
+
+
+def k_fn(s):                      # x coth x at s = x^2
+    if s == 0:
+        return mp.mpf(1)
+    x = mp.sqrt(s)
+    return x * mp.coth(x)
 
 
 def g_fn(y):                      # acosh(e^y) / sqrt(2y)
@@ -73,9 +81,11 @@ def check(name, c, f_full, arg, hi):
 def main():
     cq, nq = fit(q_fn, mp.mpf(X_MAX) ** 2)
     cr, nr = fit(r_fn, mp.mpf(X_MAX) ** 2)
+    ck, nk = fit(k_fn, mp.mpf(X_MAX) ** 2)
     cg, ng = fit(g_fn, mp.mpf(Y_MAX))
     check("log cosh x", cq, lambda c, x: x * x * horner(c, x * x), lambda x: mp.log(mp.cosh(x)), X_MAX)
     check("tanh x", cr, lambda c, x: x * horner(c, x * x), mp.tanh, X_MAX)
+    check("x coth x", ck, lambda c, x: horner(c, x * x), lambda x: x * mp.coth(x), X_MAX)
     check("acosh(e^y)", cg, lambda c, y: np.sqrt(2 * y) * horner(c, y), lambda y: mp.acosh(mp.exp(y)), Y_MAX)
 
     def arr(name, c):
@@ -85,11 +95,11 @@ def main():
     out = os.path.join(os.path.dirname(os.path.abspath(__file__)), "heatcap_poly.h")
     with open(out, "w") as fh:
         fh.write("// Generated by gen_heatcap_poly.py: Chebyshev fits (lowest degree first) of\n"
-                 "// log cosh(x)/x^2 and tanh(x)/x in s = x^2 on [0, %r], and of\n"
+                 "// log cosh(x)/x^2, tanh(x)/x and x coth(x) in s = x^2 on [0, %r], and of\n"
                  "// acosh(e^y)/sqrt(2y) in y on [0, %r], each below 2^-56 relative.\n"
                  "#pragma once\n\nnamespace sld {\n\n" % (X_MAX * X_MAX, Y_MAX))
         fh.write(f"constexpr double kPolyXMax = {X_MAX!r};\nconstexpr double kPolyYMax = {Y_MAX!r};\n")
-        fh.write(arr("kLogCoshQ", cq) + arr("kTanhR", cr) + arr("kAcoshExpG", cg))
+        fh.write(arr("kLogCoshQ", cq) + arr("kTanhR", cr) + arr("kXCothX", ck) + arr("kAcoshExpG", cg))
         fh.write("\n}  // namespace sld\n")
     print("wrote", out)
 

@@ -225,29 +225,30 @@ __device__ __forceinline__ double horner2(const double (&c)[N], double t) {
 }
 constexpr double kCeB = 2e-4 / kBoltz;
 
-// T(E) = sqrt(2y) G(y) / b with y = bE/3 written in E itself, the three
-// constant factors folded into the coefficients: sqrt(E) P(E)
+// coefficients c[k] f g^k: a polynomial in g t times f, as one in t
+template <int N>
+struct Poly {
+    double c[N];
+};
+template <int N>
+constexpr Poly<N> scaled(const double (&c)[N], double f, double g) {
+    Poly<N> p{};
+    for (int k = 0; k < N; ++k) {
+        p.c[k] = c[k] * f;
+        f *= g;
+    }
+    return p;
+}
 constexpr double const_sqrt(double x) {
     double g = x > 1.0 ? x : 1.0;
     for (int k = 0; k < 64; ++k) g = 0.5 * (g + x / g);
     return g;
 }
-struct EeToTe {
-    double c[13];
-};
-constexpr EeToTe make_ee_to_te() {
-    EeToTe p{};
-    double f = const_sqrt(2.0 * kCeB / 3.0) / kCeB;
-    for (int k = 0; k < 13; ++k) {
-        p.c[k] = kAcoshExpG[k] * f;
-        f *= kCeB / 3.0;
-    }
-    return p;
-}
-constexpr EeToTe kEeToTe = make_ee_to_te();
+// T(E) = sqrt(2y) G(y) / b with y = bE/3 written in E itself: sqrt(E) P(E)
+constexpr Poly<13> kEeToTe = scaled(kAcoshExpG, const_sqrt(2.0 * kCeB / 3.0) / kCeB, kCeB / 3.0);
 constexpr double kPolyEMax = 3.0 * kPolyYMax / kCeB;
 
-// tanh(x), x = bT, for the heat capacity 3 tanh(x)
+// tanh(x), x = bT, for the heat capacity C(T) = 3 tanh(x)
 __device__ __forceinline__ double tanh_bt(double x) {
     if (fabs(x) <= kPolyXMax) return x * horner(kTanhR, x * x);
     const double v = expm1(-2.0 * x);
@@ -256,7 +257,7 @@ __device__ __forceinline__ double tanh_bt(double x) {
 // E(T): cosh through one exp and its reciprocal outside the fitted range
 __device__ __forceinline__ double te_to_ee(double te) {
     const double x = kCeB * te;
-    if (fabs(x) <= kPolyXMax) return (3.0 / kCeB) * (x * x) * horner(kLogCoshQ, x * x);
+    if (fabs(x) <= kPolyXMax) return (3.0 / kCeB) * (x * x) * horner2(kLogCoshQ, x * x);
     const double e = exp(x);
     return 3.0 / kCeB * log(0.5 * (e + 1.0 / e));
 }
@@ -277,6 +278,52 @@ __device__ __forceinline__ double ee_to_te(double ee) {
     const double y = kCeB / 3.0 * ee;
     if (y <= kPolyYMax) return sqrt(2.0 * y) * horner(kAcoshExpG, y) * (1.0 / kCeB);
     return (y + log1p(sqrt(-expm1(-2.0 * y)))) / kCeB;
+}
+
+// ---------------------------------------------------------------------------
+// reductions in a fixed order (deterministic)
+
+// sum over the 64 lanes of a wave, in every lane; all lanes must be active.
+// Six data-parallel-primitive steps (rows of 16 by shifts of 1, 2, 4, 8, then
+// row 0 into 1 and 2 into 3, then the lower half into the upper): a step is two
+// register moves and an add, where a shuffle goes through LDS.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, true);
+    return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    v = dpp_add<0x111, 0xf>(v);
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    v = dpp_add<0x142, 0xa>(v);
+    v = dpp_add<0x143, 0xc>(v);
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane((int)b, 63);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// partials[k * blocks + block] = the block's sum of v[k] (blocks of up to 256
+// threads, whole waves): wave sums, then those in order
+template <int NK>
+__device__ __forceinline__ void block_partials(const double (&v)[NK], double* partials) {
+    __shared__ double sh[4][NK];
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+        const double w = wave_sum(v[k]);
+        if ((t & 63) == 0) sh[t >> 6][k] = w;
+    }
+    __syncthreads();
+    if (t < NK) {
+        double a = 0.0;
+        for (int w = 0; w < (int)blockDim.x >> 6; ++w) a += sh[w][t];
+        partials[(size_t)t * gridDim.x + blockIdx.x] = a;
+    }
 }
 
 }  // namespace sld

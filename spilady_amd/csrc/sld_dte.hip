@@ -1,0 +1,287 @@
+// Kernels of the electron subsystem's diffusion (core_dTe_CPU.cpp:47-217).
+//
+// Compiled with the two-address FMA off (-fmacf64-inst): the polynomials of
+// the heat capacity are long chains of a*t + c with c kept in registers, and
+// the two-address form overwrites its addend, so each term cost a move.
+#include <hip/hip_runtime.h>
+
+#include "sld_kernels.h"
+
+namespace sld {
+
+// core_dTe sub-step (core_dTe_CPU.cpp:51-55,66-140): A(h) adds the lattice's
+// and spins' energy, B(h) relaxes towards them, C diffuses. What A and B take
+// of a cell is constant over a core_dTe call: k_dte_ab leaves it in M.src for
+// the other sub-step kernels, h dE and g = -G / (3b) with G = (Gel + Ges) h /
+// k_B (16 bytes a cell instead of the 32 of the four fields they come from).
+
+// One relaxation T -> T + increment is RK4 over T (exp(-G / C(T)) - 1), C = 3
+// tanh(bT) (core_dTe_CPU.cpp:91-129). The exponent is u = (g/T) K(x^2) with
+// x = bT, K = x coth x, so T (e^u - 1) = g K (1 + u/2 + ...): one reciprocal
+// and two polynomials, where the defining form spends a division and an exp
+// and cancels (u is 0.001 to 0.1 at 1 fs, larger the colder the electrons).
+// ok turns false outside the fitted temperatures or for |u| > 1/4 (NaN
+// included).
+constexpr Poly<13> kRelaxK = scaled(kXCothX, 1.0, kCeB* kCeB);     // K(x^2) in T^2
+constexpr Poly<18> kTeToEe = scaled(kLogCoshQ, 3.0 * kCeB, kCeB* kCeB);  // E(T) / T^2 in T^2
+constexpr double kPolyT2Max = kPolyXMax * kPolyXMax / (kCeB * kCeB);
+// (e^u - 1) / u for |u| <= 1/4: the next term is 2^-24 / 13! = 1e-17
+constexpr double kExpm1[12] = {1.0,           1.0 / 2.0,      1.0 / 6.0,       1.0 / 24.0,
+                               1.0 / 120.0,   1.0 / 720.0,    1.0 / 5040.0,    1.0 / 40320.0,
+                               1.0 / 362880.0, 1.0 / 3628800.0, 1.0 / 39916800.0, 1.0 / 479001600.0};
+
+__device__ __forceinline__ double relax_fast(double g, double T, bool& ok) {
+    const double t = T * T;
+    double r = __builtin_amdgcn_rcp(T);  // 1/T to about an ulp in two Newton steps
+    r = fma(fma(-T, r, 1.0), r, r);
+    r = fma(fma(-T, r, 1.0), r, r);
+    const double w = g * horner2(kRelaxK.c, t);
+    const double u = w * r;
+    ok = ok && T >= 1e-30 && t <= kPolyT2Max && fabs(u) <= 0.25;
+    return w * horner2(kExpm1, u);
+}
+
+__device__ __forceinline__ double relax_any(double g, double T) {
+    return T * (exp(g * (3.0 * kCeB) / (3.0 * tanh_bt(kCeB * T))) - 1.0);
+}
+
+// The stages are carried as k h (the reference divides each k by h and
+// multiplies it back): the same increments up to rounding. A loop, so that the
+// code and its 25 coefficients stay small.
+template <class F>
+__device__ __forceinline__ double rk4(double T0, F relax) {
+    double q = 0.0, sum = 0.0;
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k) {
+        q = relax(fma(k == 0 ? 0.0 : k == 3 ? 1.0 : 0.5, q, T0));
+        sum = fma(k == 0 || k == 3 ? 1.0 : 2.0, q, sum);
+    }
+    return fma(sum, 1.0 / 6.0, T0);
+}
+
+// n times T(E), B(h), E(T) and, after all but the last of n == 2, A(h) twice:
+// n == 2 takes the energy a sub-step's C left to the one the next C starts
+// from. Returns the energy, T the temperature of the last relaxation.
+// Every lane takes the polynomial route, without branches; a wave with a lane
+// outside its range repeats that lane's cell with the library's functions.
+__device__ __forceinline__ double dte_relax_steps(double e0, double dE, double g, int n, double& T) {
+    bool ok = true;
+    double e = e0;
+#pragma unroll 1
+    for (int k = 0; k < n; ++k) {
+        if (k > 0) e = (e + dE) + dE;
+        ok = ok && e <= kPolyEMax && e >= 1e-200;
+        T = sqrt_normal(e) * horner2(kEeToTe.c, e);
+        T = rk4(T, [&](double x) { return relax_fast(g, x, ok); });
+        const double t = T * T;
+        ok = ok && t <= kPolyT2Max;
+        e = t * horner2(kTeToEe.c, t);
+    }
+    if (__builtin_expect(!ok, 0)) {
+        e = e0;
+#pragma unroll 1
+        for (int k = 0; k < n; ++k) {
+            if (k > 0) e = (e + dE) + dE;
+            T = rk4(ee_to_te(e), [&](double x) { return relax_any(g, x); });
+            e = te_to_ee(T);
+        }
+    }
+    return e;
+}
+
+// the first sub-step's A(h), B(h), then Ee = E(Te) as C starts
+__global__ __launch_bounds__(256) void k_dte_ab(double h, Mesh M, double* partials) {
+    int c = blockIdx.x * blockDim.x + threadIdx.x;
+    double acc[1] = {0.0};
+    if (c < M.C) {
+        double dE = 0.0, G = 0.0;
+        if (M.lattlang) {
+            dE += M.Gel[c] * M.Tl[c];
+            G += M.Gel[c];
+        }
+        if (M.spinlang) {
+            dE += M.Ges[c] * M.TsL[c];
+            G += M.Ges[c];
+        }
+        dE *= h;
+        const double g = G * (h / kBoltz) * (-1.0 / (3.0 * kCeB));
+        M.src[c] = make_double2(dE, g);
+        double T;
+        const double ee = dte_relax_steps(te_to_ee(M.Te[c]) + dE, dE, g, 1, T);
+        M.Te[c] = T;
+        M.Ee[c] = ee;
+        acc[0] = ee;
+    }
+    block_partials<1>(acc, partials);
+}
+
+// The C diffusion sweeps (core_dTe_CPU.cpp:155-197), one workgroup per tile of
+// the mesh (sld_dte_plan.h): the temperatures of the tile's cells, of their
+// closure and of what those read come into LDS, the levels of the schedule
+// run there with a workgroup barrier between them, and the tile writes its
+// own cells to the other copy of the mesh, which no tile of the launch reads.
+// The reference recomputes E(Te) of a cell first; the stored Ee of the cell's
+// last update is that value up to one rounding.
+//
+// A sweep is a chain of up to 20 dependent cell updates whatever the mesh
+// size. A launch per level cost 3.5 us each; here a level costs one LDS round
+// trip, the update's FP64 chain and a barrier, 0.2 us.
+// The energy partials are one per tile: its cells in slot order, 64 at a
+// time, so the sum does not depend on the block size.
+__global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
+    extern __shared__ double sT[];
+    __shared__ double sp[kDteMaxSlot / 64 + 1];
+    const int t = threadIdx.x, B = blockDim.x, lane = t & 63;
+    if ((int)blockIdx.x == ((S.ntile + 7) & ~7)) {  // the block past the tiles adds the starting energies
+        if (t < 64) {
+            double a = 0.0;
+            for (int k0 = t; k0 < A.na; k0 += 8 * 64) {
+                double v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = k0 + u * 64 < A.na ? A.pa[k0 + u * 64] : 0.0;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) a += v[u];
+            }
+            a = wave_sum(a);
+            if (t == 0) A.start[0] = a;
+        }
+        return;
+    }
+    const int tl = (int)(blockIdx.x & 7) * ((S.ntile + 7) >> 3) + (int)(blockIdx.x >> 3);  // see xcd_block
+    if (tl >= S.ntile) return;
+    const DteTile T = S.tile[tl];
+    const uint4* upd = S.upd + T.upd0;
+    const int32_t* slot = S.slot + T.slot0;
+    const int bound = S.lev[T.lev0 + lane];  // lane l: first update of level l
+    double* sE = sT + S.max_slot;
+    constexpr int U = 4;  // slots of a thread in flight
+    for (int s0 = t; s0 < T.nslot; s0 += U * B) {
+        int c[U];
+        double a[U], e[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) c[u] = T.origin + (slot[min(s0 + u * B, T.nslot - 1)] >> 1);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            a[u] = A.Tin[c[u]];
+            e[u] = s0 + u * B < T.nupd ? A.Ein[c[u]] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (s0 + u * B < T.nslot) sT[s0 + u * B] = a[u];
+            if (s0 + u * B < T.nupd) sE[s0 + u * B] = e[u];
+        }
+    }
+    // one update (core_dTe_CPU.cpp:161-190)
+    auto update = [&](const uint4 d) {
+        char* q = reinterpret_cast<char*>(sT);
+        auto at = [&](uint32_t o) -> double& { return *reinterpret_cast<double*>(q + o); };
+        const uint32_t self = d.x & 0xffffu;
+        const double txp = at(d.x >> 16), txm = at(d.y & 0xffffu);
+        const double typ = at(d.y >> 16), tym = at(d.z & 0xffffu);
+        const double tzp = at(d.z >> 16), tzm = at(d.w & 0xffffu);
+        const double tc = at(self);
+        double& E = *reinterpret_cast<double*>(reinterpret_cast<char*>(sE) + self);
+        double ee = E;
+        ee = fma(fma(-2.0, tc, txp + txm), A.px, ee);
+        ee = fma(fma(-2.0, tc, typ + tym), A.py, ee);
+        ee = fma(fma(-2.0, tc, tzp + tzm), A.pz, ee);
+        E = ee;
+        at(self) = ee_to_te(ee);
+    };
+    // a thread's first update of the next level is requested one level ahead
+    // (straight-line code: the wait before an update leaves the request in
+    // flight)
+    uint4 d = upd[min(t, T.nent - 1)];
+    __syncthreads();
+    int lo = 0;
+    for (int l = 0; l < T.nlev; ++l) {
+        const int hi = __builtin_amdgcn_readlane(bound, l + 1);
+        const uint4 nx = upd[min(hi + t, T.nent - 1)];
+        if (lo + t < hi) update(d);
+        if (hi - lo > B)
+            for (int k = lo + B + t; k < hi; k += B) update(upd[k]);
+        d = nx;
+        lo = hi;
+        __syncthreads();
+    }
+    const int nch = (T.nupd + 63) >> 6;
+    for (int q = t >> 6; q < nch; q += B >> 6) {
+        const int s = q * 64 + lane;
+        const int32_t c = s < T.nupd ? slot[s] : 0;
+        const bool own = (c & 1) != 0;
+        const double ee = own ? sE[s] : 0.0;
+        if (own) {
+            A.Eout[T.origin + (c >> 1)] = ee;
+            if (A.Tout) A.Tout[T.origin + (c >> 1)] = sT[s];
+        }
+        if (A.ends) {
+            const double v = wave_sum(ee);
+            if (lane == 0) sp[q] = v;
+        }
+    }
+    if (A.ends) {
+        __syncthreads();
+        if (t < 64) {
+            double a = 0.0;
+            for (int k = t; k < nch; k += 64) a += sp[k];
+            a = wave_sum(a);
+            if (t == 0) A.ends[tl] = a;
+        }
+    }
+}
+
+// the final energy of a sub-step from its n partials, by every block of 256
+// threads for itself in the same fixed order
+__device__ __forceinline__ double dte_end_total(const double* p, int n) {
+    __shared__ double sh[4];
+    const int t = threadIdx.x;
+    double a = 0.0;
+    for (int k = t; k < n; k += 256) a += p[k];
+    a = wave_sum(a);
+    if ((t & 63) == 0) sh[t >> 6] = a;
+    __syncthreads();
+    return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+
+// The sub-step's cell work between two diffusions. With 64 cells a wave and
+// 1,284 blocks at 328,509 cells every wave is resident at once, and the time is
+// the launch, one round trip to memory and a wave's own instruction stream:
+// the two polynomials of a relaxation instead of a division and an exp, and
+// wave sums without LDS, took it from 17.0 to 12.1 us there, from 6.9 to 4.6
+// at 12,167 cells.
+// end of one sub-step and start of the next: renormalise (core_dTe_CPU.cpp:199-216),
+// B(h), A(h), then the next sub-step's A(h), B(h) and E(Te) as its C starts.
+// The Te and Ee that the first A(h) leaves are overwritten by the second
+// before anything reads them, so only the final values are stored.
+__global__ __launch_bounds__(256) void k_dte_finish_ab(Mesh M, const double* E, const double* start,
+                                                       const double* ends, int nend, double* partials) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    const int cc = c < M.C ? c : M.C - 1;
+    const double2 src = M.src[cc];
+    const double e0 = E[cc];
+    const double f = start[0] / dte_end_total(ends, nend);
+    double acc[1] = {0.0};
+    if (c < M.C) {
+        double T;
+        const double ee = dte_relax_steps(e0 * f, src.x, src.y, 2, T);
+        M.Te[c] = T;
+        M.Ee[c] = ee;
+        acc[0] = ee;
+    }
+    block_partials<1>(acc, partials);
+}
+
+// renormalise to the starting total (core_dTe_CPU.cpp:199-216), then B(h), A(h)
+__global__ __launch_bounds__(256) void k_dte_finish(Mesh M, const double* E, const double* start, const double* ends,
+                                                    int nend) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    const double f = start[0] / dte_end_total(ends, nend);
+    if (c >= M.C) return;
+    const double2 src = M.src[c];
+    double T;
+    const double ee = dte_relax_steps(E[c] * f, src.x, src.y, 1, T) + src.x;
+    M.Ee[c] = ee;
+    M.Te[c] = ee_to_te(ee);
+}
+
+}  // namespace sld

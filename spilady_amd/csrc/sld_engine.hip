@@ -81,6 +81,7 @@ struct sld_ctx {
     DteTiles dte[2] = {};
     size_t dte_lds[2] = {0, 0};
     double *d_te2 = nullptr, *d_ee2 = nullptr;
+    double2* d_dte_src = nullptr;  // what a sub-step adds to each cell
     // buffers
     double *d_prow = nullptr, *d_rhotab = nullptr;
     int *d_cl2 = nullptr, *d_cn2 = nullptr;  // second cell-list buffer
@@ -494,7 +495,7 @@ int do_dTe_launches(sld_ctx* c, double dt) {
     double vf = atomic_volume / (natom / ncell);
     double pref = dtl / 2.0 * kappa * vf / kBoltz;
     int nb = nblk(c->D.C, 256);
-    const Mesh M{c->D.Te, c->D.Ee, c->D.Gel, c->D.Ges, c->D.Tl, c->D.TsL, c->D.C, c->phys.lattlang,
+    const Mesh M{c->D.Te, c->D.Ee, c->D.Gel, c->D.Ges, c->D.Tl, c->D.TsL, c->d_dte_src, c->D.C, c->phys.lattlang,
                  c->phys.spinlang};
     LAUNCH(c, k_dte_ab, nb, 256, h, M, c->d_part);
     // block partials: [0, nb) starting energies (k_dte_ab / k_dte_finish_ab),
@@ -545,9 +546,9 @@ int do_dTe_launches(sld_ctx* c, double dt) {
             ne = 1;
         }
         if (it + 1 < nloop)
-            LAUNCH(c, k_dte_finish_ab, nb, 256, h, M, Eswept, (const double*)start, ep, ne, c->d_part);
+            LAUNCH(c, k_dte_finish_ab, nb, 256, M, Eswept, (const double*)start, ep, ne, c->d_part);
         else
-            LAUNCH(c, k_dte_finish, nb, 256, h, M, Eswept, (const double*)start, ep, ne);
+            LAUNCH(c, k_dte_finish, nb, 256, M, Eswept, (const double*)start, ep, ne);
     }
     return SLD_OK;
 }
@@ -986,6 +987,7 @@ int upload_dte_schedules(sld_ctx* c) {
     }
     TRY(dalloc(c, &c->d_te2, hc.C));
     TRY(dalloc(c, &c->d_ee2, hc.C));
+    TRY(dalloc(c, &c->d_dte_src, hc.C));
     return SLD_OK;
 }
 

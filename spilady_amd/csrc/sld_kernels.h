@@ -66,6 +66,7 @@ struct Dev {
 struct Mesh {
     double *Te, *Ee;
     const double *Gel, *Ges, *Tl, *TsL;
+    double2* src;  // per cell: h (Gel Tl + Ges TsL), and -(Gel + Ges) h / (3 b k_B)
     int C, lattlang, spinlang;
 };
 
@@ -141,8 +142,8 @@ struct DteSweepArgs {
 __global__ void k_dte_sweep(DteTiles S, DteSweepArgs A);
 // E: the energies the sweeps left; start: the sub-step's starting energy;
 // ends: nend partials of its final one
-__global__ void k_dte_finish(double h, Mesh M, const double* E, const double* start, const double* ends, int nend);
-__global__ void k_dte_finish_ab(double h, Mesh M, const double* E, const double* start, const double* ends, int nend,
+__global__ void k_dte_finish(Mesh M, const double* E, const double* start, const double* ends, int nend);
+__global__ void k_dte_finish_ab(Mesh M, const double* E, const double* start, const double* ends, int nend,
                                 double* partials);
 __global__ void k_obs_atoms(Tables T, Phys P, Dev D, double* partials, int scan_spin);
 __global__ void k_obs_cells(Dev D, double* partials);

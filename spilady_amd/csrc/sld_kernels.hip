@@ -15,35 +15,7 @@
 namespace sld {
 
 // ---------------------------------------------------------------------------
-// block reductions into per-block partials (fixed tree order: deterministic)
-
-// sum over the 64 lanes of a wave, by a fixed butterfly of shuffles
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m, 64);
-    return v;
-}
-
-
-template <int NK>
-__device__ __forceinline__ void block_partials(const double (&v)[NK], double* partials) {
-    __shared__ double sh[NK][256];
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < NK; ++k) sh[k][t] = v[k];
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if (t < s) {
-#pragma unroll
-            for (int k = 0; k < NK; ++k) sh[k][t] += sh[k][t + s];
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-#pragma unroll
-        for (int k = 0; k < NK; ++k) partials[(size_t)k * gridDim.x + blockIdx.x] = sh[k][0];
-    }
-}
+// reductions
 
 // out[k] = sum over blocks of partials[k*nblk + b]; one block of 256 threads.
 __global__ __launch_bounds__(256) void k_reduce(const double* partials, int nblk, int nk, double* out) {
@@ -1236,234 +1208,6 @@ __global__ __launch_bounds__(256) void k_temperature(Tables T, Phys P, Dev D) {
     D.Ges[c] = kBoltz * P.gamma_S * ldn / apc;
     D.sRup[c] = rup; D.sRdn[c] = rdn; D.sLup[c] = lup; D.sLdn[c] = ldn;
 }
-
-// core_dTe sub-step, first half: A(h), B(h), then Ee = E(Te) as C starts
-// (core_dTe_CPU.cpp:51-55,66-129,133-140)
-__device__ __forceinline__ double dte_dE(const Mesh& M, int c) {
-    double dE = 0.0;
-    if (M.lattlang) dE += M.Gel[c] * M.Tl[c];
-    if (M.spinlang) dE += M.Ges[c] * M.TsL[c];
-    return dE;
-}
-
-__device__ __forceinline__ void dte_A(int c, double h, const Mesh& M) {
-    double ee = te_to_ee(M.Te[c]);
-    ee += h * dte_dE(M, c);
-    M.Ee[c] = ee;
-    M.Te[c] = ee_to_te(ee);
-}
-
-// exp(-G / C(T)) - 1 with C(T) = 3 tanh(bT) (heatcapacity_CPU.cpp:34-57)
-__device__ __forceinline__ double relax_factor(double G, double T) {
-    return exp(-G / (3.0 * tanh_bt(kCeB * T))) - 1.0;
-}
-
-// RK4 of the electron-ion/spin relaxation over h (core_dTe_CPU.cpp:91-129),
-// G = (Gel + Ges) h / k_B. The stages are carried as k h (the reference
-// divides each k by h and multiplies it back): the same increments up to
-// rounding.
-__device__ __forceinline__ double dte_rk4(double T0, double G) {
-    const double q1 = T0 * relax_factor(G, T0);
-    const double T1 = T0 + q1 / 2.0;
-    const double q2 = T1 * relax_factor(G, T1);
-    const double T2 = T0 + q2 / 2.0;
-    const double q3 = T2 * relax_factor(G, T2);
-    const double T3 = T0 + q3;
-    const double q4 = T3 * relax_factor(G, T3);
-    return T0 + (q1 + 2.0 * q2 + 2.0 * q3 + q4) / 6.0;
-}
-
-__device__ __forceinline__ double dte_G(int c, double h, const Mesh& M) {
-    double G = 0.0;
-    if (M.lattlang) G += M.Gel[c];
-    if (M.spinlang) G += M.Ges[c];
-    return G * (h / kBoltz);
-}
-
-__device__ __forceinline__ void dte_B(int c, double h, const Mesh& M) {
-    M.Te[c] = dte_rk4(M.Te[c], dte_G(c, h, M));
-}
-
-__global__ __launch_bounds__(256) void k_dte_ab(double h, Mesh M, double* partials) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    double acc[1] = {0.0};
-    if (c < M.C) {
-        dte_A(c, h, M);
-        dte_B(c, h, M);
-        double ee = te_to_ee(M.Te[c]);
-        M.Ee[c] = ee;
-        acc[0] = ee;
-    }
-    block_partials<1>(acc, partials);
-}
-
-// The C diffusion sweeps (core_dTe_CPU.cpp:155-197), one workgroup per tile of
-// the mesh (sld_dte_plan.h): the temperatures of the tile's cells, of their
-// closure and of what those read come into LDS, the levels of the schedule
-// run there with a workgroup barrier between them, and the tile writes its
-// own cells to the other copy of the mesh, which no tile of the launch reads.
-// The reference recomputes E(Te) of a cell first; the stored Ee of the cell's
-// last update is that value up to one rounding.
-//
-// A sweep is a chain of up to 20 dependent cell updates whatever the mesh
-// size. A launch per level cost 3.5 us each; here a level costs one LDS round
-// trip, the update's FP64 chain and a barrier, 0.2 us.
-// The energy partials are one per tile: its cells in slot order, 64 at a
-// time, so the sum does not depend on the block size.
-__global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
-    extern __shared__ double sT[];
-    __shared__ double sp[kDteMaxSlot / 64 + 1];
-    const int t = threadIdx.x, B = blockDim.x, lane = t & 63;
-    if ((int)blockIdx.x == ((S.ntile + 7) & ~7)) {  // the block past the tiles adds the starting energies
-        if (t < 64) {
-            double a = 0.0;
-            for (int k0 = t; k0 < A.na; k0 += 8 * 64) {
-                double v[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) v[u] = k0 + u * 64 < A.na ? A.pa[k0 + u * 64] : 0.0;
-#pragma unroll
-                for (int u = 0; u < 8; ++u) a += v[u];
-            }
-            a = wave_sum(a);
-            if (t == 0) A.start[0] = a;
-        }
-        return;
-    }
-    const int tl = (int)(blockIdx.x & 7) * ((S.ntile + 7) >> 3) + (int)(blockIdx.x >> 3);  // see xcd_block
-    if (tl >= S.ntile) return;
-    const DteTile T = S.tile[tl];
-    const uint4* upd = S.upd + T.upd0;
-    const int32_t* slot = S.slot + T.slot0;
-    const int bound = S.lev[T.lev0 + lane];  // lane l: first update of level l
-    double* sE = sT + S.max_slot;
-    constexpr int U = 4;  // slots of a thread in flight
-    for (int s0 = t; s0 < T.nslot; s0 += U * B) {
-        int c[U];
-        double a[U], e[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) c[u] = T.origin + (slot[min(s0 + u * B, T.nslot - 1)] >> 1);
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            a[u] = A.Tin[c[u]];
-            e[u] = s0 + u * B < T.nupd ? A.Ein[c[u]] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (s0 + u * B < T.nslot) sT[s0 + u * B] = a[u];
-            if (s0 + u * B < T.nupd) sE[s0 + u * B] = e[u];
-        }
-    }
-    // one update (core_dTe_CPU.cpp:161-190)
-    auto update = [&](const uint4 d) {
-        char* q = reinterpret_cast<char*>(sT);
-        auto at = [&](uint32_t o) -> double& { return *reinterpret_cast<double*>(q + o); };
-        const uint32_t self = d.x & 0xffffu;
-        const double txp = at(d.x >> 16), txm = at(d.y & 0xffffu);
-        const double typ = at(d.y >> 16), tym = at(d.z & 0xffffu);
-        const double tzp = at(d.z >> 16), tzm = at(d.w & 0xffffu);
-        const double tc = at(self);
-        double& E = *reinterpret_cast<double*>(reinterpret_cast<char*>(sE) + self);
-        double ee = E;
-        ee = fma(fma(-2.0, tc, txp + txm), A.px, ee);
-        ee = fma(fma(-2.0, tc, typ + tym), A.py, ee);
-        ee = fma(fma(-2.0, tc, tzp + tzm), A.pz, ee);
-        E = ee;
-        at(self) = ee_to_te(ee);
-    };
-    // a thread's first update of the next level is requested one level ahead
-    // (straight-line code: the wait before an update leaves the request in
-    // flight)
-    uint4 d = upd[min(t, T.nent - 1)];
-    __syncthreads();
-    int lo = 0;
-    for (int l = 0; l < T.nlev; ++l) {
-        const int hi = __builtin_amdgcn_readlane(bound, l + 1);
-        const uint4 nx = upd[min(hi + t, T.nent - 1)];
-        if (lo + t < hi) update(d);
-        if (hi - lo > B)
-            for (int k = lo + B + t; k < hi; k += B) update(upd[k]);
-        d = nx;
-        lo = hi;
-        __syncthreads();
-    }
-    const int nch = (T.nupd + 63) >> 6;
-    for (int q = t >> 6; q < nch; q += B >> 6) {
-        const int s = q * 64 + lane;
-        const int32_t c = s < T.nupd ? slot[s] : 0;
-        const bool own = (c & 1) != 0;
-        const double ee = own ? sE[s] : 0.0;
-        if (own) {
-            A.Eout[T.origin + (c >> 1)] = ee;
-            if (A.Tout) A.Tout[T.origin + (c >> 1)] = sT[s];
-        }
-        if (A.ends) {
-            const double v = wave_sum(ee);
-            if (lane == 0) sp[q] = v;
-        }
-    }
-    if (A.ends) {
-        __syncthreads();
-        if (t < 64) {
-            double a = 0.0;
-            for (int k = t; k < nch; k += 64) a += sp[k];
-            a = wave_sum(a);
-            if (t == 0) A.ends[tl] = a;
-        }
-    }
-}
-
-// the final energy of a sub-step from its n partials, by every block of 256
-// threads for itself in the same fixed order
-__device__ __forceinline__ double dte_end_total(const double* p, int n) {
-    __shared__ double sh[4];
-    const int t = threadIdx.x;
-    double a = 0.0;
-    for (int k = t; k < n; k += 256) a += p[k];
-    a = wave_sum(a);
-    if ((t & 63) == 0) sh[t >> 6] = a;
-    __syncthreads();
-    return (sh[0] + sh[1]) + (sh[2] + sh[3]);
-}
-
-// end of one sub-step and start of the next: renormalise (core_dTe_CPU.cpp:199-216),
-// B(h), A(h), then the next sub-step's A(h), B(h) and E(Te) as its C starts
-// In registers: the Te and Ee that the first A(h) leaves are overwritten by
-// the second before anything reads them, so only the final values are
-// computed and stored (same arithmetic as B, A, A, B applied in turn).
-__global__ __launch_bounds__(256) void k_dte_finish_ab(double h, Mesh M, const double* E, const double* start,
-                                                       const double* ends, int nend, double* partials) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    const int cc = c < M.C ? c : M.C - 1;
-    const double G = dte_G(cc, h, M);
-    const double dE = dte_dE(M, cc);
-    const double e0 = E[cc];
-    const double f = start[0] / dte_end_total(ends, nend);
-    double acc[1] = {0.0};
-    if (c < M.C) {
-        double T = ee_to_te(e0 * f);
-        T = dte_rk4(T, G);                  // B(h) ends the sub-step
-        double ee = te_to_ee(T) + h * dE;      // A(h) ends it
-        ee += h * dE;                          // A(h) starts the next
-        T = dte_rk4(ee_to_te(ee), G);       // B(h)
-        ee = te_to_ee(T);                      // E(Te) as C starts
-        M.Te[c] = T;
-        M.Ee[c] = ee;
-        acc[0] = ee;
-    }
-    block_partials<1>(acc, partials);
-}
-
-// renormalise to the starting total (core_dTe_CPU.cpp:199-216), then B(h), A(h)
-__global__ __launch_bounds__(256) void k_dte_finish(double h, Mesh M, const double* E, const double* start,
-                                                    const double* ends, int nend) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    const double f = start[0] / dte_end_total(ends, nend);
-    if (c >= M.C) return;
-    M.Te[c] = ee_to_te(E[c] * f);
-    dte_B(c, h, M);
-    dte_A(c, h, M);
-}
-
 
 // ---------------------------------------------------------------------------
 // barostats: positions follow the box (scale_pressure_CPU.cpp:59,

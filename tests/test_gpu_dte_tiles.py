@@ -54,3 +54,24 @@ def test_core_dte_on_any_mesh(cells):
         assert_close(want[k], got[0][k], f"{cells} {k}")
         for g in got[1:]:
             np.testing.assert_array_equal(g[k], got[0][k])
+
+
+@pytest.mark.parametrize("lo,hi", [(0.5, 20.0), (2.0, 20000.0), (5000.0, 8000.0)])
+def test_core_dte_outside_the_polynomials(lo, hi):
+    """Electron temperatures below and above the fitted range and relaxations
+    past |u| = 1/4, cell by cell next to ordinary ones: waves with both kinds
+    of lanes."""
+    p, at = _system((7, 6, 8))
+    o = orcpy.Oracle(p, at, compute_initial_forces=True, rng=orcpy.RNG_PHILOX)
+    te = BOLTZ * np.exp(np.random.default_rng(11).uniform(np.log(lo), np.log(hi), o.ncells))
+    o.set_cells_te(te)
+    o.core_dTe(0.5e-15)
+    want = o.cells()
+    o.close()
+    e = Engine(p, at, compute_initial_forces=True)
+    e.set_cells_te(te)
+    e.core_dTe(0.5e-15)
+    got = e.cells()
+    e.close()
+    for k in ("te", "ee"):
+        assert_close(want[k], got[k], f"{lo}-{hi} K {k}")
