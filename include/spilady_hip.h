@@ -267,7 +267,7 @@ int sld_kernel_timing(sld_ctx* ctx, int* launches, double* total_ms);
  * them: every reduction inside them sums per wavefront, so a trajectory is
  * bitwise the same under any valid shapes. */
 typedef struct {
-    int spin_block;        /* core_ds sweep level: threads (one per cell) per block; 32, 64 or 128 */
+    int spin_block;        /* core_ds sweep level: eight times the most cells a wave takes; 32, 64 or 128 */
     int sweep_block;       /* core_dTe diffusion: threads of a tile's workgroup (twice as many on meshes of
                               up to 512 tiles); 64, 128 or 256 */
     int force_block;       /* force/energy: threads (one per atom) per block; 64, 128 or 256 */
@@ -275,8 +275,8 @@ typedef struct {
     int temperature_block; /* calculate_temperature: threads (32 per cell) per block; 64, 128 or 256 */
     int sweep_tail;        /* kept for the layout: every level of a sweep runs inside its tile's workgroup;
                               0, 2048 or 8192 */
-    int spin_lanes;        /* core_ds sweep level: lanes that share one cell's walk (the neighbour
-                              gathers and field sums split among them); 1, 2 or 4 */
+    int spin_lanes;        /* core_ds sweep level: lanes that walk one cell (four times as many where the
+                              wave has them to spare); 1, 2 or 4 */
 } sld_shapes;
 int sld_get_shapes(sld_ctx* ctx, sld_shapes* out);
 /* How sld_step issues its work (no counterpart in the reference): 0 (default)

@@ -25,12 +25,34 @@ __device__ __forceinline__ double3 sub3(double3 a, double3 b) { return make_doub
 __device__ __forceinline__ double3 mul3(double k, double3 a) { return make_double3(k * a.x, k * a.y, k * a.z); }
 __device__ __forceinline__ double dot3(double3 a, double3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 __device__ __forceinline__ double sq3(double3 a) { return a.x * a.x + a.y * a.y + a.z * a.z; }
+// sqrt(x) for normal x far from the ends of the exponent range, to about an
+// ulp: the hardware's reciprocal square root (2^-23 or better) and two
+// Newton steps, without the library's scaling and final rounding step
+__device__ __forceinline__ double sqrt_normal(double x) {
+    const double r = __builtin_amdgcn_rsq(x);
+    double g = x * r, h = 0.5 * r;
+    const double d = fma(-h, g, 0.5);
+    g = fma(g, d, g);
+    h = fma(h, d, h);
+    return fma(fma(-g, g, x), h, g);
+}
+// 1/sqrt(x), likewise: one step of third order
+__device__ __forceinline__ double rsqrt_normal(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
 // |s|, the value every spin's .w payload holds. It is the only definition of
 // that value: the field sums read a neighbour's .w where the reference takes
 // vec_length(s_j) (calculate_spin_CPU.cpp:265), so every writer of .w must
 // round it the same way. The explicit fma order leaves the compiler no
 // contraction choice that could differ between kernels.
-__device__ __forceinline__ double spin_len(double3 s) { return sqrt(fma(s.z, s.z, fma(s.x, s.x, s.y * s.y))); }
+__device__ __forceinline__ double spin_len(double3 s) {
+    const double x = fma(s.z, s.z, fma(s.x, s.x, s.y * s.y));
+    double r = sqrt_normal(x);
+    if (__builtin_expect(!(x >= 1e-200 && x <= 1e200), 0)) r = sqrt(x);
+    return r;
+}
 __device__ __forceinline__ double3 cross3(double3 a, double3 b) {
     return make_double3(a.y * b.z - b.y * a.z, a.z * b.x - b.z * a.x, a.x * b.y - b.x * a.y);
 }
@@ -260,17 +282,6 @@ __device__ __forceinline__ double te_to_ee(double te) {
     if (fabs(x) <= kPolyXMax) return (3.0 / kCeB) * (x * x) * horner2(kLogCoshQ, x * x);
     const double e = exp(x);
     return 3.0 / kCeB * log(0.5 * (e + 1.0 / e));
-}
-// sqrt(x) for normal x far from the ends of the exponent range, to about an
-// ulp: the hardware's reciprocal square root (2^-23 or better) and two
-// Newton steps, without the library's scaling and final rounding step
-__device__ __forceinline__ double sqrt_normal(double x) {
-    const double r = __builtin_amdgcn_rsq(x);
-    double g = x * r, h = 0.5 * r;
-    const double d = fma(-h, g, 0.5);
-    g = fma(g, d, g);
-    h = fma(h, d, h);
-    return fma(fma(-g, g, x), h, g);
 }
 // T(E); outside the fitted range acosh(e^y) = y + log1p(sqrt(-expm1(-2y)))
 __device__ __forceinline__ double ee_to_te(double ee) {
