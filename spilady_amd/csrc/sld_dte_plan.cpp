@@ -105,8 +105,9 @@ bool dte_schedule(int nx, int ny, int nz, const std::vector<int>& group, DteSwee
         // slot of a cell in the current tile; bits of its updates in the closure
         std::vector<int> slot(C, -1);
         std::vector<uint8_t> has(C, 0);
-        std::vector<std::vector<std::pair<int, int>>> lev(maxlev);  // (slot, cell)
-        std::vector<std::pair<int, int>> todo;                      // (cell, backward)
+        std::vector<std::vector<int>> lev(maxlev);
+        std::vector<int64_t> keys;
+        std::vector<std::pair<int, int>> todo;  // (cell, backward)
         std::vector<int> cells, reads;
         std::unordered_multimap<size_t, int> by;
         for (int t = t0; t < t1; ++t) {
@@ -146,9 +147,13 @@ bool dte_schedule(int nx, int ny, int nz, const std::vector<int>& group, DteSwee
             // slots by the level of a cell's first update, then by cell: the
             // cells of a level, and mostly their neighbours, are then
             // consecutive in LDS
-            auto key = [&](int c) { return (long)(fwd ? lf[c] : lb[c]) * C + c; };
-            auto less = [&](int p, int q) { return key(p) < key(q); };
-            std::sort(cells.begin(), cells.end(), less);
+            auto order_cells = [&](std::vector<int>& v) {
+                keys.clear();
+                for (int c : v) keys.push_back((int64_t)(fwd ? lf[c] : lb[c]) * C + c);
+                std::sort(keys.begin(), keys.end());
+                for (size_t k = 0; k < v.size(); ++k) v[k] = (int)(keys[k] % C);
+            };
+            order_cells(cells);
             Lists L;
             L.nupd = (int)cells.size();
             for (int c : cells) {
@@ -163,7 +168,7 @@ bool dte_schedule(int nx, int ny, int nz, const std::vector<int>& group, DteSwee
                         reads.push_back(n);
                     }
             }
-            std::sort(reads.begin(), reads.end(), less);
+            order_cells(reads);
             for (int n : reads) {
                 slot[n] = (int)L.slot.size();
                 L.slot.push_back(2 * (n - origin));
@@ -173,15 +178,18 @@ bool dte_schedule(int nx, int ny, int nz, const std::vector<int>& group, DteSwee
                 return;
             }
             for (auto& v : lev) v.clear();
-            for (const auto& u : todo) lev[u.second ? lb[u.first] : lf[u.first]].emplace_back(slot[u.first], u.first);
-            for (auto& v : lev) {
+            for (int c : cells) {  // in slot order
+                if (has[c] & 1) lev[lf[c]].push_back(c);
+                if (has[c] & 2) lev[lb[c]].push_back(c);
+            }
+            L.upd.reserve(todo.size());
+            for (const auto& v : lev) {
                 if (v.empty()) continue;
-                std::sort(v.begin(), v.end());
                 L.lev.push_back((int32_t)L.upd.size());
-                for (const auto& u : v) {
+                for (int c : v) {
                     DteUpdate d{};
-                    d.self = (uint16_t)(8 * u.first);
-                    M.faces(u.second, f);
+                    d.self = (uint16_t)(8 * slot[c]);
+                    M.faces(c, f);
                     for (int q = 0; q < 6; ++q) d.nb[q] = (uint16_t)(8 * slot[f[q]]);
                     L.upd.push_back(d);
                 }

@@ -15,6 +15,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/spilady_hip.h"
@@ -108,6 +109,10 @@ struct sld_ctx {
     bool ev_span = false;          // an event pair spans a run of launches
     int timed_launches = 0;
     double timed_ms = 0.0;
+    // pinned host buffers that the transfer kernels write to and read from
+    double* h_stage[2] = {nullptr, nullptr};
+    size_t stage_cap = 0;  // doubles in each
+    hipEvent_t stage_ev[2] = {nullptr, nullptr};
     std::string err;
     std::vector<void*> allocs;
     std::vector<size_t> alloc_bytes;  // size of each entry of allocs
@@ -877,66 +882,176 @@ int collect_timing(sld_ctx* c) {
     return SLD_OK;
 }
 
-// host <-> device copies of replica `r`'s atom slots [atom0, atom0 + natom).
-// With with_len (spins) the device sets .w = |s| afterwards, with the one
-// rounding every other writer of .w uses.
-int up4(sld_ctx* c, double4* d, const double* src, int r, bool with_len) {
-    if (!src) return SLD_OK;
-    const Rep& R = c->reps[r];
-    std::vector<double> h((size_t)R.natom * 4);
-    for (int i = 0; i < R.natom; ++i) {
-        double x = src[3 * i], y = src[3 * i + 1], z = src[3 * i + 2];
-        h[4 * i] = x; h[4 * i + 1] = y; h[4 * i + 2] = z;
-        h[4 * i + 3] = 0.0;
-    }
-    HIPCHK(c, hipMemcpyAsync(d + R.atom0, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    if (with_len) LAUNCH(c, k_spin_len, nblk(R.natom, 256), 256, c->D, R.atom0, R.natom);
+// ---------------------------------------------------------------------------
+// state between the caller's arrays and the device
+//
+// The device's vectors are double4 and its stress is component-major; the
+// caller's arrays are dense. Kernels convert on the way, straight from and to
+// pinned host memory, in pieces of up to 4 MB: while the device fills one
+// buffer the host copies the other out. All arrays of a call share pieces, so
+// a small system's download is one launch and one wait.
+
+constexpr size_t kStageDoubles = 1 << 19;  // of each of the two buffers, at most
+
+struct Transfer {
+    const void* dev;  // first element on the device
+    double* host;
+    size_t n;         // elements
+    int kind;         // XferSeg::kind
+};
+
+int width(int kind) { return kind == kXferVec ? 3 : kind == kXferStress ? 6 : 1; }
+
+int stage_reserve(sld_ctx* c, size_t doubles) {
+    // a quarter of the call's data a buffer: pinning costs about 0.2 ms a MB
+    const size_t want = std::min(kStageDoubles, std::max(doubles / 4, (size_t)1 << 15));
+    if (want <= c->stage_cap) return SLD_OK;
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    for (int k = 0; k < 2; ++k) {
+        if (c->h_stage[k]) HIPCHK(c, hipHostFree(c->h_stage[k]));
+        c->h_stage[k] = nullptr;
+        c->stage_cap = 0;
+    }
+    for (int k = 0; k < 2; ++k) {
+        HIPCHK(c, hipHostMalloc((void**)&c->h_stage[k], want * sizeof(double), hipHostMallocDefault));
+        if (!c->stage_ev[k]) HIPCHK(c, hipEventCreateWithFlags(&c->stage_ev[k], hipEventDisableTiming));
+    }
+    c->stage_cap = want;
+    return SLD_OK;
+}
+
+// one piece: up to kXferSegs runs of elements, back to back in a buffer
+struct Piece {
+    XferArgs args{};
+    double* host[kXferSegs];
+    size_t doubles = 0;
+};
+
+std::vector<Piece> pieces_of(const std::vector<Transfer>& ts, size_t cap) {
+    std::vector<Piece> out;
+    for (const Transfer& t : ts) {
+        const size_t w = width(t.kind);
+        for (size_t done = 0; done < t.n;) {
+            if (out.empty() || out.back().args.nseg == kXferSegs || cap - out.back().doubles < w)
+                out.emplace_back();
+            Piece& p = out.back();
+            const size_t n = std::min(t.n - done, (cap - p.doubles) / w);
+            p.host[p.args.nseg] = t.host + done * w;
+            XferSeg& g = p.args.seg[p.args.nseg++];
+            g = XferSeg{t.dev, done, n, p.doubles, t.kind};
+            p.doubles += n * w;
+            done += n;
+        }
+    }
+    return out;
+}
+
+// copies between a piece's host arrays and its buffer; several threads where
+// there is enough to copy
+void copy_piece(const Piece& p, double* buf, bool to_host) {
+    auto part = [&](size_t lo, size_t hi) {  // doubles [lo, hi) of the piece
+        for (int k = 0; k < p.args.nseg; ++k) {
+            const XferSeg& g = p.args.seg[k];
+            const size_t a = std::max(lo, g.offset), b = std::min(hi, g.offset + g.n * width(g.kind));
+            if (a >= b) continue;
+            double* h = p.host[k] + (a - g.offset);
+            if (to_host) std::memcpy(h, buf + a, (b - a) * sizeof(double));
+            else std::memcpy(buf + a, h, (b - a) * sizeof(double));
+        }
+    };
+    const size_t nt = std::min<size_t>(4, p.doubles >> 16);  // a thread per 512 KB, at most four
+    if (nt < 2) return part(0, p.doubles);
+    std::vector<std::thread> th;
+    size_t done = 0;
+    try {
+        for (; done + 1 < nt; ++done) th.emplace_back(part, p.doubles * done / nt, p.doubles * (done + 1) / nt);
+    } catch (...) {
+        // no thread to be had: this one copies the rest
+    }
+    part(p.doubles * done / nt, p.doubles);
+    for (auto& x : th) x.join();
+}
+
+size_t total_doubles(const std::vector<Transfer>& ts) {
+    size_t n = 0;
+    for (const Transfer& t : ts) n += t.n * width(t.kind);
+    return n;
+}
+
+int launch_piece(sld_ctx* c, const Piece& p, double* buf, bool to_host) {
+    size_t most = 0;
+    for (int k = 0; k < p.args.nseg; ++k) most = std::max(most, p.args.seg[k].n);
+    const int nb = (int)((most + 255) / 256);
+    if (to_host) hipLaunchKernelGGL(k_pack, dim3(nb, p.args.nseg), dim3(256), 0, c->stream, p.args, c->D.N, buf);
+    else hipLaunchKernelGGL(k_unpack, dim3(nb, p.args.nseg), dim3(256), 0, c->stream, p.args, c->D.N, (const double*)buf);
+    HIPCHK(c, hipGetLastError());
+    return SLD_OK;
+}
+
+// device to the caller's arrays (transfers with a null host array are skipped)
+int stage_out(sld_ctx* c, std::vector<Transfer> ts) {
+    ts.erase(std::remove_if(ts.begin(), ts.end(), [](const Transfer& t) { return !t.host || t.n == 0; }), ts.end());
+    if (ts.empty()) return SLD_OK;
+    TRY(stage_reserve(c, total_doubles(ts)));
+    const std::vector<Piece> ps = pieces_of(ts, c->stage_cap);
+    for (size_t k = 0; k <= ps.size(); ++k) {
+        if (k < ps.size()) {
+            TRY(launch_piece(c, ps[k], c->h_stage[k & 1], true));
+            HIPCHK(c, hipEventRecord(c->stage_ev[k & 1], c->stream));
+        }
+        if (k > 0) {
+            HIPCHK(c, hipEventSynchronize(c->stage_ev[(k - 1) & 1]));
+            copy_piece(ps[k - 1], c->h_stage[(k - 1) & 1], true);
+        }
+    }
+    return SLD_OK;
+}
+
+// the caller's arrays to the device; returns when they have been read
+int stage_in(sld_ctx* c, std::vector<Transfer> ts) {
+    ts.erase(std::remove_if(ts.begin(), ts.end(), [](const Transfer& t) { return !t.host || t.n == 0; }), ts.end());
+    if (ts.empty()) return SLD_OK;
+    TRY(stage_reserve(c, total_doubles(ts)));
+    const std::vector<Piece> ps = pieces_of(ts, c->stage_cap);
+    for (size_t k = 0; k < ps.size(); ++k) {
+        if (k > 1) HIPCHK(c, hipEventSynchronize(c->stage_ev[k & 1]));
+        copy_piece(ps[k], c->h_stage[k & 1], false);
+        TRY(launch_piece(c, ps[k], c->h_stage[k & 1], false));
+        HIPCHK(c, hipEventRecord(c->stage_ev[k & 1], c->stream));
+    }
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return SLD_OK;
+}
+
+// arrays of replica r's atom slots [atom0, atom0 + natom)
+Transfer xfer_vec(sld_ctx* c, const double4* d, const double* h, int r) {
+    return Transfer{d + c->reps[r].atom0, const_cast<double*>(h), (size_t)c->reps[r].natom, kXferVec};
+}
+Transfer xfer_scal(const double* d, const double* h, size_t off, size_t n) {
+    return Transfer{d + off, const_cast<double*>(h), n, kXferScalar};
+}
+
+int up4(sld_ctx* c, double4* d, const double* src, int r) { return stage_in(c, {xfer_vec(c, d, src, r)}); }
+
+// .w = |s| of a replica's spins, with the one rounding every other writer of .w uses
+int spin_lengths(sld_ctx* c, int r) {
+    const Rep& R = c->reps[r];
+    LAUNCH(c, k_spin_len, nblk(R.natom, 256), 256, c->D, R.atom0, R.natom);
     return SLD_OK;
 }
 
 // The caller's spin field of a replica: the spins, or with magmom the moments
-// m, from which the spins follow as s = m / (-g) (read_config.cpp:136-139)
-int up_spins(sld_ctx* c, const double* src, int r) {
-    if (!c->phys.magmom) return up4(c, c->D.s, src, r, true);
-    if (!src) return SLD_OK;
-    TRY(up4(c, c->D.m, src, r, false));
+// m, from which the spins follow as s = m / (-g) (read_config.cpp:136-139).
+// What the transferred field needs before it can be used:
+int spins_arrived(sld_ctx* c, int r) {
+    if (!c->phys.magmom) return spin_lengths(c, r);
     const Rep& R = c->reps[r];
     LAUNCH(c, k_magmom_s, nblk(R.natom, 256), 256, c->D, R.atom0, R.natom);
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     return SLD_OK;
-}
-
-// electron energy of a cell at Te (eV), in the arithmetic of heatcapacity_CPU.cpp:42-48
-double host_te_to_ee(double te) {
-    const double bb = 2e-4 / kBoltz;
-    return 3e0 / bb * std::log(std::cosh(bb * te));
 }
 
 int up1(sld_ctx* c, double* d, const double* src, size_t off, size_t n) {
-    if (!src) return SLD_OK;
-    HIPCHK(c, hipMemcpyAsync(d + off, src, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return SLD_OK;
-}
-
-int down4(sld_ctx* c, const double4* d, double* dst, int r) {
-    if (!dst) return SLD_OK;
-    const Rep& R = c->reps[r];
-    std::vector<double> h((size_t)R.natom * 4);
-    HIPCHK(c, hipMemcpyAsync(h.data(), d + R.atom0, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int i = 0; i < R.natom; ++i) {
-        dst[3 * i] = h[4 * i]; dst[3 * i + 1] = h[4 * i + 1]; dst[3 * i + 2] = h[4 * i + 2];
-    }
-    return SLD_OK;
-}
-
-int down1(sld_ctx* c, const double* d, double* dst, size_t off, size_t n) {
-    if (!dst) return SLD_OK;
-    HIPCHK(c, hipMemcpyAsync(dst, d + off, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return SLD_OK;
+    return stage_in(c, {xfer_scal(d, src, off, n)});
 }
 
 template <class T>
@@ -1281,23 +1396,14 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
             lz = std::min(std::max(lz, 0), hc.nz - 1);
             cell[R.atom0 + i] = R.cell0 + lx + ly * hc.nx + lz * hc.nx * hc.ny;
         }
-        TRY(up4(c, D.r, r3.data(), r, false));
-        TRY(up4(c, D.p, in->p, r, false));
-        TRY(up4(c, D.f, in->f, r, false));
-        TRY(up_spins(c, in->s, r));
-        TRY(up4(c, D.hh, in->heff_h, r, false));
-        TRY(up4(c, D.hl, in->heff_l, r, false));
-        TRY(up1(c, D.rho, in->rho, R.atom0, n));
-        TRY(up1(c, D.pe, in->pe, R.atom0, n));
-        TRY(up1(c, D.ke, in->ke, R.atom0, n));
-        TRY(up1(c, D.me, in->me, R.atom0, n));
-        TRY(up1(c, D.me0, in->me0, R.atom0, n));
-        if (in->stress)
-            for (int k = 0; k < 6; ++k) {
-                std::vector<double> st(n);
-                for (int i = 0; i < n; ++i) st[i] = in->stress[6 * i + k];
-                TRY(up1(c, D.stress, st.data(), (size_t)k * N + R.atom0, n));
-            }
+        double4* spins = P0.magmom ? D.m : D.s;
+        TRY(stage_in(c, {xfer_vec(c, D.r, r3.data(), r), xfer_vec(c, D.p, in->p, r), xfer_vec(c, D.f, in->f, r),
+                         xfer_vec(c, spins, in->s, r), xfer_vec(c, D.hh, in->heff_h, r),
+                         xfer_vec(c, D.hl, in->heff_l, r), xfer_scal(D.rho, in->rho, R.atom0, n),
+                         xfer_scal(D.pe, in->pe, R.atom0, n), xfer_scal(D.ke, in->ke, R.atom0, n),
+                         xfer_scal(D.me, in->me, R.atom0, n), xfer_scal(D.me0, in->me0, R.atom0, n),
+                         Transfer{D.stress + R.atom0, const_cast<double*>(in->stress), (size_t)n, kXferStress}}));
+        TRY(spins_arrived(c, r));
         for (int i = n - 1; i >= 0; --i) {
             const int a = R.atom0 + i, cc = cell[a];
             if (cn[cc] >= kCellCap)
@@ -1340,10 +1446,9 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
 
     // electron temperatures (map_cells.cpp:128-159)
     if (P0.eltemp) {
-        std::vector<double> te(C, P0.temperature), ee(C);
-        for (int k = 0; k < C; ++k) ee[k] = host_te_to_ee(te[k]);
+        const std::vector<double> te(C, P0.temperature);
         TRY(up1(c, D.Te, te.data(), 0, C));
-        TRY(up1(c, D.Ee, ee.data(), 0, C));
+        LAUNCH(c, k_ee_of_te, nblk(C, 256), 256, D, 0, C);
     }
     // initial.cpp:78-87 (with the densities of the input when they are not computed)
     TRY(nbuild(c, compute_forces ? 1 : 0));
@@ -1438,6 +1543,10 @@ int sld_destroy(sld_ctx* c) {
     drop_graphs(c);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
     for (void* p : c->allocs) (void)hipFree(p);
+    for (int k = 0; k < 2; ++k) {
+        if (c->h_stage[k]) (void)hipHostFree(c->h_stage[k]);
+        if (c->stage_ev[k]) (void)hipEventDestroy(c->stage_ev[k]);
+    }
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return SLD_OK;
@@ -1563,27 +1672,16 @@ int sld_download(sld_ctx* c, sld_atoms* o) {
     const int r = c->sel;
     const Rep& R = c->reps[r];
     const size_t a0 = R.atom0, n = R.natom;
-    TRY(down4(c, D.r, o->r, r)); TRY(down4(c, D.p, o->p, r)); TRY(down4(c, D.f, o->f, r));
-    TRY(down4(c, c->phys.magmom ? D.m : D.s, o->s, r));
-    TRY(down4(c, D.hh, o->heff_h, r)); TRY(down4(c, D.hl, o->heff_l, r));
-    TRY(down1(c, D.rho, o->rho, a0, n)); TRY(down1(c, D.pe, o->pe, a0, n)); TRY(down1(c, D.ke, o->ke, a0, n));
-    TRY(down1(c, D.me, o->me, a0, n)); TRY(down1(c, D.me0, o->me0, a0, n)); TRY(down1(c, D.vir, o->vir, a0, n));
-    TRY(down1(c, D.sjs, o->sum_jij_sj, a0, n));
-    if (o->local_volume) {
-        if (c->phys.localvol) {
-            TRY(down1(c, D.lvol, o->local_volume, a0, n));
-        } else {
-            // calculate_force_energy_CPU.cpp:276
-            for (size_t i = 0; i < n; ++i) o->local_volume[i] = R.box_volume / R.natom;
-        }
-    }
-    if (o->stress) {
-        std::vector<double> st(n);
-        for (int k = 0; k < 6; ++k) {
-            TRY(down1(c, D.stress, st.data(), (size_t)k * D.N + a0, n));
-            for (size_t i = 0; i < n; ++i) o->stress[6 * i + k] = st[i];
-        }
-    }
+    TRY(stage_out(c, {xfer_vec(c, D.r, o->r, r), xfer_vec(c, D.p, o->p, r), xfer_vec(c, D.f, o->f, r),
+                      xfer_vec(c, c->phys.magmom ? D.m : D.s, o->s, r), xfer_vec(c, D.hh, o->heff_h, r),
+                      xfer_vec(c, D.hl, o->heff_l, r), xfer_scal(D.rho, o->rho, a0, n), xfer_scal(D.pe, o->pe, a0, n),
+                      xfer_scal(D.ke, o->ke, a0, n), xfer_scal(D.me, o->me, a0, n), xfer_scal(D.me0, o->me0, a0, n),
+                      xfer_scal(D.vir, o->vir, a0, n), xfer_scal(D.sjs, o->sum_jij_sj, a0, n),
+                      xfer_scal(D.lvol, c->phys.localvol ? o->local_volume : nullptr, a0, n),
+                      Transfer{D.stress + a0, o->stress, n, kXferStress}}));
+    // calculate_force_energy_CPU.cpp:276
+    if (o->local_volume && !c->phys.localvol)
+        for (size_t i = 0; i < n; ++i) o->local_volume[i] = R.box_volume / R.natom;
     return SLD_OK;
 }
 
@@ -1593,11 +1691,10 @@ int sld_upload(sld_ctx* c, const sld_atoms* in) {
     Dev& D = c->D;
     const int r = c->sel;
     const Rep& R = c->reps[r];
-    TRY(up4(c, D.r, in->r, r, false));
-    TRY(up4(c, D.p, in->p, r, false));
-    TRY(up_spins(c, in->s, r));
-    TRY(up4(c, D.f, in->f, r, false));
-    TRY(up1(c, D.rho, in->rho, R.atom0, R.natom));
+    TRY(stage_in(c, {xfer_vec(c, D.r, in->r, r), xfer_vec(c, D.p, in->p, r),
+                     xfer_vec(c, c->phys.magmom ? D.m : D.s, in->s, r), xfer_vec(c, D.f, in->f, r),
+                     xfer_scal(D.rho, in->rho, R.atom0, R.natom)}));
+    if (in->s) TRY(spins_arrived(c, r));
     TRY(refresh_landau(c));
     if (in->r) c->nb_dirty = true;
     return SLD_OK;
@@ -1609,22 +1706,19 @@ int sld_get_cells(sld_ctx* c, sld_cells* o) {
     Dev& D = c->D;
     const Rep& R = c->reps[c->sel];
     const size_t c0 = R.cell0, n = R.ncell;
-    TRY(down1(c, D.Te, o->te, c0, n)); TRY(down1(c, D.Ee, o->ee, c0, n)); TRY(down1(c, D.Tl, o->tl, c0, n));
-    TRY(down1(c, D.TsR, o->ts_r, c0, n)); TRY(down1(c, D.TsL, o->ts_l, c0, n));
-    TRY(down1(c, D.Gel, o->gel, c0, n)); TRY(down1(c, D.Ges, o->ges, c0, n));
-    TRY(down1(c, D.sRup, o->sum_r_up, c0, n)); TRY(down1(c, D.sRdn, o->sum_r_dn, c0, n));
-    TRY(down1(c, D.sLup, o->sum_l_up, c0, n)); TRY(down1(c, D.sLdn, o->sum_l_dn, c0, n));
+    TRY(stage_out(c, {xfer_scal(D.Te, o->te, c0, n), xfer_scal(D.Ee, o->ee, c0, n), xfer_scal(D.Tl, o->tl, c0, n),
+                      xfer_scal(D.TsR, o->ts_r, c0, n), xfer_scal(D.TsL, o->ts_l, c0, n),
+                      xfer_scal(D.Gel, o->gel, c0, n), xfer_scal(D.Ges, o->ges, c0, n),
+                      xfer_scal(D.sRup, o->sum_r_up, c0, n), xfer_scal(D.sRdn, o->sum_r_dn, c0, n),
+                      xfer_scal(D.sLup, o->sum_l_up, c0, n), xfer_scal(D.sLdn, o->sum_l_dn, c0, n)}));
     return SLD_OK;
 }
 
 int sld_set_cells_te(sld_ctx* c, const double* te) {
     if (!c || !te) return SLD_ERR_ARG;
     const Rep& R = c->reps[c->sel];
-    // Ee = E(Te) on the host, as map_cells.cpp:154 and sld_create compute it
-    std::vector<double> ee(R.ncell);
-    for (int k = 0; k < R.ncell; ++k) ee[k] = host_te_to_ee(te[k]);
     TRY(up1(c, c->D.Te, te, R.cell0, R.ncell));
-    TRY(up1(c, c->D.Ee, ee.data(), R.cell0, R.ncell));
+    LAUNCH(c, k_ee_of_te, nblk(R.ncell, 256), 256, c->D, R.cell0, R.ncell);  // map_cells.cpp:154
     return SLD_OK;
 }
 
@@ -1719,8 +1813,8 @@ int sld_set_external(sld_ctx* c, const double* hext, const double* fext) {
     if (!c) return SLD_ERR_ARG;
     if (hext && !c->phys.extfield) return set_err(c, SLD_ERR_STATE, "extfield is off in sld_params");
     if (fext && !c->phys.extforce) return set_err(c, SLD_ERR_STATE, "extforce is off in sld_params");
-    TRY(up4(c, c->D.hext, hext, c->sel, false));
-    TRY(up4(c, c->D.fext, fext, c->sel, false));
+    TRY(up4(c, c->D.hext, hext, c->sel));
+    TRY(up4(c, c->D.fext, fext, c->sel));
     return SLD_OK;
 }
 

@@ -152,6 +152,24 @@ __global__ void k_renorm(Dev D, const double* err, double* partials);
 __global__ void k_reduce(const double* partials, int nblk, int nk, double* out);
 __global__ void k_reduce_seg(const double* partials, const int* seg, int nk, double* out, int out_off);
 __global__ void k_check_nonfinite(Dev D);
+__global__ void k_ee_of_te(Dev D, int c0, int n);
+// Transfers between device arrays and dense host arrays: run k of a piece is n
+// elements of seg[k].dev from element `first` on, at `offset` doubles of the
+// pinned buffer. kXferVec: double4 to 3 doubles (.w = 0 on the way in);
+// kXferStress: component-major [6][N] to 6 doubles an atom.
+enum { kXferScalar = 0, kXferVec = 1, kXferStress = 2 };
+constexpr int kXferSegs = 16;
+struct XferSeg {
+    const void* dev;
+    size_t first, n, offset;
+    int kind;
+};
+struct XferArgs {
+    XferSeg seg[kXferSegs];
+    int nseg;
+};
+__global__ void k_pack(XferArgs A, int N, double* buf);
+__global__ void k_unpack(XferArgs A, int N, const double* buf);
 __global__ void k_spin_len(Dev D, int a0, int n);
 
 // ---- parametric potential model (sld_model.hip) ----

@@ -1083,6 +1083,63 @@ __global__ __launch_bounds__(256) void k_renorm(Dev D, const double* err, double
     block_partials<1>(acc, partials);
 }
 
+// Ee = E(Te) of cells [c0, c0 + n) (map_cells.cpp:128-159)
+__global__ __launch_bounds__(256) void k_ee_of_te(Dev D, int c0, int n) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) D.Ee[c0 + k] = te_to_ee(D.Te[c0 + k]);
+}
+
+// One run of a piece per blockIdx.y, one thread per element. The buffer is
+// pinned host memory: a vector's three doubles are written through LDS as
+// contiguous lines (a block's 6 KB), so the bus sees whole bursts.
+__global__ __launch_bounds__(256) void k_pack(XferArgs A, int N, double* buf) {
+    __shared__ double sh[6 * 256];
+    const XferSeg& g = A.seg[blockIdx.y];
+    const int t = threadIdx.x;
+    const size_t e0 = (size_t)blockIdx.x * 256;
+    if (e0 >= g.n) return;
+    const int m = (int)(g.n - e0 < 256 ? g.n - e0 : 256);
+    const size_t i = g.first + e0 + t;
+    const int w = g.kind == kXferVec ? 3 : g.kind == kXferStress ? 6 : 1;
+    if (t < m) {
+        if (g.kind == kXferVec) {
+            const double4 v = static_cast<const double4*>(g.dev)[i];
+            sh[3 * t] = v.x; sh[3 * t + 1] = v.y; sh[3 * t + 2] = v.z;
+        } else if (g.kind == kXferStress) {
+            const double* d = static_cast<const double*>(g.dev);
+            for (int k = 0; k < 6; ++k) sh[6 * t + k] = d[(size_t)k * N + i];
+        } else {
+            sh[t] = static_cast<const double*>(g.dev)[i];
+        }
+    }
+    __syncthreads();
+    double* out = buf + g.offset + e0 * w;
+    for (int k = t; k < m * w; k += 256) out[k] = sh[k];
+}
+
+__global__ __launch_bounds__(256) void k_unpack(XferArgs A, int N, const double* buf) {
+    __shared__ double sh[6 * 256];
+    const XferSeg& g = A.seg[blockIdx.y];
+    const int t = threadIdx.x;
+    const size_t e0 = (size_t)blockIdx.x * 256;
+    if (e0 >= g.n) return;
+    const int m = (int)(g.n - e0 < 256 ? g.n - e0 : 256);
+    const size_t i = g.first + e0 + t;
+    const int w = g.kind == kXferVec ? 3 : g.kind == kXferStress ? 6 : 1;
+    const double* in = buf + g.offset + e0 * w;
+    for (int k = t; k < m * w; k += 256) sh[k] = in[k];
+    __syncthreads();
+    if (t >= m) return;
+    void* dev = const_cast<void*>(g.dev);
+    if (g.kind == kXferVec) {
+        static_cast<double4*>(dev)[i] = make_double4(sh[3 * t], sh[3 * t + 1], sh[3 * t + 2], 0.0);
+    } else if (g.kind == kXferStress) {
+        for (int k = 0; k < 6; ++k) static_cast<double*>(dev)[(size_t)k * N + i] = sh[6 * t + k];
+    } else {
+        static_cast<double*>(dev)[i] = sh[t];
+    }
+}
+
 // .w = |s| over the atom slots [a0, a0 + n), after the host uploaded spins
 __global__ __launch_bounds__(256) void k_spin_len(Dev D, int a0, int n) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
