@@ -318,6 +318,14 @@ __device__ __forceinline__ double wave_sum(double v) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// LDS written by one lane of the wave and read by another: the accesses of a
+// wave complete in order, the compiler has to keep them so
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // partials[k * blocks + block] = the block's sum of v[k] (blocks of up to 256
 // threads, whole waves): wave sums, then those in order
 template <int NK>

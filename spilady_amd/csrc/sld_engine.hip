@@ -190,12 +190,13 @@ hipEvent_t* timing_slot(sld_ctx* c, const char* name) {
     return ev;
 }
 
-#define LAUNCH(ctx, kern, grid, block, ...)                                              \
+#define LAUNCH(ctx, kern, grid, block, ...) LAUNCH_LDS(ctx, kern, grid, block, 0, __VA_ARGS__)
+#define LAUNCH_LDS(ctx, kern, grid, block, lds, ...)                                     \
     do {                                                                                 \
         if ((grid) > 0) {                                                                \
             hipEvent_t* ev_ = timing_slot((ctx), #kern);                                 \
             if (ev_) (void)hipEventRecord(ev_[0], (ctx)->stream);                        \
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, (ctx)->stream, __VA_ARGS__); \
+            hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, (ctx)->stream, __VA_ARGS__); \
             hipError_t e_ = hipGetLastError();                                           \
             if (e_ != hipSuccess)                                                        \
                 return set_err((ctx), SLD_ERR_HIP, "launch %s: %s", #kern, hipGetErrorString(e_)); \
@@ -348,7 +349,7 @@ int refresh_landau(sld_ctx* c) {
 
 int nbuild(sld_ctx* c, int write_rho) {
     const int w = c->shapes.nbuild_cells;
-    LAUNCH(c, k_nbuild, xcd_grid(nblk(c->D.C, w)), 64 * w, c->tab, c->phys, c->D, write_rho);
+    LAUNCH_LDS(c, k_nbuild, xcd_grid(nblk(c->D.C, w)), 64 * w, w * kNbLds, c->tab, c->phys, c->D, write_rho);
     c->nb_dirty = false;
     if (write_rho) TRY(refresh_landau(c));
     return SLD_OK;

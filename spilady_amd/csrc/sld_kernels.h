@@ -92,6 +92,8 @@ constexpr int kSeg = 8;
 // ---- kernels ----
 __global__ void k_bin(Dev D);
 __global__ void k_relink(const int* cl_old, const int* cn_old, Dev D);
+// dynamic LDS of k_nbuild, bytes a wave
+constexpr int kNbLds = 256 * 16 + 27 * kCellCap * 4;
 __global__ void k_nbuild(Tables T, Phys P, Dev D, int write_rho);
 __global__ void k_fp(Tables T, Dev D);
 __global__ void k_force(Tables T, Phys P, Dev D);

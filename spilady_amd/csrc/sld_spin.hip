@@ -126,14 +126,6 @@ constexpr int kSpinPairs = 496;   // and pairs of atoms of one cell (one of 32, 
 static_assert(kSpinAtoms >= kCellCap && kSpinPairs >= kCellCap * (kCellCap - 1) / 2, "any one cell fits a pass");
 static_assert(kMaxMag == 32, "four lanes hold an atom's list in two chunks of four each");
 
-// LDS written by one lane of the wave and read by another: the accesses of a
-// wave complete in order, the compiler has to keep them so
-__device__ __forceinline__ void wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // lanes: lanes that walk a cell, a power of two with ncw * lanes <= 64
 template <bool kLang>
 __global__ __launch_bounds__(64) void k_spin_phase(const int* cells, int ncell, int ncw, int lanes, int backward,
