@@ -42,16 +42,19 @@ __device__ __forceinline__ double rsqrt_normal(double x) {
     const double e = fma(-x * y, y, 1.0);
     return fma(y * e, fma(0.375, e, 0.5), y);
 }
+// sqrt(x) of any x
+__device__ __forceinline__ double sqrt_any(double x) {
+    double r = sqrt_normal(x);
+    if (__builtin_expect(!(x >= 1e-200 && x <= 1e200), 0)) r = sqrt(x);
+    return r;
+}
 // |s|, the value every spin's .w payload holds. It is the only definition of
 // that value: the field sums read a neighbour's .w where the reference takes
 // vec_length(s_j) (calculate_spin_CPU.cpp:265), so every writer of .w must
 // round it the same way. The explicit fma order leaves the compiler no
 // contraction choice that could differ between kernels.
 __device__ __forceinline__ double spin_len(double3 s) {
-    const double x = fma(s.z, s.z, fma(s.x, s.x, s.y * s.y));
-    double r = sqrt_normal(x);
-    if (__builtin_expect(!(x >= 1e-200 && x <= 1e200), 0)) r = sqrt(x);
-    return r;
+    return sqrt_any(fma(s.z, s.z, fma(s.x, s.x, s.y * s.y)));
 }
 __device__ __forceinline__ double3 cross3(double3 a, double3 b) {
     return make_double3(a.y * b.z - b.y * a.z, a.z * b.x - b.z * a.x, a.x * b.y - b.x * a.y);

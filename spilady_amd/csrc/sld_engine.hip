@@ -384,35 +384,34 @@ int do_force(sld_ctx* c) {
     return SLD_OK;
 }
 
-// A level's cells are spread over this many waves if that leaves at least one
-// a wave: two a SIMD, so that small levels use the whole chip (4,913 cells: 15.0
-// us with 3 cells a wave, 19.6 with 8).
-constexpr int kSpinWaves = 2048;
-// Within a level the cells are listed in windows of neighbours, sorted by
-// descending atom count inside a window.
-constexpr int kSpinWindow = 512;
+// Cells a wave of the spin sweep takes: spin_block / 16 (4 by default: 2 M
+// atoms 33.5 us a level, 34.2 with 8 and 36.1 with 9), fewer where a wave's 64
+// lanes hold fewer cells of the mean size with some room, and fewer where the
+// level would leave waves idle, spread over this many times spin_lanes (2,048
+// by default, two a SIMD: levels of 4,913 cells 12.5 us, 18 with 512).
+constexpr int kSpinLanes = 58;
+constexpr int kSpinWaves = 512;
 
 int do_ds(sld_ctx* c, double dt) {
     TRY(ensure_nb(c));
     double dth = dt / 2.0;
     if (c->phys.magmom) LAUNCH(c, k_magmom_s, nblk(c->D.N, 256), 256, c->D, 0, c->D.N);
+    const int fit = (int)((int64_t)kSpinLanes * c->D.C / std::max(c->D.N, 1));
     for (int dir = 0; dir < 2; ++dir) {
         LevelSet& L = dir == 0 ? c->spin_fwd : c->spin_bwd;
         if (c->phys.spinlang)
             LAUNCH(c, k_spin_noise, nblk(c->D.N, 256), 256, c->D, (int)(c->pass - c->pass_dev));
         for (int l = 0; l < L.nlev(); ++l) {
             const int n = L.off[l + 1] - L.off[l];
-            const int ncw = std::max(1, std::min(c->shapes.spin_block / 8, nblk(n, kSpinWaves)));
-            // lanes of a wave that its cells leave idle help to spread the changes
-            int lanes = c->shapes.spin_lanes;
-            while (lanes < 4 * c->shapes.spin_lanes && 2 * lanes * ncw <= 64) lanes *= 2;
+            const int ncw = std::max(1, std::min({c->shapes.spin_block / 16, fit,
+                                                  nblk(n, kSpinWaves * c->shapes.spin_lanes)}));
             const int nw = xcd_grid(nblk(n, ncw));
             const int* cells = L.d_cells + L.off[l];
             // only the backward sweep's Heff_H, Heff_L and sum J|s_j| last
             if (c->phys.spinlang)
-                LAUNCH(c, k_spin_phase<true>, nw, 64, cells, n, ncw, lanes, dir, dir, dth, c->phys, c->D);
+                LAUNCH(c, k_spin_phase<true>, nw, 64, cells, n, ncw, dir, dir, dth, c->phys, c->D);
             else
-                LAUNCH(c, k_spin_phase<false>, nw, 64, cells, n, ncw, lanes, dir, dir, dth, c->phys, c->D);
+                LAUNCH(c, k_spin_phase<false>, nw, 64, cells, n, ncw, dir, dir, dth, c->phys, c->D);
         }
         c->pass++;
     }
@@ -1429,18 +1428,6 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
     HIPCHK(c, hipStreamSynchronize(c->stream));
     merge_levels(sf, c->reps, c->spin_fwd);
     merge_levels(sb, c->reps, c->spin_bwd);
-    // A wave of the spin sweep walks as many atoms as its fullest cell holds,
-    // and the cells of one level are independent, so cells of like starting
-    // atom count share a wave. Sorted over the whole level, neighbouring cells
-    // would run far apart and fetch the spins they share again: windows of 512
-    // cells read 0.84 M lines a launch at 2 M atoms, the whole level 1.1 M, and
-    // take 41.7 us against 47.8. The order of a level does not change any result.
-    for (LevelSet* L : {&c->spin_fwd, &c->spin_bwd})
-        for (int l = 0; l < L->nlev(); ++l)
-            for (int k = L->off[l]; k < L->off[l + 1]; k += kSpinWindow)
-                std::stable_sort(L->cells.begin() + k,
-                                 L->cells.begin() + std::min(k + kSpinWindow, L->off[l + 1]),
-                                 [&](int a, int b) { return cn[a] > cn[b]; });
     TRY(upload_levels(c, c->spin_fwd));
     TRY(upload_levels(c, c->spin_bwd));
     if (nrep == 1) TRY(upload_dte_schedules(c));

@@ -110,12 +110,11 @@ __global__ void k_reduce_max2(const double* partials, int nblk, double* out);
 __global__ void k_pass_advance(Dev D, int n);
 __global__ void k_qn_init(Phys P, Dev D);
 __global__ void k_qn_refresh(Phys P, Dev D, uint64_t r);
-// ncw <= 16 cells a wave, lanes (a power of two) that walk a cell, ncw * lanes
-// <= 64; store_fields: write Heff_H, Heff_L and sum J|s_j| (the backward sweep
-// of a core_ds call)
+// ncw <= 16 cells a wave; store_fields: write Heff_H, Heff_L and sum J|s_j|
+// (the backward sweep of a core_ds call)
 template <bool kLang>
-__global__ void k_spin_phase(const int* cells, int ncell, int ncw, int lanes, int backward, int store_fields,
-                             double dt, Phys P, Dev D);
+__global__ void k_spin_phase(const int* cells, int ncell, int ncw, int backward, int store_fields, double dt,
+                             Phys P, Dev D);
 __global__ void k_dp_cells(double dt, Phys P, Dev D, int pass_off, double* partials);
 __global__ void k_dp_center(Phys P, Dev D, const double* scal, double* partials);
 __global__ void k_dp_scale(Phys P, Dev D, const double* scal);

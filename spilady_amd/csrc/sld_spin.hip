@@ -94,47 +94,57 @@ __device__ __forceinline__ double quad_sum(double v) {
     return v + quad_swap<2>(v);
 }
 
+// value of the lane N places before in the row of 16, or 0
+template <int N>
+__device__ __forceinline__ int row_shr(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x110 + N, 0xf, 0xf, true);
+}
+
+// v | the values of the other three lanes of the quad
+__device__ __forceinline__ unsigned quad_or(unsigned v) {
+    v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, true);
+    return v | (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, true);
+}
+
 // One dependency level of a core_ds sweep: each listed cell walks its list
 // head to tail (forward) or tail to head (backward)
 // (calculate_spin_CPU.cpp:33-235, core_ds_CPU.cpp:35-83).
 //
 // Cells of a level do not interact, so all a walk can miss of its neighbours
-// are the new spins of its own cell's earlier atoms. A wave takes up to 16
-// cells in two phases:
-// 1. four lanes per atom: the field H = Hext + sum J s_j and S = sum J|s_j|
+// are the new spins of its own cell's earlier atoms. And of those it needs only
+// the ones within the exchange range: an atom whose earlier neighbours in the
+// cell are done can be updated, whatever else is still to come. A wave takes
+// the cells that fit its 64 lanes, a lane per atom:
+// 1. four lanes gather an atom's field H = Hext + sum J s_j and S = sum J|s_j|
 //    over the spins as they are, lane j adding list entries 4j..4j+3 and
 //    4j+16..4j+19; J of each pair of atoms of one cell goes into a triangle in
-//    LDS;
-// 2. the lanes of a cell walk it: an atom is updated from LDS alone, and what
-//    its spin changed by is added to the fields of the cell's later atoms.
+//    LDS, and the atom's earlier neighbours into a bit mask;
+// 2. in each round the atoms that wait for none are updated, and then every
+//    atom adds J times their change to its own field, in walking order.
 // The sum H + sum J (s_new - s_old) is the field of the sequential walk up to
-// the rounding of the corrections. Every lane of a cell computes the same
-// update and the additions to one field come in walking order, so the result
-// does not depend on the lanes, nor on the cells per wave.
+// the rounding of the corrections. A cell's rounds depend on its own atoms
+// only, so the result does not depend on how many cells share a wave.
 //
 // A walk that loads as it goes waits for memory once an atom and fetches a
 // neighbour's line again for every atom that reads it; here a launch waits
-// about four times in all. What is left is the update itself, 240 instructions
-// a visit (about 0.7 us for a wave on its own) and, at 2 M atoms, the traffic:
-// 41.7 us a level on average (108 MB) where the walk took 46 (164 MB); levels
-// of 27 cells of 9 atoms 18.5 us instead of 30, of 960 cells 15.0 instead of 18.
-// LDS is kept to 14 KB for 11 waves a compute unit: with 22 KB (16 cells a
-// wave) 2 M atoms took 50 us.
+// about four times in all. The update is a chain of 240 instructions, about 0.7
+// us for a wave on its own, so rounds count: cells of 9.3 atoms on average and
+// 16 at most need 6.1 and 9 of them, cells of 6.5 and 10 need 4.9 and 6.
+// At 27 cells a launch that leaves 3 us of launch, 2 of first loads, 1 of
+// gathering and 4 of rounds: 9.7 us where the walk atom by atom took 16.5. Of
+// 2 M atoms a level moves 108 MB in 31.1 us (39.5); registers are kept to 128 for
+// four waves a SIMD, the atoms' own values loaded after the gathering (before
+// it: 150 registers, 1 us more at 64 x 16,000 atoms, 0.2 less at 2,000).
 
-constexpr int kSpinAtoms = 80;    // atoms of a wave's pass in LDS (8 cells of 10)
-constexpr int kSpinPairs = 496;   // and pairs of atoms of one cell (one of 32, 8 of 11)
-static_assert(kSpinAtoms >= kCellCap && kSpinPairs >= kCellCap * (kCellCap - 1) / 2, "any one cell fits a pass");
+constexpr int kSpinPairs = 496;  // pairs of atoms of one cell in a pass (one of 32, 8 of 11)
+static_assert(kCellCap <= 32 && kSpinPairs >= kCellCap * (kCellCap - 1) / 2, "any one cell fits a pass");
 static_assert(kMaxMag == 32, "four lanes hold an atom's list in two chunks of four each");
 
-// lanes: lanes that walk a cell, a power of two with ncw * lanes <= 64
 template <bool kLang>
-__global__ __launch_bounds__(64) void k_spin_phase(const int* cells, int ncell, int ncw, int lanes, int backward,
+__global__ __launch_bounds__(64) void k_spin_phase(const int* cells, int ncell, int ncw, int backward,
                                                    int store_fields, double dt, Phys P, Dev D) {
-    __shared__ double sH[4][kSpinAtoms];              // field x, y, z and sum J|s_j|
-    __shared__ double sS[4][kSpinAtoms];              // spin x, y, z and its length
-    __shared__ double sZ[kLang ? 3 : 1][kSpinAtoms];  // Langevin normals
-    __shared__ double sL[kLang ? 4 : 1][kSpinAtoms];  // Landau coefficients
-    __shared__ int sA[kSpinAtoms];                    // atom
+    __shared__ double sV[4][64];  // phase 1: field x, y, z and sum J|s_j|; phase 2: change of the spin and its length
+    __shared__ unsigned sM[64];   // bit q: the atom's neighbour at place q of its cell's walk comes earlier
     __shared__ double sJ[kSpinPairs];
     const int lane = threadIdx.x;
     const int lb = xcd_block((ncell + ncw - 1) / ncw);
@@ -145,63 +155,76 @@ __global__ __launch_bounds__(64) void k_spin_phase(const int* cells, int ncell, 
         c = cells[lb * ncw + lane];
         n = D.cn[c];
     }
-    // atoms and pairs of the cells up to this lane's
-    int atoms = n, pairs = n * (n - 1) / 2;
-#pragma unroll
-    for (int d = 1; d < 16; d <<= 1) {
-        const int ta = __shfl_up(atoms, d, 64), tp = __shfl_up(pairs, d, 64);
-        if (lane >= d) {
-            atoms += ta;
-            pairs += tp;
-        }
-    }
-    const int atom0 = atoms - n, pair0 = pairs - n * (n - 1) / 2;
+    // atoms and pairs of the cells before this lane's, in the low and the high half
+    const int own_sum = n | (n * (n - 1) / 2) << 16;
+    int sum = own_sum;
+    sum += row_shr<1>(sum);
+    sum += row_shr<2>(sum);
+    sum += row_shr<4>(sum);
+    sum += row_shr<8>(sum);
+    const int atoms = sum & 0xffff, pairs = sum >> 16;
+    const int sum0 = sum - own_sum;
     const double dth = dt / 2.0, gS = P.gamma_S;
-    const double ch = gS * dth, cq = gS * (dt / 4.0);
-    double cz = 0.0;
-    if (kLang && c >= 0) {
-        const double Tk = P.eltemp ? D.Te[c] : D.rep[D.crep[c]].temperature;
-        cz = dt * sqrt(2.0 * Tk * gS / dt);
-    }
-    // passes over as many cells as fit in LDS
+    const double ch = gS * dth, cq = gS * (dt / 4.0), noise = 2.0 * gS / dt;
+    // passes over as many cells as fit the lanes and the triangles
     for (int k0 = 0; k0 < ncw;) {
-        const int a0 = __builtin_amdgcn_readlane(atom0, k0), p0 = __builtin_amdgcn_readlane(pair0, k0);
+        const int s0 = __builtin_amdgcn_readlane(sum0, k0), a0 = s0 & 0xffff, p0 = s0 >> 16;
         const unsigned long long fit =
-            __ballot(lane >= k0 && lane < ncw && atoms - a0 <= kSpinAtoms && pairs - p0 <= kSpinPairs);
+            __ballot(lane >= k0 && lane < ncw && atoms - a0 <= 64 && pairs - p0 <= kSpinPairs);
         const int k1 = k0 + __builtin_ctzll(~(fit >> k0));  // cells [k0, k1)
         const int natom = __builtin_amdgcn_readlane(atoms, k1 - 1) - a0;
-        const int npair = __builtin_amdgcn_readlane(pairs, k1 - 1) - p0;
-        for (int i = lane; i < npair; i += 64) sJ[i] = 0.0;
-        wave_fence();
+        // this lane's atom: cell ck of nk atoms, the first of them in lane base, place q in its walk
+        int ck = __builtin_amdgcn_readlane(c, k0), nk = __builtin_amdgcn_readlane(n, k0), base = 0, tri = 0;
+        for (int u = k0 + 1; u < k1; ++u) {
+            const int su = __builtin_amdgcn_readlane(sum0, u) - s0;
+            const int cu = __builtin_amdgcn_readlane(c, u), nu = __builtin_amdgcn_readlane(n, u);
+            if (lane >= (su & 0xffff)) {
+                ck = cu;
+                nk = nu;
+                base = su & 0xffff;
+                tri = su >> 16;
+            }
+        }
+        const int q = lane - base;
+        tri += q * (q - 1) / 2;  // pairs of the atom and its predecessors
+        const bool mine = lane < natom;
+        int a = 0, rep = 0;
+        double Tk = 0.0;
+        double4 own = make_double4(0.0, 0.0, 0.0, 0.0), lc = own, zn = own;
+        double3 H = d3(own);
+        if (mine) {
+            a = D.cl[ck * kCellCap + (backward ? nk - 1 - q : q)];
+            if (kLang && !P.eltemp) rep = D.crep[ck];
+        }
         const int j = lane & 3;
+        const int place = (tri << 16) | (q << 8) | nk;
         for (int f0 = 0; f0 < natom; f0 += 16) {
             const int f = f0 + (lane >> 2);
-            int k = k0;
-            for (int q = k0 + 1; q < k1; ++q) k += f >= __builtin_amdgcn_readlane(atom0, q) - a0 ? 1 : 0;
-            const int ck = __shfl(c, k, 64), nk = __shfl(n, k, 64);
-            const int q = f - (__shfl(atom0, k, 64) - a0);
-            double* tri = sJ + (__shfl(pair0, k, 64) - p0) + q * (q - 1) / 2;  // pairs of the atom and its predecessors
+            const int af = __shfl(a, f, 64), cf = __shfl(ck, f, 64), pf = __shfl(place, f, 64);
+            const int qf = (pf >> 8) & 255, nf = pf & 255;
+            double* trif = sJ + (pf >> 16);
             if (f < natom) {
-                const int a = D.cl[ck * kCellCap + (backward ? nk - 1 - q : q)];
-                const int nm = D.nbmn[a];
-                // lane j's part of what the update needs besides the field
-                double4 own = make_double4(0.0, 0.0, 0.0, 0.0), he = own;
-                if (j == 0) own = D.s[a];
-                if (kLang && j == 1) own = D.zn[a];
-                if (kLang && j == 2) own = D.lan[a];
-                if (P.extfield && j == 0) he = D.hext[a];
-                double hx = he.x, hy = he.y, hz = he.z, ss = 0.0;
+                double hx = 0.0, hy = 0.0, hz = 0.0, ss = 0.0;
+                unsigned earlier = 0;
+                // the first chunk's ids and J do not wait for the list's length
+                const int* ids = D.nbm + (size_t)af * kMaxMag + 4 * j;
+                const double2* js = reinterpret_cast<const double2*>(D.nbJ + (size_t)af * kMaxMag + 4 * j);
+                int4 i0 = *reinterpret_cast<const int4*>(ids);
+                double2 j0 = js[0], j1 = js[1];
+                const int nm = D.nbmn[af];
                 for (int b0 = 4 * j; b0 < nm; b0 += 16) {
-                    const int4 i0 = *reinterpret_cast<const int4*>(D.nbm + (size_t)a * kMaxMag + b0);
-                    const double2* js = reinterpret_cast<const double2*>(D.nbJ + (size_t)a * kMaxMag + b0);
-                    const double2 j0 = js[0], j1 = js[1];
+                    if (b0 >= 16) {
+                        i0 = *reinterpret_cast<const int4*>(ids + 16);
+                        j0 = js[8];
+                        j1 = js[9];
+                    }
                     int id[4] = {i0.x, i0.y, i0.z, i0.w};
                     const double J[4] = {j0.x, j0.y, j1.x, j1.y};
                     double4 sj[4];
                     int sl[4];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        if (b0 + e >= nm) id[e] = a;
+                        if (b0 + e >= nm) id[e] = af;
                         sj[e] = D.s[id[e]];
                         sl[e] = D.cslot[id[e]];
                     }
@@ -212,96 +235,101 @@ __global__ __launch_bounds__(64) void k_spin_phase(const int* cells, int ncell, 
                         hy = fma(Je, sj[e].y, hy);
                         hz = fma(Je, sj[e].z, hz);
                         ss = fma(Je, sj[e].w, ss);
-                        const int pos = sl[e] - ck * kCellCap;  // in the list of this cell if 0 <= pos < nk
-                        const int qe = backward ? nk - 1 - pos : pos;
-                        if ((unsigned)pos < (unsigned)nk && qe < q && b0 + e < nm) tri[qe] = Je;
+                        const int pos = sl[e] - cf * kCellCap;  // in the list of this cell if 0 <= pos < nf
+                        const int qe = backward ? nf - 1 - pos : pos;
+                        if ((unsigned)pos < (unsigned)nf && qe < qf && b0 + e < nm) {
+                            trif[qe] = Je;
+                            earlier |= 1u << qe;
+                        }
                     }
                 }
                 hx = quad_sum(hx);
                 hy = quad_sum(hy);
                 hz = quad_sum(hz);
                 ss = quad_sum(ss);
-                if (j == 0) {
-                    sS[0][f] = own.x; sS[1][f] = own.y; sS[2][f] = own.z; sS[3][f] = own.w;
-                    sA[f] = a;
-                }
-                if (kLang && j == 1) {
-                    sZ[0][f] = own.x; sZ[kLang ? 1 : 0][f] = own.y; sZ[kLang ? 2 : 0][f] = own.z;
-                }
-                if (kLang && j == 2) {
-                    sL[0][f] = -2.0 * own.x; sL[kLang ? 1 : 0][f] = -4.0 * own.y;
-                    sL[kLang ? 2 : 0][f] = -6.0 * own.z; sL[kLang ? 3 : 0][f] = -8.0 * own.w;
-                }
-                if (j == 3) {
-                    sH[0][f] = hx; sH[1][f] = hy; sH[2][f] = hz; sH[3][f] = ss;
-                }
+                earlier = quad_or(earlier);
+                sV[j][f] = j == 0 ? hx : j == 1 ? hy : j == 2 ? hz : ss;
+                if (j == 0) sM[f] = earlier;
             }
         }
+        if (mine) {
+            own = D.s[a];
+            if (kLang) {
+                lc = D.lan[a];
+                zn = D.zn[a];
+                Tk = P.eltemp ? D.Te[ck] : D.rep[rep].temperature;
+            }
+            if (P.extfield) H = d3(D.hext[a]);
+        }
         wave_fence();
-        const int k = k0 + lane / lanes, sub = lane & (lanes - 1);
-        const int kk = min(k, k1 - 1);
-        const int nk = __shfl(n, kk, 64);
-        const int base = __shfl(atom0, kk, 64) - a0;
-        const double* tri0 = sJ + (__shfl(pair0, kk, 64) - p0);
-        const double ck = __shfl(cz, kk, 64);
-        const int nw = k < k1 ? nk : 0;
-        for (int q = 0; q < nw; ++q) {
-            const int f = base + q;
-            const double3 H = make_double3(sH[0][f], sH[1][f], sH[2][f]);
-            const double S = sH[3][f];
-            const double4 old = make_double4(sS[0][f], sS[1][f], sS[2][f], sS[3][f]);
-            const int a = sA[f];
-            double3 s = d3(old);
-            double3 L = make_double3(0.0, 0.0, 0.0);
-            if (!kLang) {
-                s = apply_rot(make_rot(H, dt), s);
-            } else {
-                const double4 lc = make_double4(sL[0][f], sL[kLang ? 1 : 0][f], sL[kLang ? 2 : 0][f],
-                                                sL[kLang ? 3 : 0][f]);
-                // s + c (H + m v): a stage of the RK2 of the damping, m v the Landau field at v
-                auto stage = [&](double3 at, double c, double m, double3 v) {
-                    return make_double3(fma(c, fma(m, v.x, H.x), at.x), fma(c, fma(m, v.y, H.y), at.y),
-                                        fma(c, fma(m, v.z, H.z), at.z));
-                };
-                const Rot R = make_rot(H, dth);
-                s = apply_rot(R, s);
-                double3 st = stage(s, cq, landau_scale(s, lc, S), s);
-                s = stage(s, ch, landau_scale(st, lc, S), st);
-                s = make_double3(fma(ck, sZ[0][f], s.x), fma(ck, sZ[kLang ? 1 : 0][f], s.y),
-                                 fma(ck, sZ[kLang ? 2 : 0][f], s.z));
-                st = stage(s, cq, landau_scale(s, lc, S), s);
-                const double m = landau_scale(st, lc, S);
-                s = stage(s, ch, m, st);
-                L = mul3(m, st);
-                s = apply_rot(R, s);
-            }
-            const double w = spin_len(s);
-            const double3 ds = sub3(s, d3(old));
-            const double dw = w - old.w;
-            for (int p = q + 1 + sub; p < nk; p += lanes) {
-                const double J = tri0[p * (p - 1) / 2 + q];
-                const int g = base + p;
-                sH[0][g] = fma(J, ds.x, sH[0][g]);
-                sH[1][g] = fma(J, ds.y, sH[1][g]);
-                sH[2][g] = fma(J, ds.z, sH[2][g]);
-                sH[3][g] = fma(J, dw, sH[3][g]);
-            }
-            if (sub == 0) {
-                D.s[a] = make_double4(s.x, s.y, s.z, w);
-                // the fields of the forward sweep are overwritten by the
-                // backward sweep before anything reads them
-                if (store_fields) {
-                    if (kLang) D.sjs[a] = S;
-                    D.hh[a] = make_double4(H.x, H.y, H.z, 0.0);
-                    D.hl[a] = make_double4(L.x, L.y, L.z, 0.0);
+        double S = 0.0;
+        unsigned long long earlier = 0;  // lanes whose atoms this one waits for
+        if (mine) {
+            H = make_double3(H.x + sV[0][lane], H.y + sV[1][lane], H.z + sV[2][lane]);
+            S = sV[3][lane];
+            earlier = (unsigned long long)sM[lane] << base;
+        }
+        wave_fence();
+        lc = make_double4(-2.0 * lc.x, -4.0 * lc.y, -6.0 * lc.z, -8.0 * lc.w);
+        const double czk = dt * sqrt_any(Tk * noise);
+        const double* J0 = sJ + tri - base;  // J0[u]: with the atom of lane u
+        double3 s = d3(own), L = make_double3(0.0, 0.0, 0.0);
+        double w = own.w;
+        // a round ends at least the first atom of each walk that is not done
+        const unsigned long long all = natom < 64 ? (1ull << natom) - 1 : ~0ull;
+        for (unsigned long long done = 0; done != all;) {
+            const bool ready = mine && !((done >> lane) & 1) && !(earlier & ~done);
+            const unsigned long long now = __ballot(ready);
+            if (ready) {
+                if (!kLang) {
+                    s = apply_rot(make_rot(H, dt), s);
+                } else {
+                    // s + c (H + m v): a stage of the RK2 of the damping, m v the Landau field at v
+                    auto stage = [&](double3 at, double c, double m, double3 v) {
+                        return make_double3(fma(c, fma(m, v.x, H.x), at.x), fma(c, fma(m, v.y, H.y), at.y),
+                                            fma(c, fma(m, v.z, H.z), at.z));
+                    };
+                    const Rot R = make_rot(H, dth);
+                    s = apply_rot(R, s);
+                    double3 st = stage(s, cq, landau_scale(s, lc, S), s);
+                    s = stage(s, ch, landau_scale(st, lc, S), st);
+                    s = make_double3(fma(czk, zn.x, s.x), fma(czk, zn.y, s.y), fma(czk, zn.z, s.z));
+                    st = stage(s, cq, landau_scale(s, lc, S), s);
+                    const double m = landau_scale(st, lc, S);
+                    s = stage(s, ch, m, st);
+                    L = mul3(m, st);
+                    s = apply_rot(R, s);
                 }
+                w = spin_len(s);
+                sV[0][lane] = s.x - own.x;
+                sV[1][lane] = s.y - own.y;
+                sV[2][lane] = s.z - own.z;
+                sV[3][lane] = w - own.w;
             }
             wave_fence();
+            for (unsigned long long m = earlier & now; m; m &= m - 1) {
+                const int u = __builtin_ctzll(m);
+                const double J = J0[u];
+                H = make_double3(fma(J, sV[0][u], H.x), fma(J, sV[1][u], H.y), fma(J, sV[2][u], H.z));
+                S = fma(J, sV[3][u], S);
+            }
+            wave_fence();
+            done |= now;
+        }
+        if (mine) {
+            D.s[a] = make_double4(s.x, s.y, s.z, w);
+            // the fields of the forward sweep are overwritten by the
+            // backward sweep before anything reads them
+            if (store_fields) {
+                if (kLang) D.sjs[a] = S;
+                D.hh[a] = make_double4(H.x, H.y, H.z, 0.0);
+                D.hl[a] = make_double4(L.x, L.y, L.z, 0.0);
+            }
         }
         k0 = k1;
     }
 }
-template __global__ void k_spin_phase<false>(const int*, int, int, int, int, int, double, Phys, Dev);
-template __global__ void k_spin_phase<true>(const int*, int, int, int, int, int, double, Phys, Dev);
+template __global__ void k_spin_phase<false>(const int*, int, int, int, int, double, Phys, Dev);
+template __global__ void k_spin_phase<true>(const int*, int, int, int, int, double, Phys, Dev);
 
 }  // namespace sld
