@@ -12,15 +12,15 @@ constexpr double kPi = 3.141592653589793238462e0;  // Pi_num (spilady.h:61)
 
 // potential tables (global.h:66): 10^6 points per table
 constexpr int kNInput = 1000000;
-constexpr int kRStride = 8;     // sf dsf pr dpr J dJ pad pad
 constexpr int kRhoStride = 16;  // F dF A B C D dA dB dC dD pad...
 
-enum RCol { R_SF = 0, R_DSF, R_PR, R_DPR, R_J, R_DJ };
-// Device r table, one 128-byte row per lookup index n holding the pair
-// (t[n-1], t[n]) that the interpolation at n reads, for each column: a pair
-// term's lookup touches one cache line instead of two 64-byte rows.
+// The r table of the force pass: one 128-byte row per lookup index n holding
+// the pair (t[n-1], t[n]) that the interpolation at n reads, for each column, so
+// that a pair term's lookup touches one line. The neighbour build reads J and
+// the density function only, each from a table of its own: 16 MB instead of 128
+// (0.95 ms instead of 0.98 at 2 M atoms).
 constexpr int kPRowStride = 16;
-enum PCol { P_DSF = 0, P_DPR = 2, P_PR = 4, P_J = 6, P_DJ = 8, P_SF = 10 };
+enum PCol { P_DSF = 0, P_DPR = 2, P_PR = 4, P_DJ = 6, P_J = 8 };
 enum RhoCol { H_F = 0, H_DF, H_A, H_B, H_C, H_D, H_DA, H_DB, H_DC, H_DD };
 
 // Fixed capacities; exceeding one sets an error flag that the host turns

@@ -48,6 +48,12 @@ __device__ __forceinline__ double sqrt_any(double x) {
     if (__builtin_expect(!(x >= 1e-200 && x <= 1e200), 0)) r = sqrt(x);
     return r;
 }
+// sqrt(x) and 1/sqrt(x), likewise
+__device__ __forceinline__ double sqrt_rsqrt(double x, double& inv) {
+    inv = rsqrt_normal(x);
+    const double g = x * inv;
+    return fma(fma(-g, g, x), 0.5 * inv, g);
+}
 // |s|, the value every spin's .w payload holds. It is the only definition of
 // that value: the field sums read a neighbour's .w where the reference takes
 // vec_length(s_j) (calculate_spin_CPU.cpp:265), so every writer of .w must
@@ -152,10 +158,12 @@ __device__ __forceinline__ int neigh_cell(const Box& b, int c, int slot) {
 // Tables: linear interpolation between entries n-1 and n with
 // n = int(x * N / max) (potential_CPU.cpp:172-179). Entry k holds the value
 // at x = max * (k+1) / N.
-//   r tables interleaved per entry: [sf dsf pr dpr J dJ - -]
+//   r tables: pairs (n - 1, n) of [dsf dpr pr dJ J]; J; sf
 //   rho tables interleaved per entry: [F dF A B C D dA dB dC dD - ...]
 struct Tables {
-    const double* prow;    // [NINPUT][16]: interpolation pairs of the r columns
+    const double* prow;    // [NINPUT][16]
+    const double* jtab;    // [NINPUT]
+    const double* sftab;   // [NINPUT]
     const double* rhotab;  // [NINPUT][16]
     double in_over_rmax, in_over_rhomax;
 };
@@ -186,6 +194,15 @@ __device__ __forceinline__ void interp_index(double x, double in_over_max, int& 
 
 __device__ __forceinline__ double lerp_tab(const double* tab, int stride, int k, int n, double ratio) {
     return tab[(size_t)(n - 1) * stride + k] * ratio + tab[(size_t)n * stride + k] * (1.0 - ratio);
+}
+
+// entries n - 1 and n of a table, a 16-byte load at any multiple of 8
+struct __attribute__((packed, aligned(8))) Pair {
+    double x, y;
+};
+__device__ __forceinline__ double lerp_at(const double* tab, int n, double ratio) {
+    const Pair p = *reinterpret_cast<const Pair*>(tab + n - 1);
+    return p.x * ratio + p.y * (1.0 - ratio);
 }
 
 // ---------------------------------------------------------------------------
@@ -296,6 +313,42 @@ __device__ __forceinline__ double ee_to_te(double ee) {
 
 // ---------------------------------------------------------------------------
 // reductions in a fixed order (deterministic)
+
+// value of the lane whose index differs in bit 0 (XOR = 1) or bit 1 (XOR = 2)
+template <int XOR>
+__device__ __forceinline__ double quad_swap(double v) {
+    constexpr int kPerm = XOR == 1 ? 0xb1 : 0x4e;  // quad_perm [1,0,3,2], [2,3,0,1]
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, kPerm, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), kPerm, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double quad_sum(double v) {
+    v += quad_swap<1>(v);
+    return v + quad_swap<2>(v);
+}
+
+// the value of lane U of the quad, in all four
+template <int U>
+__device__ __forceinline__ int quad_from(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, U * 0x55, 0xf, 0xf, true);
+}
+template <int U>
+__device__ __forceinline__ double quad_from(double v) {
+    const long long b = __double_as_longlong(v);
+    return __longlong_as_double(((long long)quad_from<U>((int)(b >> 32)) << 32) | (unsigned)quad_from<U>((int)b));
+}
+// v[u] of lane j becomes v[j] of lane u
+__device__ __forceinline__ void quad_transpose(double (&v)[4], int j) {
+    const bool b0 = j & 1, b1 = j & 2;
+    const double s0 = quad_swap<1>(v[0]), s1 = quad_swap<1>(v[1]), s2 = quad_swap<1>(v[2]), s3 = quad_swap<1>(v[3]);
+    const double n0 = b0 ? s1 : v[0], n1 = b0 ? v[1] : s0, n2 = b0 ? s3 : v[2], n3 = b0 ? v[3] : s2;
+    const double t0 = quad_swap<2>(n0), t1 = quad_swap<2>(n1), t2 = quad_swap<2>(n2), t3 = quad_swap<2>(n3);
+    v[0] = b1 ? t2 : n0;
+    v[1] = b1 ? t3 : n1;
+    v[2] = b1 ? n2 : t0;
+    v[3] = b1 ? n3 : t1;
+}
 
 // sum over the 64 lanes of a wave, in every lane; all lanes must be active.
 // Six data-parallel-primitive steps (rows of 16 by shifts of 1, 2, 4, 8, then

@@ -84,7 +84,7 @@ struct sld_ctx {
     double *d_te2 = nullptr, *d_ee2 = nullptr;
     double2* d_dte_src = nullptr;  // what a sub-step adds to each cell
     // buffers
-    double *d_prow = nullptr, *d_rhotab = nullptr;
+    double *d_prow = nullptr, *d_jtab = nullptr, *d_sftab = nullptr, *d_rhotab = nullptr;
     int *d_cl2 = nullptr, *d_cn2 = nullptr;  // second cell-list buffer
     double* d_part = nullptr;                // block partials
     double* d_scal = nullptr;                // reduced scalars
@@ -372,8 +372,8 @@ int do_links(sld_ctx* c) {
 int do_force(sld_ctx* c) {
     TRY(ensure_nb(c));
     LAUNCH(c, k_fp, xcd_grid(nblk(c->D.N, 256)), 256, c->tab, c->D);
-    LAUNCH(c, k_force, xcd_grid(nblk(c->D.N, c->shapes.force_block)), c->shapes.force_block, c->tab, c->phys,
-           c->D);
+    const int fb = c->shapes.force_block;
+    LAUNCH(c, k_force, xcd_grid(nblk(c->D.N, fb / 4)), fb, c->tab, c->phys, c->D);
     if (c->phys.localvol) {
         // calculate_force_energy_CPU.cpp:270-293: the volumes normalised per
         // replica, then the stress over them
@@ -1289,8 +1289,12 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
     // tables (shared)
     std::shared_ptr<const HostTables> ht = shared_tables(P0.rcut_max, P0.magmom != 0);
     TRY(upload_vec(c, &c->d_prow, ht->prow));
+    TRY(upload_vec(c, &c->d_jtab, ht->jtab));
+    TRY(upload_vec(c, &c->d_sftab, ht->sftab));
     TRY(upload_vec(c, &c->d_rhotab, ht->rhotab));
     c->tab.prow = c->d_prow;
+    c->tab.jtab = c->d_jtab;
+    c->tab.sftab = c->d_sftab;
     c->tab.rhotab = c->d_rhotab;
     c->tab.in_over_rmax = ht->in_over_rmax;
     c->tab.in_over_rhomax = ht->in_over_rhomax;
@@ -1340,7 +1344,7 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
         LAUNCH(c, k_qn_init, nblk(N, 256), 256, ph, D);
     }
     TRY(dalloc(c, &D.pass_base, 1));
-    TRY(dalloc(c, &D.sjs, N)); TRY(dalloc(c, &D.fp, N)); TRY(dalloc(c, &D.stress, (size_t)6 * N));
+    TRY(dalloc(c, &D.sjs, N)); TRY(dalloc(c, &D.stress, (size_t)6 * N));
     TRY(dalloc(c, &D.lvol, P0.localvol ? N : 1));
     TRY(dalloc(c, &D.m, P0.magmom ? N : 1));
     TRY(dalloc(c, &D.cell, N)); TRY(dalloc(c, &D.cell_prev, N)); TRY(dalloc(c, &D.cslot, N));

@@ -42,7 +42,7 @@ struct Dev {
     // null when off
     double *qring, *qval;
     const double* qH;
-    double *rho, *pe, *ke, *me, *me0, *vir, *sjs, *fp;
+    double *rho, *pe, *ke, *me, *me0, *vir, *sjs;
     double4* lan;              // Landau A, B, C, D at each atom's density [N] (kept current with rho)
     double* stress;            // [6][N]: 11 22 33 12 23 31
     double* lvol;              // localvol: each atom's local volume

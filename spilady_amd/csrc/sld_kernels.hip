@@ -315,16 +315,14 @@ __global__ __launch_bounds__(256) void k_nbuild(Tables T, Phys P, Dev D, int wri
             int n0;
             double ratio;
             interp_index(r, T.in_over_rmax, n0, ratio);
-            const double* row = T.prow + (size_t)n0 * kPRowStride;
-            const double2 sf = *reinterpret_cast<const double2*>(row + P_SF);
+            const double sf = lerp_at(T.sftab, n0, ratio);
             const int mag = e.y >> 16;
             D.nb[a * kMaxNb + ((e.y >> 8) & 255)] = e.x;
             if (mag) {
-                const double2 jv = *reinterpret_cast<const double2*>(row + P_J);
                 D.nbm[a * kMaxMag + mag - 1] = e.x;
-                D.nbJ[a * kMaxMag + mag - 1] = jv.x * ratio + jv.y * (1.0 - ratio);
+                D.nbJ[a * kMaxMag + mag - 1] = lerp_at(T.jtab, n0, ratio);
             }
-            rsqs[p] = r < P.rcut_pot ? sf.x * ratio + sf.y * (1.0 - ratio) : 0.0;
+            rsqs[p] = r < P.rcut_pot ? sf : 0.0;
         }
         wave_fence();
         // densities: eight lanes an atom
@@ -372,95 +370,123 @@ __global__ __launch_bounds__(256) void k_fp(Tables T, Dev D) {
     double dC = lerp_tab(T.rhotab, kRhoStride, H_DC, n0, ratio);
     double dD = lerp_tab(T.rhotab, kRhoStride, H_DD, n0, ratio);
     double s4 = s2 * s2;
-    D.fp[i] = dF + (dA * s2 + dB * s4 + dC * s4 * s2 + dD * s4 * s4);
+    D.r[i].w = dF + (dA * s2 + dB * s4 + dC * s4 * s2 + dD * s4 * s4);
 }
 
-constexpr int kForceBatch = 8;  // neighbour pairs whose loads the force pass issues together
-
+// Four lanes an atom: lane j takes list entries j, j + 4, ..., and the sums of
+// the four are added at the end. The lanes of a quad fetch each other's data
+// together: two lanes load the halves of a pair's r with F'(rho) in r.w, two
+// those of its s, and each a column of its table row, so that a load
+// instruction touches 32 or 16 lines and not 64; the quad then swaps the pieces
+// by register moves (the columns after the interpolation).
+//
+// What bounds it are the rows: 44 M pairs of 2 M atoms read lines of a 64 MB
+// range, 3.1 GB from beyond the L2s. 893 us, where a lane an atom, which loaded
+// all of a pair by itself and had eight pairs in flight to hide it, took 1,340;
+// 64 x 16,000 atoms 655 (910), 250,000 atoms 110 (160), 2,000 14 (40). Smaller
+// rows lose again what they save as soon as a pair needs a second line (J in a
+// table of its own: 970 with rows of 64 bytes, 1,000 with entries of 32 that are
+// not stored twice), loads straight to LDS save the moves but not the lines
+// (970), and 128 registers spill (1,840).
 __global__ __launch_bounds__(256) void k_force(Tables T, Phys P, Dev D) {
-    const int lb = xcd_block((D.N + blockDim.x - 1) / blockDim.x);
+    const int lb = xcd_block((4 * D.N + blockDim.x - 1) / blockDim.x);
     if (lb < 0) return;
-    int i = lb * blockDim.x + threadIdx.x;
+    const int i = (lb * blockDim.x + threadIdx.x) >> 2, j = threadIdx.x & 3;
     if (i >= D.N) return;
     const int rr = D.arep[i];
     if (rr < 0) return;
     const Rep& R = D.rep[rr];
     const Box b = R.box;
-    const double3 ri = d3(D.r[i]);
+    const double4 ri4 = D.r[i];
+    const double3 ri = d3(ri4);
     const double4 si4 = D.s[i];
     const double3 si = d3(si4);
-    const double si_sq = sq3(si);
-    const double fpi = D.fp[i];
+    const double fpi = ri4.w;
     double3 f = make_double3(0.0, 0.0, 0.0);
-    double pe = 0.0, me = 0.0, me0 = 0.0, vir = 0.0;
+    double pe = 0.0, me = 0.0, me0 = 0.0;
     double st0 = 0.0, st1 = 0.0, st2 = 0.0, st3 = 0.0, st4 = 0.0, st5 = 0.0;
     double m1 = 0.0, m2 = 0.0;  // localvol: sums of 1/r and 1/r^2 within rcut_vol
     const int nn = D.nbn[i];
     const int* nb = D.nb + (size_t)i * kMaxNb;
-    // kForceBatch pairs at a time: their neighbour ids, then their
-    // positions, F'(rho) and spins, then their table rows, all in flight
-    // together; the pair terms are then added in list order, as a
-    // pair-at-a-time loop adds them
-    for (int k0 = 0; k0 < nn; k0 += kForceBatch) {
-        int jj[kForceBatch];
-#pragma unroll
-        for (int u = 0; u < kForceBatch; ++u)
-            jj[u] = k0 + u < nn ? nb[k0 + u] : i;  // past the list: a valid slot, never added
-        double4 rj[kForceBatch], sj4[kForceBatch];
-        double fpj[kForceBatch];
-#pragma unroll
-        for (int u = 0; u < kForceBatch; ++u) {
-            rj[u] = D.r[jj[u]];
-            fpj[u] = D.fp[jj[u]];
-            sj4[u] = D.s[jj[u]];
+    // this lane's half of every pair's r or s, and its column of every row
+    const double2* rec = reinterpret_cast<const double2*>(j < 2 ? D.r : D.s) + (j & 1);
+    const double2* col = reinterpret_cast<const double2*>(T.prow) + j;
+    static_assert(P_DSF == 0 && P_DPR == 2 && P_PR == 4 && P_DJ == 6, "the first columns, in the lanes' order");
+    constexpr int kRow = kPRowStride / 2;
+    double2 v[4];
+    auto gather = [&](int id) {
+        v[0] = rec[2 * (size_t)quad_from<0>(id)];
+        v[1] = rec[2 * (size_t)quad_from<1>(id)];
+        v[2] = rec[2 * (size_t)quad_from<2>(id)];
+        v[3] = rec[2 * (size_t)quad_from<3>(id)];
+    };
+    // past the list: a valid atom, never added
+    auto entry = [&](int k) { return k < nn ? nb[k] : i; };
+    gather(entry(j));
+    int next = entry(j + 4);
+    for (int k0 = 0; k0 < nn; k0 += 4) {
+        double x[4] = {v[0].x, v[1].x, v[2].x, v[3].x}, y[4] = {v[0].y, v[1].y, v[2].y, v[3].y};
+        quad_transpose(x, j);
+        quad_transpose(y, j);
+        const double3 sj = make_double3(x[2], y[2], x[3]);
+        const double fpj = y[1], sj_len = y[3];
+        double rsq, inv, ratio;
+        int n0;
+        const double3 rij = min_image_sq(b, sub3(ri, make_double3(x[0], y[0], x[1])), rsq);
+        const double r = sqrt_rsqrt(rsq, inv);
+        interp_index(r, T.in_over_rmax, n0, ratio);
+        double2 q[4];
+        q[0] = col[(size_t)quad_from<0>(n0) * kRow];
+        q[1] = col[(size_t)quad_from<1>(n0) * kRow];
+        q[2] = col[(size_t)quad_from<2>(n0) * kRow];
+        q[3] = col[(size_t)quad_from<3>(n0) * kRow];
+        const bool in = k0 + j < nn, mag = in && r < P.rcut_mag;
+        double2 qJ = make_double2(0.0, 0.0);
+        if (mag) qJ = *reinterpret_cast<const double2*>(T.prow + (size_t)n0 * kPRowStride + P_J);
+        // the next pairs' loads go out before this one's rows are waited for
+        gather(next);
+        next = entry(k0 + 8 + j);
+        double c[4];
+        auto lerp = [&](double2 t, double rt) { return t.x * rt + t.y * (1.0 - rt); };
+        c[0] = lerp(q[0], quad_from<0>(ratio));
+        c[1] = lerp(q[1], quad_from<1>(ratio));
+        c[2] = lerp(q[2], quad_from<2>(ratio));
+        c[3] = lerp(q[3], quad_from<3>(ratio));
+        quad_transpose(c, j);
+        if (!in) continue;
+        double dudr = 0.0;
+        if (r < P.rcut_pot) {
+            dudr = (fpi + fpj) * c[0] + c[1];
+            pe += 0.5 * c[2];
         }
-        double3 rij[kForceBatch];
-        double rsq[kForceBatch], r[kForceBatch], ratio[kForceBatch];
-        const double* q[kForceBatch];
-#pragma unroll
-        for (int u = 0; u < kForceBatch; ++u) {
-            rij[u] = min_image_sq(b, sub3(ri, d3(rj[u])), rsq[u]);
-            r[u] = sqrt(rsq[u]);
-            int n0;
-            interp_index(r[u], T.in_over_rmax, n0, ratio[u]);
-            q[u] = T.prow + (size_t)n0 * kPRowStride;
+        if (mag) {
+            const double sdot = dot3(si, sj), stimes = si4.w * sj_len;
+            const double Jh = lerp(qJ, ratio) / 2.0;
+            dudr += -c[3] * (sdot - stimes);
+            me0 += Jh * stimes;
+            me += -Jh * sdot;
         }
-#pragma unroll
-        for (int u = 0; u < kForceBatch; ++u) {
-            if (k0 + u >= nn) break;
-            const double* qq = q[u];
-            const double rt = ratio[u], wr = 1.0 - rt;
-            double dudr = 0.0;
-            if (r[u] < P.rcut_pot) {
-                double dsf = qq[P_DSF] * rt + qq[P_DSF + 1] * wr;
-                double dpr = qq[P_DPR] * rt + qq[P_DPR + 1] * wr;
-                double pr = qq[P_PR] * rt + qq[P_PR + 1] * wr;
-                dudr = (fpi + fpj[u]) * dsf + dpr;
-                pe += 0.5 * pr;
-            }
-            if (r[u] < P.rcut_mag) {
-                double3 sj = d3(sj4[u]);
-                double sdot = dot3(si, sj);
-                double stimes = sqrt(si_sq * sq3(sj));
-                double J = qq[P_J] * rt + qq[P_J + 1] * wr;
-                double dJ = qq[P_DJ] * rt + qq[P_DJ + 1] * wr;
-                dudr += -dJ * (sdot - stimes);
-                double Jh = J / 2.0;
-                me0 += Jh * stimes;
-                me += -Jh * sdot;
-            }
-            double force = -dudr / r[u];
-            double3 fij = mul3(force, rij[u]);
-            f = add3(f, fij);
-            st0 += fij.x * rij[u].x; st1 += fij.y * rij[u].y; st2 += fij.z * rij[u].z;
-            st3 += fij.x * rij[u].y; st4 += fij.y * rij[u].z; st5 += fij.z * rij[u].x;
-            vir += -force * rsq[u];
-            if (P.localvol && r[u] < P.rcut_vol) {  // calculate_force_energy_CPU.cpp:80-90
-                m1 += 1.0 / r[u];
-                m2 += 1.0 / rsq[u];
-            }
+        const double force = -dudr * inv;
+        const double3 fij = mul3(force, rij);
+        f = add3(f, fij);
+        st0 += fij.x * rij.x; st1 += fij.y * rij.y; st2 += fij.z * rij.z;
+        st3 += fij.x * rij.y; st4 += fij.y * rij.z; st5 += fij.z * rij.x;
+        if (P.localvol && r < P.rcut_vol) {  // calculate_force_energy_CPU.cpp:80-90
+            m1 += inv;
+            m2 += inv * inv;
         }
     }
+    f = make_double3(quad_sum(f.x), quad_sum(f.y), quad_sum(f.z));
+    pe = quad_sum(pe);
+    me = quad_sum(me);
+    me0 = quad_sum(me0);
+    st0 = quad_sum(st0); st1 = quad_sum(st1); st2 = quad_sum(st2);
+    st3 = quad_sum(st3); st4 = quad_sum(st4); st5 = quad_sum(st5);
+    if (P.localvol) {
+        m1 = quad_sum(m1);
+        m2 = quad_sum(m2);
+    }
+    const double si_sq = sq3(si);
     // one-body terms (calculate_force_energy_CPU.cpp:196-215)
     int n0;
     double ratio;
@@ -472,31 +498,33 @@ __global__ __launch_bounds__(256) void k_force(Tables T, Phys P, Dev D) {
     pe += F;
     if (P.extfield) me -= dot3(si, d3(D.hext[i]));  // calculate_force_energy_CPU.cpp:199-201
     me += A * si_sq + B * s4 + C * s4 * si_sq + Dd * s4 * s4;
-    D.f[i] = make_double4(f.x, f.y, f.z, 0.0);
-    D.pe[i] = pe;
-    D.me[i] = me;
-    D.me0[i] = me0;
-    // the reference books -force*r^2 once per pair on the half-shell owner;
-    // here each atom keeps half of each of its pairs (same total virial)
-    D.vir[i] = 0.5 * vir;
-    // per-atom stress with the kinetic part (calculate_force_energy_CPU.cpp:283-293);
-    // with localvol the local volume (:270-276) is normalised over the
-    // replica first, so the numerators are stored and k_lvol_apply divides
     const double m = P.atmass;
     const double4 p = D.p[i];
     const size_t N = D.N;
-    double num[6] = {p.x * p.x / m + st0 / 2.0,   p.y * p.y / m + st1 / 2.0,   p.z * p.z / m + st2 / 2.0,
-                     (p.x * p.y) / m + st3 / 2.0, (p.y * p.z) / m + st4 / 2.0, (p.z * p.x) / m + st5 / 2.0};
+    if (j == 0) {
+        D.f[i] = make_double4(f.x, f.y, f.z, 0.0);
+        D.pe[i] = pe;
+        D.me[i] = me;
+        D.me0[i] = me0;
+    }
+    // the reference books -force*r^2 once per pair on the half-shell owner;
+    // here each atom keeps half of each of its pairs (same total virial)
+    if (j == 1) D.vir[i] = -0.5 * (st0 + st1 + st2);
+    // per-atom stress with the kinetic part (calculate_force_energy_CPU.cpp:283-293);
+    // with localvol the local volume (:270-276) is normalised over the
+    // replica first, so the numerators are stored and k_lvol_apply divides
+    const double num[6] = {p.x * p.x / m + st0 / 2.0,   p.y * p.y / m + st1 / 2.0,   p.z * p.z / m + st2 / 2.0,
+                           (p.x * p.y) / m + st3 / 2.0, (p.y * p.z) / m + st4 / 2.0, (p.z * p.x) / m + st5 / 2.0};
+    double lv = 1.0;
     if (P.localvol) {
         const double local_radius = 0.5 * m1 / m2;
-        D.lvol[i] = 4.0 * kPi / 3.0 * pow(local_radius, 3.0);
-#pragma unroll
-        for (int k = 0; k < 6; ++k) D.stress[k * N + i] = num[k];
+        if (j == 0) D.lvol[i] = 4.0 * kPi / 3.0 * pow(local_radius, 3.0);
     } else {
-        const double lv = R.box_volume / R.natom;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) D.stress[k * N + i] = num[k] / lv;
+        lv = R.box_volume / R.natom;
     }
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+        if (j == (k & 3)) D.stress[k * N + i] = num[k] / lv;
 }
 
 // localvol: each replica's sum of the local volumes, one partial per 256

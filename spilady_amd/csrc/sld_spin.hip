@@ -80,20 +80,6 @@ __device__ __forceinline__ double3 apply_rot(const Rot& r, double3 s) {
                         fma(r.C, u.z, fma(r.S, t.z, s.z)));
 }
 
-// value of the lane whose index differs in bit 0 (XOR = 1) or bit 1 (XOR = 2)
-template <int XOR>
-__device__ __forceinline__ double quad_swap(double v) {
-    constexpr int kPerm = XOR == 1 ? 0xb1 : 0x4e;  // quad_perm [1,0,3,2], [2,3,0,1]
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, kPerm, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), kPerm, 0xf, 0xf, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ double quad_sum(double v) {
-    v += quad_swap<1>(v);
-    return v + quad_swap<2>(v);
-}
-
 // value of the lane N places before in the row of 16, or 0
 template <int N>
 __device__ __forceinline__ int row_shr(int v) {

@@ -174,20 +174,22 @@ void build_tables(double rcut_max, bool magmom, HostTables& t) {
     const double finput = (double)kNInput;
     t.in_over_rmax = finput / t.rmax;
     t.in_over_rhomax = finput / t.rhomax;
-    t.rtab.assign((size_t)kNInput * kRStride, 0.0);
+    t.prow.assign((size_t)kNInput * kPRowStride, 0.0);
+    t.jtab.assign(kNInput, 0.0);
+    t.sftab.assign(kNInput, 0.0);
     t.rhotab.assign((size_t)kNInput * kRhoStride, 0.0);
     (void)bridge();
     auto work = [&](int n0, int n1) {
         for (int n = n0; n < n1; ++n) {
             double r = t.rmax / (double)kNInput * (double)(n + 1);
             double rho = t.rhomax / (double)kNInput * (double)(n + 1);
-            double* R = &t.rtab[(size_t)n * kRStride];
-            R[R_SF] = smallf_gen(r);
-            R[R_DSF] = deriv6(smallf_gen, r);
-            R[R_PR] = pair_gen(r);
-            R[R_DPR] = deriv6(pair_gen, r);
-            R[R_J] = jij_gen(r);
-            R[R_DJ] = deriv6(jij_gen, r);
+            double dsf, dpr, pr, dJ;
+            t.sftab[n] = smallf_gen(r);
+            dsf = deriv6(smallf_gen, r);
+            pr = pair_gen(r);
+            dpr = deriv6(pair_gen, r);
+            t.jtab[n] = jij_gen(r);
+            dJ = deriv6(jij_gen, r);
             double* H = &t.rhotab[(size_t)n * kRhoStride];
             H[H_F] = bigf_gen(rho);
             H[H_DF] = deriv6(bigf_gen, rho);
@@ -200,8 +202,8 @@ void build_tables(double rcut_max, bool magmom, HostTables& t) {
             H[H_DC] = deriv6(landauC, rho);
             H[H_DD] = deriv6(landauD, rho);
             if (magmom) {
-                R[R_J] *= std::pow(kElG, 2);
-                R[R_DJ] *= std::pow(kElG, 2);
+                t.jtab[n] *= std::pow(kElG, 2);
+                dJ *= std::pow(kElG, 2);
                 H[H_A] *= std::pow(kElG, 2);
                 H[H_B] *= std::pow(kElG, 4);
                 H[H_C] *= std::pow(kElG, 6);
@@ -210,6 +212,12 @@ void build_tables(double rcut_max, bool magmom, HostTables& t) {
                 H[H_DB] *= std::pow(kElG, 4);
                 H[H_DC] *= std::pow(kElG, 6);
                 H[H_DD] *= std::pow(kElG, 8);
+            }
+            // entry n is the second of row n and the first of row n + 1
+            const double v[5] = {dsf, dpr, pr, dJ, t.jtab[n]};
+            for (int k = 0; k < 5; ++k) {
+                t.prow[(size_t)n * kPRowStride + 2 * k + 1] = v[k];
+                if (n + 1 < kNInput) t.prow[(size_t)(n + 1) * kPRowStride + 2 * k] = v[k];
             }
         }
     };
@@ -223,16 +231,6 @@ void build_tables(double rcut_max, bool magmom, HostTables& t) {
         if (a < b) th.emplace_back(work, a, b);
     }
     for (auto& x : th) x.join();
-    // interpolation rows of the device r table
-    t.prow.assign((size_t)kNInput * kPRowStride, 0.0);
-    const int cols[6][2] = {{P_DSF, R_DSF}, {P_DPR, R_DPR}, {P_PR, R_PR}, {P_J, R_J}, {P_DJ, R_DJ}, {P_SF, R_SF}};
-    for (int n = 1; n < kNInput; ++n) {
-        double* q = &t.prow[(size_t)n * kPRowStride];
-        for (const auto& cc : cols) {
-            q[cc[0]] = t.rtab[(size_t)(n - 1) * kRStride + cc[1]];
-            q[cc[0] + 1] = t.rtab[(size_t)n * kRStride + cc[1]];
-        }
-    }
 }
 
 std::shared_ptr<const HostTables> shared_tables(double rcut_max, bool magmom) {

@@ -8,9 +8,9 @@ namespace sld {
 
 struct HostTables {
     double rmax = 0, rhomax = 0, in_over_rmax = 0, in_over_rhomax = 0;
-    std::vector<double> rtab;    // [kNInput][kRStride]
-    std::vector<double> prow;    // [kNInput][kPRowStride]: (rtab[n-1], rtab[n]) per column
-    std::vector<double> rhotab;  // [kNInput][kRhoStride]
+    std::vector<double> prow;         // [kNInput][kPRowStride]: entries n-1 and n per column
+    std::vector<double> jtab, sftab;  // [kNInput]
+    std::vector<double> rhotab;       // [kNInput][kRhoStride]
 };
 
 // magmom: the J and Landau columns scaled by powers of the electron g factor
