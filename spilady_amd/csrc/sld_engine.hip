@@ -126,7 +126,7 @@ struct sld_ctx {
         sld::ModelTab tab{};
         std::shared_ptr<const sld::ModelBridge> bridge;
         double* d_bridge = nullptr;
-        double *d_r = nullptr, *d_rd = nullptr, *d_h = nullptr;
+        double *d_r = nullptr, *d_h = nullptr;
         double *d_rho = nullptr, *d_fp = nullptr, *d_Q = nullptr;
         double *d_F = nullptr, *d_H = nullptr, *d_gE = nullptr, *d_gF = nullptr, *d_gH = nullptr;
         double *d_E = nullptr, *d_grad = nullptr, *d_part = nullptr;
@@ -322,7 +322,7 @@ void make_levels(const HostCells& h, const std::vector<int>& gsize, const std::v
 // device building blocks
 
 int reduce(sld_ctx* c, int nblocks, int nk, double* out, size_t part_offset = 0) {
-    LAUNCH(c, k_reduce, 1, 256, (const double*)(c->d_part + part_offset), nblocks, nk, out);
+    LAUNCH(c, k_reduce, nk, 256, (const double*)(c->d_part + part_offset), nblocks, out);
     return SLD_OK;
 }
 
@@ -2006,7 +2006,6 @@ int sld_model_set_params(sld_ctx* c, const double* theta) {
         m.bridge = model_bridge(c->prm.rcut_max);
         TRY(upload_vec(c, &m.d_bridge, m.bridge->q));
         TRY(dalloc(c, &m.d_r, (size_t)kNInput * kMRStride));
-        TRY(dalloc(c, &m.d_rd, (size_t)kNInput * kMRDStride));
         TRY(dalloc(c, &m.d_h, (size_t)kNInput * kMHStride));
         std::vector<int> coff(c->R);
         int tot = 0;
@@ -2021,15 +2020,19 @@ int sld_model_set_params(sld_ctx* c, const double* theta) {
         TRY(dalloc(c, &m.d_gF, (size_t)3 * tot)); TRY(dalloc(c, &m.d_gH, (size_t)3 * tot));
         TRY(dalloc(c, &m.d_gE, c->R)); TRY(dalloc(c, &m.d_E, (size_t)kScal * c->R));
         TRY(dalloc(c, &m.d_grad, kNParam));
-        TRY(dalloc(c, &m.d_part, (size_t)nblk(N, 256) * kNParam));
+        TRY(dalloc(c, &m.d_part, std::max((size_t)nblk(N, 256), (size_t)kNParam * kAdjBlocks)));
     }
     const ModelCoef mc = model_coef(theta, c->prm.rcut_max, *m.bridge);
     LAUNCH(c, k_model_tab_r, nblk(kNInput - 1, 255), 256, mc, (const double*)m.d_bridge, m.d_r);
-    LAUNCH(c, k_model_tab_rd, nblk(kNInput, 64), 64, mc, (const double*)m.d_bridge, m.d_rd);
     LAUNCH(c, k_model_tab_h, nblk(kNInput, 256), 256, mc, m.d_h);
     HIPCHK(c, hipStreamSynchronize(c->stream));
     m.tab.r = m.d_r;
-    m.tab.rd = m.d_rd;
+    m.tab.JA = mc.JA;
+    m.tab.Jrc = mc.Jrc;
+    m.tab.rmax = mc.rmax;
+    m.tab.step = mc.rmax / (double)kNInput;
+    m.tab.bridge = m.d_bridge;
+    m.tab.row0 = mc.row0;
     m.tab.h = m.d_h;
     m.tab.in_over_rmax = (double)kNInput / mc.rmax;
     m.tab.in_over_rhomax = (double)kNInput / mc.rhomax;
@@ -2103,10 +2106,12 @@ int sld_model_vjp(sld_ctx* c, const double* g_energy, const double* g_force, con
     else HIPCHK(c, hipMemsetAsync(m.d_gH, 0, b3, c->stream));
     const int nb = nblk(c->D.N, 256);
     LAUNCH(c, k_model_q, xcd_grid(nb), 256, m.tab, c->phys, c->D, (const int*)m.d_coff, (const double*)m.d_gF, m.d_Q);
-    LAUNCH(c, k_model_adjoint, xcd_grid(nb), 256, m.tab, c->phys, c->D, (const double*)m.d_rho, (const double*)m.d_fp,
+    // the kNParam partial sums of at most kAdjBlocks blocks, of 16 atoms at a time
+    const int per = nblk(nblk(c->D.N, 16), kAdjBlocks) * 16, na = nblk(c->D.N, per);
+    LAUNCH(c, k_model_adjoint, xcd_grid(na), 256, m.tab, c->phys, c->D, per, (const double*)m.d_rho, (const double*)m.d_fp,
            (const double*)m.d_Q, (const int*)m.d_coff, (const double*)m.d_gE, (const double*)m.d_gF,
            (const double*)m.d_gH, m.d_part);
-    LAUNCH(c, k_reduce, 1, 256, (const double*)m.d_part, nb, kNParam, m.d_grad);
+    LAUNCH(c, k_reduce, kNParam, 256, (const double*)m.d_part, na, m.d_grad);
     TRY(copy_any(c, grad, m.d_grad, kNParam * sizeof(double)));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return collect_timing(c);

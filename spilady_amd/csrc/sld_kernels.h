@@ -150,7 +150,7 @@ __global__ void k_dte_finish_ab(Mesh M, const double* E, const double* start, co
 __global__ void k_obs_atoms(Tables T, Phys P, Dev D, double* partials, int scan_spin);
 __global__ void k_obs_cells(Dev D, double* partials);
 __global__ void k_renorm(Dev D, const double* err, double* partials);
-__global__ void k_reduce(const double* partials, int nblk, int nk, double* out);
+__global__ void k_reduce(const double* partials, int nblk, double* out);
 __global__ void k_reduce_seg(const double* partials, const int* seg, int nk, double* out, int out_off);
 __global__ void k_check_nonfinite(Dev D);
 __global__ void k_ee_of_te(Dev D, int c0, int n);
@@ -174,21 +174,24 @@ __global__ void k_unpack(XferArgs A, int N, const double* buf);
 __global__ void k_spin_len(Dev D, int a0, int n);
 
 // ---- parametric potential model (sld_model.hip) ----
+constexpr int kAdjBlocks = 2048;  // most blocks of the adjoint: four a compute unit
 struct ModelTab {
     const double* r;    // [N][kMRStride]
-    const double* rd;   // [N][kMRDStride]
     const double* h;    // [N][kMHStride]
     double in_over_rmax, in_over_rhomax;
     double L[4];        // Landau A B C D
+    double JA, Jrc;
+    double rmax, step;     // entry e of the r tables is at step * (e + 1)
+    const double* bridge;  // ModelBridge
+    int row0;
 };
 __global__ void k_model_tab_r(ModelCoef m, const double* bridge, double* out);
-__global__ void k_model_tab_rd(ModelCoef m, const double* bridge, double* out);
 __global__ void k_model_tab_h(ModelCoef m, double* out);
 __global__ void k_model_rho(ModelTab M, Phys P, Dev D, double* rho_out, double* fp_out);
 __global__ void k_model_forward(ModelTab M, Phys P, Dev D, const double* rho, const double* fp, const int* coff,
                                 double* F, double* H, double* partials);
 __global__ void k_model_q(ModelTab M, Phys P, Dev D, const int* coff, const double* gF, double* Q);
-__global__ void k_model_adjoint(ModelTab M, Phys P, Dev D, const double* rho, const double* fp, const double* Q,
+__global__ void k_model_adjoint(ModelTab M, Phys P, Dev D, int per_block, const double* rho, const double* fp, const double* Q,
                                 const int* coff, const double* gE, const double* gF, const double* gH,
                                 double* partials);
 

@@ -17,22 +17,19 @@ namespace sld {
 // ---------------------------------------------------------------------------
 // reductions
 
-// out[k] = sum over blocks of partials[k*nblk + b]; one block of 256 threads.
-__global__ __launch_bounds__(256) void k_reduce(const double* partials, int nblk, int nk, double* out) {
+// out[k] = sum over blocks of partials[k*nblk + b]; one block of 256 threads for each k.
+__global__ __launch_bounds__(256) void k_reduce(const double* partials, int nblk, double* out) {
     __shared__ double sh[256];
-    const int t = threadIdx.x;
-    for (int k = 0; k < nk; ++k) {
-        double acc = 0.0;
-        for (int b = t; b < nblk; b += 256) acc += partials[(size_t)k * nblk + b];
-        sh[t] = acc;
-        __syncthreads();
-        for (int s = 128; s > 0; s >>= 1) {
-            if (t < s) sh[t] += sh[t + s];
-            __syncthreads();
-        }
-        if (t == 0) out[k] = sh[0];
+    const int t = threadIdx.x, k = blockIdx.x;
+    double acc = 0.0;
+    for (int b = t; b < nblk; b += 256) acc += partials[(size_t)k * nblk + b];
+    sh[t] = acc;
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+        if (t < s) sh[t] += sh[t + s];
         __syncthreads();
     }
+    if (t == 0) out[k] = sh[0];
 }
 
 // Per-replica sums: block r of the grid (1,024 threads) reduces partial rows

@@ -21,11 +21,8 @@ enum ParamIndex { P_A0 = 0, P_V0 = 6, P_AA = 14, P_BB = 15, P_JA = 16, P_JRC = 1
 // and 6-point derivative stencil):
 //   r value table   [N][16]: the interpolation pair (t[n-1], t[n]) of each of f f' V V' J J', then padding:
 //                            a lookup touches one 128-byte line
-//   r derivative    [N][32]: df/da_k, df'/da_k (k<6, interleaved), dV/dV_k, dV'/dV_k (k<8),
-//                            dJ/dA dJ'/dA dJ/drc dJ'/drc
 //   rho table       [N][8]:  F F' dF/daa dF'/daa dF/dbb dF'/dbb - -
 constexpr int kMRStride = 16;
-constexpr int kMRDStride = 32;
 constexpr int kMHStride = 8;
 enum MRCol { MR_F = 0, MR_DF, MR_V, MR_DV, MR_J, MR_DJ };
 enum MHCol { MH_F = 0, MH_DF, MH_AA, MH_DAA, MH_BB, MH_DBB };

@@ -19,6 +19,7 @@
 
 #include "sld_kernels.h"
 #include "sld_model.h"
+#include "sld_model_device.h"
 
 namespace sld {
 
@@ -176,90 +177,223 @@ __global__ __launch_bounds__(256) void k_model_q(ModelTab M, Phys P, Dev D, cons
     Q[i] = q;
 }
 
-// adjoint, second pass: the kNParam components of grad_theta per atom
-__global__ __launch_bounds__(256) void k_model_adjoint(ModelTab M, Phys P, Dev D, const double* rho,
-                                                       const double* fp, const double* Q, const int* coff,
-                                                       const double* gE, const double* gF, const double* gH,
-                                                       double* partials) {
-    const int lb = xcd_block((D.N + blockDim.x - 1) / blockDim.x);
+// The basis functions of the 16 pair parameters, one a lane: with d = R - r for
+// r < R, a density or pair spline is d^3, dJ/dA is d^3 / rc^3 and dJ/drc is
+// 3 A d^2 r / rc^4, all of them d^2 (alpha d + beta r).
+struct Basis {
+    double R, alpha, beta;
+    int bridge;  // place among the knots of the quintic bridge, or -1
+};
+
+__device__ __forceinline__ Basis pair_basis(const ModelTab& M, int l) {
+    Basis B;
+    const double irc = 1.0 / M.Jrc;
+    B.R = l < 6 ? kDFR[l] : l < 14 ? kDVR[l - 6] : M.Jrc;
+    B.alpha = l < 14 ? 1.0 : l == 14 ? irc * irc * irc : 0.0;
+    B.beta = l == 15 ? 3.0 * M.JA * (irc * irc) * (irc * irc) : 0.0;
+    B.bridge = l >= 6 && l < 14 ? l - 6 : -1;
+    return B;
+}
+
+// 6-point derivative at r near the knot, where the stencil sees it
+__device__ __forceinline__ double basis_knot(const Basis& B, double r) {
+    auto at = [&](double x) {
+        const double d = fmax(B.R - x, 0.0);
+        return d * d * fma(B.alpha, d, B.beta * x);
+    };
+    const double dx = 1e-3 * r;
+    double q = __builtin_amdgcn_rcp(r);
+    q = fma(fma(-r, q, 1.0), q, q);
+    q = fma(fma(-r, q, 1.0), q, q);
+    const double s = 45.0 * (at(r + dx) - at(r - dx)) - 9.0 * (at(fma(2.0, dx, r)) - at(fma(-2.0, dx, r))) +
+                     (at(fma(3.0, dx, r)) - at(fma(-3.0, dx, r)));
+    return s * (q * (1000.0 / 60.0));
+}
+
+// value and derivative of a pair spline that reaches the quintic bridge below 2,
+// where the ZBL core ends at 1.8, interpolated in its entries
+__device__ __forceinline__ double2 basis_bridge(const double* bridge, int row0, int k, double R, double step,
+                                             double in_over_rmax, double r) {
+    int n;
+    double ratio;
+    interp_index(r, in_over_rmax, n, ratio);
+    double2 out = make_double2(0.0, 0.0);
+    for (int e = n - 1; e <= n; ++e) {
+        const double x = step * (double)(e + 1);
+        double v[7];
+        for (int s = 0; s < 7; ++s) {
+            const double xs = stencil_x(x, s), d = fmax(R - xs, 0.0);
+            v[s] = xs <= 1.8   ? 0.0
+                   : xs <= 2.0 ? bridge[(size_t)(e - row0) * kModelBridgeRow + 9 * s + 1 + k]
+                               : d * d * d;
+        }
+        const double w = e == n ? 1.0 - ratio : ratio;
+        out.x += w * v[0];
+        out.y += w * stencil_deriv(v, x);
+    }
+    return out;
+}
+
+// Value and derivative at r as a table of step h interpolates them: g + q g''
+// for a smooth g, with q = (r - x0)(x1 - r) / 2 between the entries x0 and x1.
+// Away from the knots the 6-point derivative of these cubics is their
+// derivative; near one q g'' (1e-11) is below the stencil's own rounding of the
+// knot and left out.
+__device__ __forceinline__ double2 basis_at(const ModelTab& M, const Basis& B, double r, double q) {
+    double2 out = make_double2(0.0, 0.0);
+    if (r * 0.9969 < B.R) {  // else every point of the stencil is past the knot
+        const double d = fmax(B.R - r, 0.0), g = 3.0 * B.alpha;
+        out.x = fma(q, fma(2.0 * g, d, B.beta * fma(-4.0, d, 2.0 * r)), d * d * fma(B.alpha, d, B.beta * r));
+        out.y = fma(q, fma(6.0, B.beta, -2.0 * g), d * fma(-g, d, B.beta * fma(-2.0, r, d)));
+        if (r * 1.0031 >= B.R) {
+            out.x = d * d * fma(B.alpha, d, B.beta * r);
+            out.y = basis_knot(B, r);
+        }
+        if (__builtin_expect(B.bridge >= 0 && r * 0.9969 <= 2.0, 0))
+            out = basis_bridge(M.bridge, M.row0, B.bridge, B.R, M.step, M.in_over_rmax, r);
+    }
+    return out;
+}
+
+// adjoint, second pass: the kNParam components of grad_theta, in partial sums
+// of a block's atoms [lb * per_block, (lb + 1) * per_block).
+//
+// Sixteen lanes an atom. First they take a pair each: geometry, lookup and the
+// weights of the three kinds of parameters (density and pair spline, exchange)
+// go to LDS. Then lane l goes over the pairs for its own pair parameter, whose
+// basis function it evaluates: a table of them has 512 bytes a lookup, 3 GB a
+// call at 262,144 atoms and as much as the memory gives (712 us, and 70 us and
+// 256 MB to build the table at every parameter change), and the arithmetic takes
+// 267 us; of 4,096 atoms 13 (119). A pair near some lane's knot costs its wave
+// the stencil, two of five rounds. 128 registers with seven spilled for four
+// waves a SIMD: 331 us with 145 and three.
+constexpr int kAdjWaves = 4;
+
+__global__ __launch_bounds__(64 * kAdjWaves, 4) void k_model_adjoint(ModelTab M, Phys P, Dev D, int per_block,
+                                                                  const double* rho, const double* fp,
+                                                                  const double* Q, const int* coff, const double* gE,
+                                                                  const double* gF, const double* gH,
+                                                                  double* partials) {
+    __shared__ double sR[kAdjWaves][64];     // r
+    __shared__ double sW[kAdjWaves][6][64];  // weights of the derivative, then of the value
+    __shared__ double sQ[kAdjWaves][64];     // q of the interpolation
+    __shared__ double sP[kAdjWaves][2][16];
+    const int nblocks = (D.N + per_block - 1) / per_block;
+    const int lb = xcd_block(nblocks);
     if (lb < 0) return;  // whole padding block
-    const int i = lb * blockDim.x + threadIdx.x;
-    double acc[kNParam];
-#pragma unroll
-    for (int k = 0; k < kNParam; ++k) acc[k] = 0.0;
-    const int rr = i < D.N ? D.arep[i] : -1;
-    if (rr >= 0) {
-        const Rep& R = D.rep[rr];
-        const Box b = R.box;
-        const double3 ri = d3(D.r[i]);
-        const double3 si = d3(D.s[i]);
-        const double si_sq = sq3(si), si0 = sqrt(si_sq);
-        const double fpi = fp[i];
-        const size_t ci = (size_t)coff[rr] + (i - R.atom0);
-        const double ge = gE[rr];
-        const double3 gf = make_double3(gF[3 * ci], gF[3 * ci + 1], gF[3 * ci + 2]);
-        const double3 gh = make_double3(gH[3 * ci], gH[3 * ci + 1], gH[3 * ci + 2]);
-        const double gh_si = dot3(gh, si);
-        double drho[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        const int nn = D.nbn[i];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 15;
+    const Basis B = pair_basis(M, l);
+    const int kind = l < 6 ? 0 : l < 14 ? 1 : 2;
+    double acc = 0.0, one = 0.0;  // this lane's pair parameter; lanes 0 to 5: aa, bb and Landau A to D
+    const int end = min(lb * per_block + per_block, D.N);
+    for (int i0 = lb * per_block + 4 * wave; i0 < end; i0 += 4 * kAdjWaves) {
+        const int i = i0 + (lane >> 4);
+        const int rr = i < end ? D.arep[i] : -1;
+        const Rep& R = D.rep[rr < 0 ? 0 : rr];
+        const double safe_sq = R.box.safe_sq;
+        const int nn = rr < 0 ? 0 : D.nbn[i];
         const int* nb = D.nb + (size_t)i * kMaxNb;
-        for (int k = 0; k < nn; ++k) {
-            const int j = nb[k];
-            double rsq;
-            const double3 rij = min_image_sq(b, sub3(ri, d3(D.r[j])), rsq);
-            const double r = sqrt(rsq);
-            const double cij = -dot3(gf, rij) / r;
+        double3 ri = make_double3(0.0, 0.0, 0.0), si = ri, gf = ri, gh = ri;
+        double fpi = 0.0, ge = 0.0;
+        if (rr >= 0) {
+            ri = d3(D.r[i]);
+            si = d3(D.s[i]);
+            fpi = fp[i];
+            ge = gE[rr];
+            const size_t ci = (size_t)coff[rr] + (i - R.atom0);
+            gf = make_double3(gF[3 * ci], gF[3 * ci + 1], gF[3 * ci + 2]);
+            gh = make_double3(gH[3 * ci], gH[3 * ci + 1], gH[3 * ci + 2]);
+        }
+        const double si_sq = sq3(si), si0 = sqrt(si_sq);
+        const double gh_si = dot3(gh, si);
+        double val = 0.0;  // the value's part: drho/da_k, or the sum itself
+        for (int k0 = 0; __ballot(k0 < nn) != 0; k0 += 16) {
+            double rp = M.rmax, qp = 0.0, w[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+            if (k0 + l < nn) {
+                const int j = nb[k0 + l];
+                double3 rij = sub3(ri, d3(D.r[j]));
+                double rsq = sq3(rij);
+                if (__builtin_expect(rsq >= safe_sq, 0)) {
+                    rij = min_image(R.box, rij);
+                    rsq = sq3(rij);
+                }
+                const double r = sqrt(rsq);
+                const double cij = -dot3(gf, rij) / r;
+                if (r < P.rcut_pot || r < P.rcut_mag) {
+                    int n;
+                    double ratio;
+                    interp_index(r, M.in_over_rmax, n, ratio);
+                    rp = r;
+                    qp = 0.5 * M.step * M.step * ratio * (1.0 - ratio);
+                }
+                if (r < P.rcut_pot) {
+                    w[0] = cij * (fpi + fp[j]);
+                    w[1] = cij;
+                    w[3] = 1.0;
+                    w[4] = ge * 0.5;
+                }
+                if (r < P.rcut_mag) {
+                    const double4 sj4 = D.s[j];
+                    const double3 sj = d3(sj4);
+                    const double X = dot3(si, sj) - sqrt(si_sq * sq3(sj));
+                    w[2] = -cij * X;
+                    w[5] = ge * (-0.5 * X) + (dot3(gh, sj) - (si0 > 0.0 ? sj4.w / si0 * gh_si : 0.0));
+                }
+            }
+            sR[wave][lane] = rp;
+            sQ[wave][lane] = qp;
+#pragma unroll
+            for (int q = 0; q < 6; ++q) sW[wave][q][lane] = w[q];
+            wave_fence();
+            const int left = min(nn - k0, 16);
+            for (int p = 0; p < left; ++p) {
+                const int at = (lane & 48) + p;
+                const double2 b = basis_at(M, B, sR[wave][at], sQ[wave][at]);
+                acc += sW[wave][kind][at] * b.y;
+                val += sW[wave][3 + kind][at] * b.x;
+            }
+            wave_fence();
+        }
+        if (rr >= 0) {
+            // one-body terms: F(rho_i) (energy), F'(rho_i) (through Q_i), Landau
             int n;
             double ratio;
-            interp_index(r, M.in_over_rmax, n, ratio);
-            const double* d0 = M.rd + (size_t)(n - 1) * kMRDStride;
-            const double* d1 = d0 + kMRDStride;
-            const double wr = 1.0 - ratio;
-            if (r < P.rcut_pot) {
-                const double fsum = fpi + fp[j];
-#pragma unroll
-                for (int q = 0; q < 6; ++q) {
-                    drho[q] += d0[2 * q] * ratio + d1[2 * q] * wr;
-                    acc[P_A0 + q] += cij * fsum * (d0[2 * q + 1] * ratio + d1[2 * q + 1] * wr);
-                }
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const double bv = d0[12 + 2 * q] * ratio + d1[12 + 2 * q] * wr;
-                    const double bdv = d0[13 + 2 * q] * ratio + d1[13 + 2 * q] * wr;
-                    acc[P_V0 + q] += ge * 0.5 * bv + cij * bdv;
-                }
+            interp_index(rho[i], M.in_over_rhomax, n, ratio);
+            const double* h0 = M.h + (size_t)(n - 1) * kMHStride;
+            const double* h1 = h0 + kMHStride;
+            const double slope_f = (h1[MH_F] - h0[MH_F]) * M.in_over_rhomax;
+            const double slope_fp = (h1[MH_DF] - h0[MH_DF]) * M.in_over_rhomax;
+            const double qi = Q[i];
+            acc += kind == 0 ? (ge * slope_f + qi * slope_fp) * val : val;
+            const double s2 = si_sq, s4 = s2 * s2, s6 = s4 * s2;
+            if (l < 2) {
+                const int kv = l == 0 ? MH_AA : MH_BB, kd = l == 0 ? MH_DAA : MH_DBB;
+                one += ge * lerp_tab(M.h, kMHStride, kv, n, ratio) + qi * lerp_tab(M.h, kMHStride, kd, n, ratio);
             }
-            if (r < P.rcut_mag) {
-                const double4 sj4 = D.s[j];
-                const double3 sj = d3(sj4);
-                const double X = dot3(si, sj) - sqrt(si_sq * sq3(sj));
-                const double hv = dot3(gh, sj) - (si0 > 0.0 ? sj4.w / si0 * gh_si : 0.0);
-                const double ba = d0[28] * ratio + d1[28] * wr, bda = d0[29] * ratio + d1[29] * wr;
-                const double bc = d0[30] * ratio + d1[30] * wr, bdc = d0[31] * ratio + d1[31] * wr;
-                acc[P_JA] += ge * (-0.5 * ba * X) + cij * (-bda * X) + ba * hv;
-                acc[P_JRC] += ge * (-0.5 * bc * X) + cij * (-bdc * X) + bc * hv;
-            }
+            if (l == 2) one += ge * s2 - 2.0 * gh_si;
+            if (l == 3) one += ge * s4 - 4.0 * s2 * gh_si;
+            if (l == 4) one += ge * s6 - 6.0 * s4 * gh_si;
+            if (l == 5) one += ge * s4 * s4 - 8.0 * s6 * gh_si;
         }
-        // one-body terms: F(rho_i) (energy), F'(rho_i) (through Q_i), Landau
-        int n;
-        double ratio;
-        interp_index(rho[i], M.in_over_rhomax, n, ratio);
-        const double* h0 = M.h + (size_t)(n - 1) * kMHStride;
-        const double* h1 = h0 + kMHStride;
-        const double slope_f = (h1[MH_F] - h0[MH_F]) * M.in_over_rhomax;
-        const double slope_fp = (h1[MH_DF] - h0[MH_DF]) * M.in_over_rhomax;
-        const double qi = Q[i];
-#pragma unroll
-        for (int q = 0; q < 6; ++q) acc[P_A0 + q] += (ge * slope_f + qi * slope_fp) * drho[q];
-        acc[P_AA] += ge * lerp_tab(M.h, kMHStride, MH_AA, n, ratio) + qi * lerp_tab(M.h, kMHStride, MH_DAA, n, ratio);
-        acc[P_BB] += ge * lerp_tab(M.h, kMHStride, MH_BB, n, ratio) + qi * lerp_tab(M.h, kMHStride, MH_DBB, n, ratio);
-        const double s2 = si_sq, s4 = s2 * s2, s6 = s4 * s2;
-        acc[P_LA + 0] += ge * s2 - 2.0 * gh_si;
-        acc[P_LA + 1] += ge * s4 - 4.0 * s2 * gh_si;
-        acc[P_LA + 2] += ge * s6 - 6.0 * s4 * gh_si;
-        acc[P_LA + 3] += ge * s4 * s4 - 8.0 * s6 * gh_si;
     }
-    model_partials<kNParam>(acc, partials, lb, (D.N + blockDim.x - 1) / blockDim.x);
+    acc += __shfl_xor(acc, 16, 64);
+    acc += __shfl_xor(acc, 32, 64);
+    one += __shfl_xor(one, 16, 64);
+    one += __shfl_xor(one, 32, 64);
+    if (lane < 16) {
+        sP[wave][0][l] = acc;
+        sP[wave][1][l] = one;
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < kNParam) {
+        // theta's order: 14 splines, aa and bb, the two of J, Landau
+        const int which = t < 14 || t == P_JA || t == P_JRC ? 0 : 1;
+        const int at = t < 14 ? t : t < P_JA ? t - P_AA : t < P_LA ? t - P_JA + 14 : t - P_LA + 2;
+        double v = 0.0;
+        for (int w = 0; w < kAdjWaves; ++w) v += sP[w][which][at];
+        partials[(size_t)t * nblocks + lb] = v;
+    }
 }
 
 }  // namespace sld

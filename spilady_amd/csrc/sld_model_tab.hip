@@ -4,10 +4,8 @@
 // stencil behind every second one, 16 threads) took about 250 ms of every
 // parameter change, against 2 ms for the whole loss gradient of 262,144
 // atoms. The rows are independent, so one thread makes one row and the rows
-// leave through LDS as contiguous lines: 448 MB in 154 us (2.9 TB/s; the
-// derivative table 70 us, the r values 65 us, the rho table 19 us). A training
-// step of 32 x 8,192 atoms went from 278 to 2.58 ms, of 4 x 1,024 from 277 to
-// 0.99 ms.
+// leave through LDS as contiguous lines: 192 MB in 83
+// us (the r values 64, the rho table 19).
 //
 // Every value is evaluated in the order of the forms' definition with no
 // contraction, so a table entry is the host's to the rounding of exp and log
@@ -19,25 +17,11 @@
 
 #include "sld_kernels.h"
 #include "sld_model.h"
+#include "sld_model_device.h"
 
 #pragma clang fp contract(off)
 
 namespace sld {
-
-__constant__ static const double kDFR[6] = {3.0, 2.8666666666666666, 2.7333333333333333, 2.6, 2.4, 2.3};
-__constant__ static const double kDVR[8] = {4.1, 3.8, 3.5, 3.2, 2.9, 2.6, 2.4, 2.3};
-
-// stencil slot s of a row at x: x, x + dx, x - dx, x + 2dx, x - 2dx, x + 3dx, x - 3dx
-__device__ __forceinline__ double stencil_x(double x, int s) {
-    const double dx = x / 1000e0;
-    const double d = (double)((s + 1) >> 1) * dx;
-    return s == 0 ? x : (s & 1 ? x + d : x - d);
-}
-
-__device__ __forceinline__ double stencil_deriv(const double (&v)[7], double x) {
-    const double dx = x / 1000e0;
-    return (45e0 * (v[1] - v[2]) - 9e0 * (v[3] - v[4]) + (v[5] - v[6])) / (60e0 * dx);
-}
 
 __device__ __forceinline__ double cube_knot(double R, double r) {
     const double d = R - r;
@@ -109,49 +93,6 @@ __global__ __launch_bounds__(256) void k_model_tab_r(ModelCoef m, const double* 
         const int row = e / kMRStride, c = e % kMRStride;
         o[e] = c < 12 ? sh[c >> 1][row + (c & 1)] : 0e0;
     }
-}
-
-// The derivative table: 64 rows of 32 columns a block of 64 threads.
-__global__ __launch_bounds__(64) void k_model_tab_rd(ModelCoef m, const double* bridge, double* out) {
-    constexpr int kPad = kMRDStride + 1;  // rows start on different LDS banks
-    __shared__ double sh[64 * kPad];
-    const int t = threadIdx.x;
-    const int n0 = blockIdx.x * 64, n = n0 + t;
-    if (n < kNInput) {
-        const double r = m.rmax / (double)kNInput * (double)(n + 1);
-        const double* q = bridge + (size_t)(n - m.row0) * kModelBridgeRow;
-        double* D = sh + t * kPad;
-        for (int k = 0; k < 6; ++k) {
-            double v[7];
-            for (int s = 0; s < 7; ++s) v[s] = cube_knot(kDFR[k], stencil_x(r, s));
-            D[2 * k] = v[0];
-            D[2 * k + 1] = stencil_deriv(v, r);
-        }
-        for (int k = 0; k < 8; ++k) {
-            double v[7];
-            for (int s = 0; s < 7; ++s) {
-                const double x = stencil_x(r, s);
-                v[s] = x <= 1.8 ? 0e0 : x <= 2.0 ? q[9 * s + 1 + k] : cube_knot(kDVR[k], x);
-            }
-            D[12 + 2 * k] = v[0];
-            D[13 + 2 * k] = stencil_deriv(v, r);
-        }
-        double a[7], b[7];
-        for (int s = 0; s < 7; ++s) {
-            const double x = stencil_x(r, s);
-            a[s] = cube_j(x, m.Jrc);
-            const double u = 1.0 - x / m.Jrc;
-            b[s] = x < m.Jrc ? m.JA * 3.0 * (u * u) * x / (m.Jrc * m.Jrc) : 0e0;
-        }
-        D[28] = a[0];
-        D[29] = stencil_deriv(a, r);
-        D[30] = b[0];
-        D[31] = stencil_deriv(b, r);
-    }
-    __syncthreads();
-    const int rows = min(64, kNInput - n0);
-    double* o = out + (size_t)n0 * kMRDStride;
-    for (int e = t; e < rows * kMRDStride; e += 64) o[e] = sh[(e / kMRDStride) * kPad + e % kMRDStride];
 }
 
 // The rho table: 256 rows of 8 columns a block.
