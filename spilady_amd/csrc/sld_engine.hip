@@ -126,7 +126,7 @@ struct sld_ctx {
         sld::ModelTab tab{};
         std::shared_ptr<const sld::ModelBridge> bridge;
         double* d_bridge = nullptr;
-        double *d_r = nullptr, *d_h = nullptr;
+        double *d_r = nullptr, *d_f = nullptr, *d_df = nullptr, *d_h = nullptr;
         double *d_rho = nullptr, *d_fp = nullptr, *d_Q = nullptr;
         double *d_F = nullptr, *d_H = nullptr, *d_gE = nullptr, *d_gF = nullptr, *d_gH = nullptr;
         double *d_E = nullptr, *d_grad = nullptr, *d_part = nullptr;
@@ -2006,6 +2006,7 @@ int sld_model_set_params(sld_ctx* c, const double* theta) {
         m.bridge = model_bridge(c->prm.rcut_max);
         TRY(upload_vec(c, &m.d_bridge, m.bridge->q));
         TRY(dalloc(c, &m.d_r, (size_t)kNInput * kMRStride));
+        TRY(dalloc(c, &m.d_f, kNInput)); TRY(dalloc(c, &m.d_df, kNInput));
         TRY(dalloc(c, &m.d_h, (size_t)kNInput * kMHStride));
         std::vector<int> coff(c->R);
         int tot = 0;
@@ -2023,10 +2024,12 @@ int sld_model_set_params(sld_ctx* c, const double* theta) {
         TRY(dalloc(c, &m.d_part, std::max((size_t)nblk(N, 256), (size_t)kNParam * kAdjBlocks)));
     }
     const ModelCoef mc = model_coef(theta, c->prm.rcut_max, *m.bridge);
-    LAUNCH(c, k_model_tab_r, nblk(kNInput - 1, 255), 256, mc, (const double*)m.d_bridge, m.d_r);
+    LAUNCH(c, k_model_tab_r, nblk(kNInput - 1, 255), 256, mc, (const double*)m.d_bridge, m.d_r, m.d_f, m.d_df);
     LAUNCH(c, k_model_tab_h, nblk(kNInput, 256), 256, mc, m.d_h);
     HIPCHK(c, hipStreamSynchronize(c->stream));
     m.tab.r = m.d_r;
+    m.tab.f = m.d_f;
+    m.tab.df = m.d_df;
     m.tab.JA = mc.JA;
     m.tab.Jrc = mc.Jrc;
     m.tab.rmax = mc.rmax;
@@ -2052,13 +2055,21 @@ int sld_model_get_params(sld_ctx* c, double* theta) {
 }  // extern "C"
 
 namespace {
-// densities and F'(rho) of the current configurations at the current parameters
-int model_rho(sld_ctx* c) {
-    auto& m = c->model;
-    if (!m.ready) return set_err(c, SLD_ERR_STATE, "model parameters not set (sld_model_set_params)");
+// what the passes over the current configurations need
+int model_ready(sld_ctx* c) {
+    if (!c->model.ready) return set_err(c, SLD_ERR_STATE, "model parameters not set (sld_model_set_params)");
     TRY(ensure_nb(c));
-    TRY(read_flags(c));
-    LAUNCH(c, k_model_rho, xcd_grid(nblk(c->D.N, 256)), 256, m.tab, c->phys, c->D, m.d_rho, m.d_fp);
+    return read_flags(c);
+}
+// energies, forces and fields into device buffers, partial sums of the energy included
+int model_forward(sld_ctx* c, double* rho, double* fp, double* F, double* H, double* part, double* esum) {
+    auto& m = c->model;
+    static_assert(kFwdAtoms == 256, "d_atom_seg counts blocks of 256 atoms");
+    LAUNCH(c, k_model_rho<false>, xcd_grid(nblk(c->D.N, 64)), 256, m.tab, c->phys, c->D, rho, fp, (const int*)nullptr,
+           (const double*)nullptr, (double*)nullptr);
+    LAUNCH(c, k_model_forward, xcd_grid(nblk(c->D.N, kFwdAtoms)), 4 * kFwdAtoms, m.tab, c->phys, c->D,
+           (const double*)rho, (const double*)fp, (const int*)m.d_coff, F, H, part);
+    LAUNCH(c, k_reduce_seg, c->R, 1024, (const double*)part, (const int*)c->d_atom_seg, 1, esum, 0);
     return SLD_OK;
 }
 
@@ -2075,11 +2086,8 @@ int sld_model_eval(sld_ctx* c, double* energy, double* force, double* field) {
     if (!c) return SLD_ERR_ARG;
     auto& m = c->model;
     c->ev_used = 0;
-    TRY(model_rho(c));
-    const int nb = nblk(c->D.N, 256);
-    LAUNCH(c, k_model_forward, xcd_grid(nb), 256, m.tab, c->phys, c->D, (const double*)m.d_rho, (const double*)m.d_fp,
-           (const int*)m.d_coff, m.d_F, m.d_H, m.d_part);
-    LAUNCH(c, k_reduce_seg, c->R, 1024, (const double*)m.d_part, (const int*)c->d_atom_seg, 1, m.d_E, 0);
+    TRY(model_ready(c));
+    TRY(model_forward(c, m.d_rho, m.d_fp, m.d_F, m.d_H, m.d_part, m.d_E));
     if (energy)
         HIPCHK(c, hipMemcpy2DAsync(energy, sizeof(double), m.d_E, kScal * sizeof(double), sizeof(double), c->R,
                                    hipMemcpyDefault, c->stream));
@@ -2096,7 +2104,7 @@ int sld_model_vjp(sld_ctx* c, const double* g_energy, const double* g_force, con
     if (!grad) return set_err(c, SLD_ERR_ARG, "null gradient output");
     auto& m = c->model;
     c->ev_used = 0;
-    TRY(model_rho(c));
+    TRY(model_ready(c));
     const size_t b3 = (size_t)3 * m.ntot * sizeof(double);
     if (g_energy) TRY(copy_any(c, m.d_gE, g_energy, c->R * sizeof(double)));
     else HIPCHK(c, hipMemsetAsync(m.d_gE, 0, c->R * sizeof(double), c->stream));
@@ -2104,8 +2112,8 @@ int sld_model_vjp(sld_ctx* c, const double* g_energy, const double* g_force, con
     else HIPCHK(c, hipMemsetAsync(m.d_gF, 0, b3, c->stream));
     if (g_field) TRY(copy_any(c, m.d_gH, g_field, b3));
     else HIPCHK(c, hipMemsetAsync(m.d_gH, 0, b3, c->stream));
-    const int nb = nblk(c->D.N, 256);
-    LAUNCH(c, k_model_q, xcd_grid(nb), 256, m.tab, c->phys, c->D, (const int*)m.d_coff, (const double*)m.d_gF, m.d_Q);
+    LAUNCH(c, k_model_rho<true>, xcd_grid(nblk(c->D.N, 64)), 256, m.tab, c->phys, c->D, m.d_rho, m.d_fp,
+           (const int*)m.d_coff, (const double*)m.d_gF, m.d_Q);
     // the kNParam partial sums of at most kAdjBlocks blocks, of 16 atoms at a time
     const int per = nblk(nblk(c->D.N, 16), kAdjBlocks) * 16, na = nblk(c->D.N, per);
     LAUNCH(c, k_model_adjoint, xcd_grid(na), 256, m.tab, c->phys, c->D, per, (const double*)m.d_rho, (const double*)m.d_fp,
@@ -2192,12 +2200,7 @@ int sld_model_eval_noalloc(sld_ctx* c, double* energy, double* force, double* fi
     // segmented sum one value per replica
     TRY(ensure_nb(c));
     TRY(read_flags(c));
-    LAUNCH(c, k_model_rho, xcd_grid(nb), 256, m.tab, c->phys, c->D, rho, fp);
-    double* F = force ? force : m.d_F;
-    double* H = field ? field : m.d_H;
-    LAUNCH(c, k_model_forward, xcd_grid(nb), 256, m.tab, c->phys, c->D, (const double*)rho, (const double*)fp,
-           (const int*)m.d_coff, F, H, part);
-    LAUNCH(c, k_reduce_seg, c->R, 1024, (const double*)part, (const int*)c->d_atom_seg, 1, esum, 0);
+    TRY(model_forward(c, rho, fp, force ? force : m.d_F, field ? field : m.d_H, part, esum));
     if (energy)
         HIPCHK(c, hipMemcpy2DAsync(energy, sizeof(double), esum, kScal * sizeof(double), sizeof(double), c->R,
                                    hipMemcpyDefault, c->stream));

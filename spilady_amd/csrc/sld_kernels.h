@@ -174,9 +174,11 @@ __global__ void k_unpack(XferArgs A, int N, const double* buf);
 __global__ void k_spin_len(Dev D, int a0, int n);
 
 // ---- parametric potential model (sld_model.hip) ----
-constexpr int kAdjBlocks = 2048;  // most blocks of the adjoint: four a compute unit
+constexpr int kAdjBlocks = 2048;  // most blocks of the adjoint
+constexpr int kFwdAtoms = 256;    // atoms of a block of the forward pass
 struct ModelTab {
     const double* r;    // [N][kMRStride]
+    const double *f, *df;  // [N]
     const double* h;    // [N][kMHStride]
     double in_over_rmax, in_over_rhomax;
     double L[4];        // Landau A B C D
@@ -185,12 +187,13 @@ struct ModelTab {
     const double* bridge;  // ModelBridge
     int row0;
 };
-__global__ void k_model_tab_r(ModelCoef m, const double* bridge, double* out);
+__global__ void k_model_tab_r(ModelCoef m, const double* bridge, double* out, double* out_f, double* out_df);
 __global__ void k_model_tab_h(ModelCoef m, double* out);
-__global__ void k_model_rho(ModelTab M, Phys P, Dev D, double* rho_out, double* fp_out);
+template <bool kQ>
+__global__ void k_model_rho(ModelTab M, Phys P, Dev D, double* rho_out, double* fp_out, const int* coff,
+                            const double* gF, double* Q);
 __global__ void k_model_forward(ModelTab M, Phys P, Dev D, const double* rho, const double* fp, const int* coff,
                                 double* F, double* H, double* partials);
-__global__ void k_model_q(ModelTab M, Phys P, Dev D, const int* coff, const double* gF, double* Q);
 __global__ void k_model_adjoint(ModelTab M, Phys P, Dev D, int per_block, const double* rho, const double* fp, const double* Q,
                                 const int* coff, const double* gE, const double* gF, const double* gH,
                                 double* partials);

@@ -19,12 +19,13 @@ enum ParamIndex { P_A0 = 0, P_V0 = 6, P_AA = 14, P_BB = 15, P_JA = 16, P_JRC = 1
 
 // Columns of the model tables (10^6 entries each, the reference's sampling
 // and 6-point derivative stencil):
-//   r value table   [N][16]: the interpolation pair (t[n-1], t[n]) of each of f f' V V' J J', then padding:
+//   r value table   [N][16]: the interpolation pair (t[n-1], t[n]) of each of f' V V' J J', then padding:
 //                            a lookup touches one 128-byte line
+//   f, f'           [N]:     for the passes that read nothing else
 //   rho table       [N][8]:  F F' dF/daa dF'/daa dF/dbb dF'/dbb - -
 constexpr int kMRStride = 16;
 constexpr int kMHStride = 8;
-enum MRCol { MR_F = 0, MR_DF, MR_V, MR_DV, MR_J, MR_DJ };
+enum MRCol { MR_DF = 0, MR_V, MR_DV, MR_J, MR_DJ };
 enum MHCol { MH_F = 0, MH_DF, MH_AA, MH_DAA, MH_BB, MH_DBB };
 
 // The quintic bridge of the pair term at the stencil points of the rows that

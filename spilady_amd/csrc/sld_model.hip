@@ -23,26 +23,6 @@
 
 namespace sld {
 
-template <int NK>
-__device__ __forceinline__ void model_partials(const double (&v)[NK], double* partials, int block, int nblocks) {
-    __shared__ double sh[NK][256];
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < NK; ++k) sh[k][t] = v[k];
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if (t < s) {
-#pragma unroll
-            for (int k = 0; k < NK; ++k) sh[k][t] += sh[k][t + s];
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-#pragma unroll
-        for (int k = 0; k < NK; ++k) partials[(size_t)k * nblocks + block] = sh[k][0];
-    }
-}
-
 // column k of the r value table at lookup n: the row holds the interpolation pair
 __device__ __forceinline__ double lerp_pair(const double* row, int k, double ratio) {
     const double2 t = reinterpret_cast<const double2*>(row)[k];
@@ -51,47 +31,88 @@ __device__ __forceinline__ double lerp_pair(const double* row, int k, double rat
 
 // density and F'(rho) of every atom (calculate_rho_CPU.cpp:33-92,
 // calculate_force_energy_CPU.cpp:98-107; the Fe Landau coefficients do not
-// depend on rho)
-__global__ __launch_bounds__(256) void k_model_rho(ModelTab M, Phys P, Dev D, double* rho_out, double* fp_out) {
-    const int lb = xcd_block((D.N + blockDim.x - 1) / blockDim.x);
+// depend on rho) and, for the adjoint (kQ), Q_i = sum_j (c_ij + c_ji) f'(r_ij).
+//
+// Four lanes an atom, lane j taking list entries j, j + 4, ...; the next
+// position is on its way while a pair is added. f and f' are tables of their
+// own, 8 MB of which the range below kFEnd stays in the L2s: from the 128-byte
+// rows of all columns, a lane an atom, the two sums took 218 and 234 us at
+// 262,144 atoms, and the adjoint made both, now 61 and, together, 81.
+template <bool kQ>
+__global__ __launch_bounds__(256) void k_model_rho(ModelTab M, Phys P, Dev D, double* rho_out, double* fp_out,
+                                                   const int* coff, const double* gF, double* Q) {
+    const int lb = xcd_block((4 * D.N + blockDim.x - 1) / blockDim.x);
     if (lb < 0) return;
-    const int i = lb * blockDim.x + threadIdx.x;
+    const int i = (lb * blockDim.x + threadIdx.x) >> 2, j = threadIdx.x & 3;
     if (i >= D.N) return;
     const int rr = D.arep[i];
     if (rr < 0) return;
-    const Box b = D.rep[rr].box;
+    const Rep& R = D.rep[rr];
+    const double safe_sq = R.box.safe_sq;
+    const double end_sq = fmin(P.rcut_pot_sq, kFEnd * kFEnd);
     const double3 ri = d3(D.r[i]);
-    double rho = 0.0;
+    const size_t c0 = kQ ? (size_t)coff[rr] - R.atom0 : 0;  // of atom a: 3 (c0 + a)
+    double3 gi = make_double3(0.0, 0.0, 0.0);
+    if (kQ) gi = make_double3(gF[3 * (c0 + i)], gF[3 * (c0 + i) + 1], gF[3 * (c0 + i) + 2]);
+    double rho = 0.0, q = 0.0;
     const int nn = D.nbn[i];
     const int* nb = D.nb + (size_t)i * kMaxNb;
-    for (int k = 0; k < nn; ++k) {
-        double rsq;
-        (void)min_image_sq(b, sub3(ri, d3(D.r[nb[k]])), rsq);
-        if (rsq < P.rcut_pot_sq) {
+    auto entry = [&](int k) { return k < nn ? nb[k] : i; };
+    int a = entry(j), next = entry(j + 4);
+    double4 ra = D.r[a];
+    for (int k = j; k < nn; k += 4) {
+        const int at = a;
+        double3 rij = sub3(ri, d3(ra));
+        a = next;
+        ra = D.r[a];
+        next = entry(k + 8);
+        double rsq = sq3(rij);
+        if (__builtin_expect(rsq >= safe_sq, 0)) {
+            rij = min_image(R.box, rij);
+            rsq = sq3(rij);
+        }
+        if (rsq < end_sq) {
+            const double r = sqrt(rsq);
             int n;
             double ratio;
-            interp_index(sqrt(rsq), M.in_over_rmax, n, ratio);
-            rho += lerp_pair(M.r + (size_t)n * kMRStride, MR_F, ratio);
+            interp_index(r, M.in_over_rmax, n, ratio);
+            rho += lerp_at(M.f, n, ratio);
+            if (kQ) {
+                const double* g = gF + 3 * (c0 + at);
+                q += -dot3(sub3(gi, make_double3(g[0], g[1], g[2])), rij) / r * lerp_at(M.df, n, ratio);
+            }
         }
     }
-    int n;
-    double ratio;
-    interp_index(rho, M.in_over_rhomax, n, ratio);
-    rho_out[i] = rho;
-    fp_out[i] = lerp_tab(M.h, kMHStride, MH_DF, n, ratio);
+    rho = quad_sum(rho);
+    if (kQ) q = quad_sum(q);
+    if (j == 0) {
+        int n;
+        double ratio;
+        interp_index(rho, M.in_over_rhomax, n, ratio);
+        rho_out[i] = rho;
+        fp_out[i] = lerp_tab(M.h, kMHStride, MH_DF, n, ratio);
+        if (kQ) Q[i] = q;
+    }
 }
+template __global__ void k_model_rho<false>(ModelTab, Phys, Dev, double*, double*, const int*, const double*, double*);
+template __global__ void k_model_rho<true>(ModelTab, Phys, Dev, double*, double*, const int*, const double*, double*);
 
-__global__ __launch_bounds__(256) void k_model_forward(ModelTab M, Phys P, Dev D, const double* rho,
+// Energies, forces and fields: four lanes an atom, blocks of kFwdAtoms atoms,
+// which are the rows of the energy's partial sums. 262,144 atoms take 135 us, a
+// line of the 128 MB table for each of 5.8 M pairs (5.5 TB/s); a lane an atom,
+// whose pairs waited for one another, took 265.
+__global__ __launch_bounds__(4 * kFwdAtoms) void k_model_forward(ModelTab M, Phys P, Dev D, const double* rho,
                                                        const double* fp, const int* coff, double* F,
                                                        double* H, double* partials) {
-    const int lb = xcd_block((D.N + blockDim.x - 1) / blockDim.x);
+    const int nblocks = (D.N + kFwdAtoms - 1) / kFwdAtoms;
+    const int lb = xcd_block(nblocks);
     if (lb < 0) return;  // whole padding block
-    const int i = lb * blockDim.x + threadIdx.x;
-    double acc[1] = {0.0};
+    const int i = lb * kFwdAtoms + (threadIdx.x >> 2), lane4 = threadIdx.x & 3;
+    double acc = 0.0;
     const int rr = i < D.N ? D.arep[i] : -1;
     if (rr >= 0) {
         const Rep& R = D.rep[rr];
-        const Box b = R.box;
+        const double safe_sq = R.box.safe_sq;
         const double3 ri = d3(D.r[i]);
         const double3 si = d3(D.s[i]);
         const double si_sq = sq3(si);
@@ -100,10 +121,14 @@ __global__ __launch_bounds__(256) void k_model_forward(ModelTab M, Phys P, Dev D
         double e = 0.0, S = 0.0;
         const int nn = D.nbn[i];
         const int* nb = D.nb + (size_t)i * kMaxNb;
-        for (int k = 0; k < nn; ++k) {
+        for (int k = lane4; k < nn; k += 4) {
             const int j = nb[k];
-            double rsq;
-            const double3 rij = min_image_sq(b, sub3(ri, d3(D.r[j])), rsq);
+            double3 rij = sub3(ri, d3(D.r[j]));
+            double rsq = sq3(rij);
+            if (__builtin_expect(rsq >= safe_sq, 0)) {
+                rij = min_image(R.box, rij);
+                rsq = sq3(rij);
+            }
             const double r = sqrt(rsq);
             int n;
             double ratio;
@@ -126,6 +151,10 @@ __global__ __launch_bounds__(256) void k_model_forward(ModelTab M, Phys P, Dev D
             }
             f = add3(f, mul3(-dudr / r, rij));
         }
+        e = quad_sum(e);
+        S = quad_sum(S);
+        f = make_double3(quad_sum(f.x), quad_sum(f.y), quad_sum(f.z));
+        h = make_double3(quad_sum(h.x), quad_sum(h.y), quad_sum(h.z));
         int n;
         double ratio;
         interp_index(rho[i], M.in_over_rhomax, n, ratio);
@@ -137,45 +166,23 @@ __global__ __launch_bounds__(256) void k_model_forward(ModelTab M, Phys P, Dev D
         const double hc = s0 > 0.0 ? -S / s0 : 0.0;
         h = add3(h, mul3(kl + hc, si));
         const size_t c = (size_t)coff[rr] + (i - R.atom0);
-        F[3 * c] = f.x; F[3 * c + 1] = f.y; F[3 * c + 2] = f.z;
-        H[3 * c] = h.x; H[3 * c + 1] = h.y; H[3 * c + 2] = h.z;
-        acc[0] = e;
+        if (lane4 < 3) {
+            F[3 * c + lane4] = lane4 == 0 ? f.x : lane4 == 1 ? f.y : f.z;
+            H[3 * c + lane4] = lane4 == 0 ? h.x : lane4 == 1 ? h.y : h.z;
+        }
+        if (lane4 == 0) acc = e;
     }
-    model_partials<1>(acc, partials, lb, (D.N + blockDim.x - 1) / blockDim.x);
+    __shared__ double sh[4 * kFwdAtoms / 64];
+    acc = wave_sum(acc);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double v = 0.0;
+        for (int w = 0; w < 4 * kFwdAtoms / 64; ++w) v += sh[w];
+        partials[lb] = v;
+    }
 }
 
-// adjoint, first pass: Q_i = sum_j (c_ij + c_ji) f'(r_ij)
-__global__ __launch_bounds__(256) void k_model_q(ModelTab M, Phys P, Dev D, const int* coff, const double* gF,
-                                                 double* Q) {
-    const int lb = xcd_block((D.N + blockDim.x - 1) / blockDim.x);
-    if (lb < 0) return;
-    const int i = lb * blockDim.x + threadIdx.x;
-    if (i >= D.N) return;
-    const int rr = D.arep[i];
-    if (rr < 0) return;
-    const Rep& R = D.rep[rr];
-    const Box b = R.box;
-    const double3 ri = d3(D.r[i]);
-    const size_t ci = (size_t)coff[rr] + (i - R.atom0);
-    const double3 gi = make_double3(gF[3 * ci], gF[3 * ci + 1], gF[3 * ci + 2]);
-    double q = 0.0;
-    const int nn = D.nbn[i];
-    const int* nb = D.nb + (size_t)i * kMaxNb;
-    for (int k = 0; k < nn; ++k) {
-        const int j = nb[k];
-        double rsq;
-        const double3 rij = min_image_sq(b, sub3(ri, d3(D.r[j])), rsq);
-        if (rsq >= P.rcut_pot_sq) continue;
-        const double r = sqrt(rsq);
-        const size_t cj = (size_t)coff[rr] + (j - R.atom0);
-        const double3 gj = make_double3(gF[3 * cj], gF[3 * cj + 1], gF[3 * cj + 2]);
-        int n;
-        double ratio;
-        interp_index(r, M.in_over_rmax, n, ratio);
-        q += -dot3(sub3(gi, gj), rij) / r * lerp_pair(M.r + (size_t)n * kMRStride, MR_DF, ratio);
-    }
-    Q[i] = q;
-}
 
 // The basis functions of the 16 pair parameters, one a lane: with d = R - r for
 // r < R, a density or pair spline is d^3, dJ/dA is d^3 / rc^3 and dJ/drc is

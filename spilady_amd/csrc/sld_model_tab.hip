@@ -50,8 +50,9 @@ __device__ __forceinline__ double big_f(const ModelCoef& m, double rho) {
 // Row n of the r value table holds the pairs (t[n-1], t[n]) of its columns;
 // a block of 256 threads evaluates entries n0 - 1 .. n0 + 254 and writes rows
 // n0 .. n0 + 254.
-__global__ __launch_bounds__(256) void k_model_tab_r(ModelCoef m, const double* bridge, double* out) {
-    __shared__ double sh[6][256];
+__global__ __launch_bounds__(256) void k_model_tab_r(ModelCoef m, const double* bridge, double* out, double* out_f,
+                                                     double* out_df) {
+    __shared__ double sh[5][256];
     const int t = threadIdx.x;
     const int n0 = 1 + blockIdx.x * 255;
     const int n = n0 - 1 + t;
@@ -79,8 +80,12 @@ __global__ __launch_bounds__(256) void k_model_tab_r(ModelCoef m, const double* 
             v[s] = b;
             J[s] = m.JA * cube_j(x, m.Jrc);
         }
-        sh[MR_F][t] = f[0];
-        sh[MR_DF][t] = stencil_deriv(f, r);
+        const double df = stencil_deriv(f, r);
+        if (t < 255 || n == kNInput - 1) {
+            out_f[n] = f[0];
+            out_df[n] = df;
+        }
+        sh[MR_DF][t] = df;
         sh[MR_V][t] = v[0];
         sh[MR_DV][t] = stencil_deriv(v, r);
         sh[MR_J][t] = J[0];
@@ -91,7 +96,7 @@ __global__ __launch_bounds__(256) void k_model_tab_r(ModelCoef m, const double* 
     double* o = out + (size_t)n0 * kMRStride;
     for (int e = t; e < rows * kMRStride; e += 256) {
         const int row = e / kMRStride, c = e % kMRStride;
-        o[e] = c < 12 ? sh[c >> 1][row + (c & 1)] : 0e0;
+        o[e] = c < 10 ? sh[c >> 1][row + (c & 1)] : 0e0;
     }
 }
 

@@ -14,7 +14,7 @@ from helpers import TOL, assert_close
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("sizes", [(5,), (4, 5, 6), (8,) * 33, (11,) * 26, (7, 9, 8) * 30])
+@pytest.mark.parametrize("sizes", [(5,), (5, 7, 6), (8,) * 33, (11,) * 26, (7, 9, 8) * 30])
 def test_a_large_context_is_the_sum_of_its_configurations(sizes):
     confs = [fit.frozen_configs(n, [400 + k])[0] for k, n in enumerate(sizes)]
     th = fit.perturbed_params(fit.default_params(), 0.02, 7)
