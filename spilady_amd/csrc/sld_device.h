@@ -303,9 +303,11 @@ __device__ __forceinline__ double te_to_ee(double te) {
     const double e = exp(x);
     return 3.0 / kCeB * log(0.5 * (e + 1.0 / e));
 }
+__device__ __forceinline__ bool te_fits(double ee) { return ee <= kPolyEMax && ee >= 1e-200; }
+__device__ __forceinline__ double ee_to_te_fit(double ee) { return sqrt_normal(ee) * horner2(kEeToTe.c, ee); }
 // T(E); outside the fitted range acosh(e^y) = y + log1p(sqrt(-expm1(-2y)))
 __device__ __forceinline__ double ee_to_te(double ee) {
-    if (ee <= kPolyEMax && ee >= 1e-200) return sqrt_normal(ee) * horner2(kEeToTe.c, ee);
+    if (te_fits(ee)) return ee_to_te_fit(ee);
     const double y = kCeB / 3.0 * ee;
     if (y <= kPolyYMax) return sqrt(2.0 * y) * horner(kAcoshExpG, y) * (1.0 / kCeB);
     return (y + log1p(sqrt(-expm1(-2.0 * y)))) / kCeB;

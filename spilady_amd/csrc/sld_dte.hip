@@ -125,9 +125,15 @@ __global__ __launch_bounds__(256) void k_dte_ab(double h, Mesh M, double* partia
 //
 // A sweep is a chain of up to 20 dependent cell updates whatever the mesh
 // size. A launch per level cost 3.5 us each; here a level costs one LDS round
-// trip, the update's FP64 chain and a barrier, 0.2 us.
+// trip, the update's FP64 chain and a barrier, 600 cycles or 0.25 us, of which
+// neither the number of waves nor the lists' loads are a part any more (7^3
+// cells, 33 levels of both sweeps: 14.2 us a launch, 15.7 with the lists
+// requested one level ahead, whose hand-over waited for them, and a branch per
+// lane for temperatures outside the fit; 33 x 25 x 10 cells 13.0 and 14.2).
 // The energy partials are one per tile: its cells in slot order, 64 at a
 // time, so the sum does not depend on the block size.
+constexpr int kAhead = 4;  // levels
+
 __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
     extern __shared__ double sT[];
     __shared__ double sp[kDteMaxSlot / 64 + 1];
@@ -155,16 +161,28 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
     const int bound = S.lev[T.lev0 + lane];  // lane l: first update of level l
     double* sE = sT + S.max_slot;
     constexpr int U = 4;  // slots of a thread in flight
+    int32_t c[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) c[u] = slot[min(t + u * B, T.nslot - 1)];
+    // a thread's first update of a level, requested kAhead levels ahead:
+    // ring[l % kAhead] (straight-line code, so that the wait before an update
+    // leaves the later requests in flight)
+    auto request = [&](int l) {
+        return upd[min(__builtin_amdgcn_readlane(bound, min(l, T.nlev)) + t, T.nent - 1)];
+    };
+    uint4 ring[kAhead];
+#pragma unroll
+    for (int l = 0; l < kAhead; ++l) ring[l] = request(l);
     for (int s0 = t; s0 < T.nslot; s0 += U * B) {
-        int c[U];
         double a[U], e[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) c[u] = T.origin + (slot[min(s0 + u * B, T.nslot - 1)] >> 1);
-#pragma unroll
         for (int u = 0; u < U; ++u) {
-            a[u] = A.Tin[c[u]];
-            e[u] = s0 + u * B < T.nupd ? A.Ein[c[u]] : 0.0;
+            const int cell = T.origin + (c[u] >> 1);
+            a[u] = A.Tin[cell];
+            e[u] = s0 + u * B < T.nupd ? A.Ein[cell] : 0.0;
         }
+#pragma unroll
+        for (int u = 0; u < U; ++u) c[u] = slot[min(s0 + (U + u) * B, T.nslot - 1)];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (s0 + u * B < T.nslot) sT[s0 + u * B] = a[u];
@@ -172,7 +190,10 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
         }
     }
     // one update (core_dTe_CPU.cpp:161-190)
-    auto update = [&](const uint4 d) {
+    auto update = [&](uint4 d) {
+        // keeps the split of the last word here: ahead of the loop's end it
+        // would wait for the requests
+        asm volatile("" : "+v"(d.w));
         char* q = reinterpret_cast<char*>(sT);
         auto at = [&](uint32_t o) -> double& { return *reinterpret_cast<double*>(q + o); };
         const uint32_t self = d.x & 0xffffu;
@@ -186,23 +207,33 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
         ee = fma(fma(-2.0, tc, typ + tym), A.py, ee);
         ee = fma(fma(-2.0, tc, tzp + tzm), A.pz, ee);
         E = ee;
-        at(self) = ee_to_te(ee);
+        double T = ee_to_te_fit(ee);
+        if (__builtin_expect(__ballot(!te_fits(ee)) != 0, 0)) T = ee_to_te(ee);  // without a branch per lane
+        at(self) = T;
     };
-    // a thread's first update of the next level is requested one level ahead
-    // (straight-line code: the wait before an update leaves the request in
-    // flight)
-    uint4 d = upd[min(t, T.nent - 1)];
     __syncthreads();
-    int lo = 0;
-    for (int l = 0; l < T.nlev; ++l) {
-        const int hi = __builtin_amdgcn_readlane(bound, l + 1);
-        const uint4 nx = upd[min(hi + t, T.nent - 1)];
-        if (lo + t < hi) update(d);
-        if (hi - lo > B)
-            for (int k = lo + B + t; k < hi; k += B) update(upd[k]);
-        d = nx;
-        lo = hi;
-        __syncthreads();
+    const int after = __shfl_down(bound, 1, 64);
+    if (__ballot(lane < T.nlev && after - bound > B) == 0) {  // a thread has at most one update a level
+        // past the last level nothing is left to update
+        int lo = 0, hi = __builtin_amdgcn_readlane(bound, 1);
+        for (int l0 = 0; l0 < T.nlev; l0 += kAhead) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const uint4 d = ring[u];
+                const bool on = lo + t < hi;
+                lo = hi;
+                hi = __builtin_amdgcn_readlane(bound, min(l0 + u + 2, T.nlev));
+                ring[u] = request(l0 + u + kAhead);
+                if (on) update(d);
+                __syncthreads();
+            }
+        }
+    } else {
+        for (int l = 0; l < T.nlev; ++l) {
+            const int hi = __builtin_amdgcn_readlane(bound, l + 1);
+            for (int k = __builtin_amdgcn_readlane(bound, l) + t; k < hi; k += B) update(upd[k]);
+            __syncthreads();
+        }
     }
     const int nch = (T.nupd + 63) >> 6;
     for (int q = t >> 6; q < nch; q += B >> 6) {
