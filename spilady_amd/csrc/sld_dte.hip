@@ -129,11 +129,12 @@ __global__ __launch_bounds__(256) void k_dte_ab(double h, Mesh M, double* partia
 // neither the number of waves nor the lists' loads are a part any more (7^3
 // cells, 33 levels of both sweeps: 14.2 us a launch, 15.7 with the lists
 // requested one level ahead, whose hand-over waited for them, and a branch per
-// lane for temperatures outside the fit; 33 x 25 x 10 cells 13.0 and 14.2).
+// lane for temperatures outside the fit; 33 x 25 x 10 cells 12.6 and 14.2).
 // The energy partials are one per tile: its cells in slot order, 64 at a
 // time, so the sum does not depend on the block size.
 constexpr int kAhead = 4;  // levels
 
+template <int U>
 __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
     extern __shared__ double sT[];
     __shared__ double sp[kDteMaxSlot / 64 + 1];
@@ -160,7 +161,10 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
     const int32_t* slot = S.slot + T.slot0;
     const int bound = S.lev[T.lev0 + lane];  // lane l: first update of level l
     double* sE = sT + S.max_slot;
-    constexpr int U = 4;  // slots of a thread in flight
+    // a thread's first U slots t, t + B, ... are in flight together, and their
+    // cells stay in registers until the results go out: 8 where a thread has
+    // that many (69^3 cells: 11.1 us a launch instead of 12.2), 4 where the
+    // other four would be loads for nothing (7^3: 14.1 and 14.8; 40^3 8.2 and 9.3)
     int32_t c[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) c[u] = slot[min(t + u * B, T.nslot - 1)];
@@ -173,21 +177,24 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
     uint4 ring[kAhead];
 #pragma unroll
     for (int l = 0; l < kAhead; ++l) ring[l] = request(l);
-    for (int s0 = t; s0 < T.nslot; s0 += U * B) {
+    {
         double a[U], e[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int cell = T.origin + (c[u] >> 1);
             a[u] = A.Tin[cell];
-            e[u] = s0 + u * B < T.nupd ? A.Ein[cell] : 0.0;
+            e[u] = t + u * B < T.nupd ? A.Ein[cell] : 0.0;
         }
-#pragma unroll
-        for (int u = 0; u < U; ++u) c[u] = slot[min(s0 + (U + u) * B, T.nslot - 1)];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (s0 + u * B < T.nslot) sT[s0 + u * B] = a[u];
-            if (s0 + u * B < T.nupd) sE[s0 + u * B] = e[u];
+            if (t + u * B < T.nslot) sT[t + u * B] = a[u];
+            if (t + u * B < T.nupd) sE[t + u * B] = e[u];
         }
+    }
+    for (int s = t + U * B; s < T.nslot; s += B) {
+        const int cell = T.origin + (slot[s] >> 1);
+        sT[s] = A.Tin[cell];
+        if (s < T.nupd) sE[s] = A.Ein[cell];
     }
     // one update (core_dTe_CPU.cpp:161-190)
     auto update = [&](uint4 d) {
@@ -236,10 +243,8 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
         }
     }
     const int nch = (T.nupd + 63) >> 6;
-    for (int q = t >> 6; q < nch; q += B >> 6) {
-        const int s = q * 64 + lane;
-        const int32_t c = s < T.nupd ? slot[s] : 0;
-        const bool own = (c & 1) != 0;
+    auto put = [&](int s, int32_t c) {
+        const bool own = s < T.nupd && (c & 1) != 0;
         const double ee = own ? sE[s] : 0.0;
         if (own) {
             A.Eout[T.origin + (c >> 1)] = ee;
@@ -247,9 +252,13 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
         }
         if (A.ends) {
             const double v = wave_sum(ee);
-            if (lane == 0) sp[q] = v;
+            if (lane == 0) sp[s >> 6] = v;
         }
-    }
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (((t + u * B) >> 6) < nch) put(t + u * B, c[u]);
+    for (int s = t + U * B; (s >> 6) < nch; s += B) put(s, slot[min(s, T.nslot - 1)]);
     if (A.ends) {
         __syncthreads();
         if (t < 64) {
@@ -260,6 +269,9 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
         }
     }
 }
+
+template __global__ void k_dte_sweep<4>(DteTiles, DteSweepArgs);
+template __global__ void k_dte_sweep<8>(DteTiles, DteSweepArgs);
 
 // the final energy of a sub-step from its n partials, by every block of 256
 // threads for itself in the same fixed order

@@ -528,8 +528,8 @@ int do_dTe_launches(sld_ctx* c, double dt) {
         for (int k = 0; k < c->dte_n; ++k) {
             const DteTiles& S = c->dte[k];
             const bool first = k == 0, last = k == c->dte_n - 1;
-            // with at most two tiles a compute unit a tile gets twice the waves
-            // (41^3 cells: 28.5 us a sub-step against 29.9; 69^3 in 729 tiles: 50.5 against 45.0)
+            // with at most two tiles a compute unit a tile gets twice the waves,
+            // and a thread half the slots in flight (41^3 cells: 28.5 us a sub-step against 29.9; 69^3 in 729 tiles: 50.5 against 45.0)
             const int bs = c->shapes.sweep_block * (S.ntile <= 512 ? 2 : 1);
             DteSweepArgs A{px, py, pz, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr};
             A.Tin = first ? c->D.Te : c->d_te2;
@@ -541,8 +541,8 @@ int do_dTe_launches(sld_ctx* c, double dt) {
             A.pa = c->d_part;
             A.na = nb;
             A.start = first ? start : nullptr;
-            hipLaunchKernelGGL(k_dte_sweep, dim3(xcd_grid(S.ntile) + (first ? 1 : 0)), dim3(bs), c->dte_lds[k], c->stream, S,
-                               A);
+            hipLaunchKernelGGL(S.ntile <= 512 ? k_dte_sweep<4> : k_dte_sweep<8>,
+                               dim3(xcd_grid(S.ntile) + (first ? 1 : 0)), dim3(bs), c->dte_lds[k], c->stream, S, A);
             HIPCHK(c, hipGetLastError());
         }
         const double* Eswept = c->dte_n == 1 ? c->d_ee2 : c->D.Ee;

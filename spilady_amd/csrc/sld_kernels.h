@@ -141,6 +141,7 @@ struct DteSweepArgs {
     int na;
     double* start;
 };
+template <int U>
 __global__ void k_dte_sweep(DteTiles S, DteSweepArgs A);
 // E: the energies the sweeps left; start: the sub-step's starting energy;
 // ends: nend partials of its final one
