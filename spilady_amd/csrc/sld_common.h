@@ -12,7 +12,7 @@ constexpr double kPi = 3.141592653589793238462e0;  // Pi_num (spilady.h:61)
 
 // potential tables (global.h:66): 10^6 points per table
 constexpr int kNInput = 1000000;
-constexpr int kRhoStride = 16;  // F dF A B C D dA dB dC dD pad...
+constexpr int kRhoStride = 10;  // F dF A B C D dA dB dC dD
 
 // The r table of the force pass: one 128-byte row per lookup index n holding
 // the pair (t[n-1], t[n]) that the interpolation at n reads, for each column, so

@@ -159,12 +159,12 @@ __device__ __forceinline__ int neigh_cell(const Box& b, int c, int slot) {
 // n = int(x * N / max) (potential_CPU.cpp:172-179). Entry k holds the value
 // at x = max * (k+1) / N.
 //   r tables: pairs (n - 1, n) of [dsf dpr pr dJ J]; J; sf
-//   rho tables interleaved per entry: [F dF A B C D dA dB dC dD - ...]
+//   rho tables interleaved per entry: [F dF A B C D dA dB dC dD]
 struct Tables {
     const double* prow;    // [NINPUT][16]
     const double* jtab;    // [NINPUT]
     const double* sftab;   // [NINPUT]
-    const double* rhotab;  // [NINPUT][16]
+    const double* rhotab;  // [NINPUT][10]
     double in_over_rmax, in_over_rhomax;
 };
 
