@@ -419,8 +419,16 @@ int do_ds(sld_ctx* c, double dt) {
     return SLD_OK;
 }
 
-// scalar block of each replica: [0..2] momentum sum, [3..4] kinetic energy
-// before and after centring
+// A replica's sums are added by a launch of their own (scalars 0..2 and 3..4 of
+// its block) or, if it has few partials, by each block of the next kernel: 2,000
+// atoms 4,450 us a ten-step pass instead of 4,523; above kFewRows the blocks'
+// reads (a replica's partials each) outgrow the 6 us of the launch.
+int most_rows(const std::vector<int>& seg) {
+    int m = 0;
+    for (size_t r = 0; r + 1 < seg.size(); ++r) m = std::max(m, seg[r + 1] - seg[r]);
+    return m;
+}
+
 int do_dp(sld_ctx* c, double dt) {
     int nb = nblk(c->D.C, 8);
     // quantum_noise (quantum_noise_CPU.cpp:60-81): every M-th core_dp_A call
@@ -433,11 +441,15 @@ int do_dp(sld_ctx* c, double dt) {
     // eight cells (8 lanes each) per 64-thread block
     LAUNCH(c, k_dp_cells, nb, 64, dt, c->phys, c->D, (int)(c->pass - c->pass_dev), c->d_part);
     if (c->phys.lattlang) c->pass++;
-    TRY(reduce_seg(c, c->d_cell8_seg, 3, 0));
-    int na = nblk(c->D.N, 256);
-    LAUNCH(c, k_dp_center, na, 256, c->phys, c->D, (const double*)c->d_scal, c->d_part);
-    TRY(reduce_seg(c, c->d_atom_seg, 2, 3));
-    LAUNCH(c, k_dp_scale, na, 256, c->phys, c->D, (const double*)c->d_scal);
+    const int na = nblk(c->D.N, 256);
+    const bool few_c = most_rows(c->cell8_seg) <= kFewRows, few_a = most_rows(c->atom_seg) <= kFewRows;
+    if (!few_c) TRY(reduce_seg(c, c->d_cell8_seg, 3, 0));
+    double* ke = c->d_part + (size_t)3 * nb;
+    LAUNCH(c, k_dp_center, na, 256, c->phys, c->D, (const double*)c->d_scal, (const double*)c->d_part,
+           few_c ? (const int*)c->d_cell8_seg : nullptr, nb, ke);
+    if (!few_a) LAUNCH(c, k_reduce_seg, c->R, 1024, (const double*)ke, (const int*)c->d_atom_seg, 2, c->d_scal, 3);
+    LAUNCH(c, k_dp_scale, na, 256, c->phys, c->D, (const double*)(c->d_scal + 3), (const double*)ke,
+           few_a ? (const int*)c->d_atom_seg : nullptr, na);
     return SLD_OK;
 }
 
@@ -1360,7 +1372,7 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
     TRY(dalloc(c, &D.sLup, C)); TRY(dalloc(c, &D.sLdn, C)); TRY(dalloc(c, &D.cellv, C));
     TRY(dalloc(c, &D.err, 1));
     int maxblk = std::max(nblk(N, 256), nblk(C, 8)) + 1;
-    TRY(dalloc(c, &c->d_part, (size_t)maxblk * 16));
+    TRY(dalloc(c, &c->d_part, (size_t)maxblk * 20));  // at most kObsAtomK + 1 components a block
     TRY(dalloc(c, &c->d_scal, (size_t)kScal * nrep));
     TRY(dalloc(c, &c->d_einit, 4));
     c->obs_cap = 1;

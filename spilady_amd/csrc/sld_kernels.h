@@ -116,8 +116,11 @@ template <bool kLang>
 __global__ void k_spin_phase(const int* cells, int ncell, int ncw, int backward, int store_fields, double dt,
                              Phys P, Dev D);
 __global__ void k_dp_cells(double dt, Phys P, Dev D, int pass_off, double* partials);
-__global__ void k_dp_center(Phys P, Dev D, const double* scal, double* partials);
-__global__ void k_dp_scale(Phys P, Dev D, const double* scal);
+// partial sums of a replica that every block of a kernel may add for itself
+constexpr int kFewRows = 512;
+__global__ void k_dp_center(Phys P, Dev D, const double* scal, const double* in, const int* seg, int nrow,
+                            double* partials);
+__global__ void k_dp_scale(Phys P, Dev D, const double* scal, const double* in, const int* seg, int nrow);
 __global__ void k_dr(double dt, Phys P, Dev D);
 __global__ void k_temperature(Tables T, Phys P, Dev D);
 __global__ void k_dte_ab(double h, Mesh M, double* partials);

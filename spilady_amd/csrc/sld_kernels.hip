@@ -849,14 +849,49 @@ __global__ __launch_bounds__(64) void k_dp_cells(double dt, Phys P, Dev D, int p
     block_partials<3>(acc, partials);
 }
 
-// rescale_momentum, part 1: remove the mean momentum (core_dp_CPU.cpp:270-302);
-// the replica's momentum sum is scal[0..2] of its scalar block
-__global__ __launch_bounds__(256) void k_dp_center(Phys P, Dev D, const double* scal, double* partials) {
+// The NK sums of the block's replica (a block of 256 slots holds one replica's
+// atoms, the first slot one of them): scal[0..NK) of its scalar block, or, given
+// seg, the sum of the rows seg[rr]..seg[rr + 1) of the nrow partial sums, at most
+// kFewRows, by every block for itself and to the bit what k_reduce_seg makes of
+// them. In replicas of 2,000 atoms that spares a step four launches of 4 us.
+template <int NK>
+__device__ __forceinline__ void replica_sums(const Dev& D, const double* scal, const double* in, const int* seg,
+                                             int nrow, double (&out)[NK]) {
+    const int rr = D.arep[(size_t)blockIdx.x * blockDim.x];
+#pragma unroll
+    for (int k = 0; k < NK; ++k) out[k] = 0.0;
+    if (rr < 0) return;
+    if (!seg) {
+#pragma unroll
+        for (int k = 0; k < NK; ++k) out[k] = scal[(size_t)rr * kScal + k];
+        return;
+    }
+    __shared__ double sh[kFewRows / 64][NK];
+    const int t = threadIdx.x, end = seg[rr + 1];
+#pragma unroll
+    for (int u = 0; u < kFewRows; u += 256) {
+        const int b = seg[rr] + u + t;
+#pragma unroll
+        for (int k = 0; k < NK; ++k) {
+            const double v = wave_sum(b < end ? in[(size_t)k * nrow + b] : 0.0);
+            if ((t & 63) == 0) sh[(u + t) >> 6][k] = v;
+        }
+    }
+    __syncthreads();
+    for (int w = 0; w < kFewRows / 64; ++w)
+#pragma unroll
+        for (int k = 0; k < NK; ++k) out[k] += sh[w][k];
+}
+
+// rescale_momentum, part 1: remove the mean momentum (core_dp_CPU.cpp:270-302)
+__global__ __launch_bounds__(256) void k_dp_center(Phys P, Dev D, const double* scal, const double* in,
+                                                   const int* seg, int nrow, double* partials) {
+    double psum[3];  // the replica's momentum
+    replica_sums(D, scal, in, seg, nrow, psum);
     int a = blockIdx.x * blockDim.x + threadIdx.x;
     double acc[2] = {0.0, 0.0};
     const int rr = a < D.N ? D.arep[a] : -1;
     if (rr >= 0) {
-        const double* psum = scal + (size_t)rr * kScal;
         const double inv_n = 1.0 / D.rep[rr].natom;
         double3 mean = make_double3(psum[0] * inv_n, psum[1] * inv_n, psum[2] * inv_n);
         double3 p = d3(D.p[a]);
@@ -868,14 +903,15 @@ __global__ __launch_bounds__(256) void k_dp_center(Phys P, Dev D, const double* 
     block_partials<2>(acc, partials);
 }
 
-// rescale_momentum, part 2, and the kinetic energies (core_dp_CPU.cpp:78-84,304-310);
-// the replica's kinetic energies before and after centring are scal[3..4]
-__global__ __launch_bounds__(256) void k_dp_scale(Phys P, Dev D, const double* scal) {
+// rescale_momentum, part 2, and the kinetic energies (core_dp_CPU.cpp:78-84,304-310)
+__global__ __launch_bounds__(256) void k_dp_scale(Phys P, Dev D, const double* scal, const double* in, const int* seg,
+                                                  int nrow) {
+    double ke2[2];  // the replica's kinetic energies before and after centring
+    replica_sums(D, scal, in, seg, nrow, ke2);
     int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= D.N) return;
     const int rr = D.arep[a];
     if (rr < 0) return;
-    const double* ke2 = scal + (size_t)rr * kScal + 3;
     double factor = sqrt(ke2[0] / ke2[1]);
     if (ke2[1] < 1e-10) factor = 1.0;
     double3 p = mul3(factor, d3(D.p[a]));
