@@ -267,16 +267,16 @@ int sld_kernel_timing(sld_ctx* ctx, int* launches, double* total_ms);
  * them: every reduction inside them sums per wavefront, so a trajectory is
  * bitwise the same under any valid shapes. */
 typedef struct {
-    int spin_block;        /* core_ds sweep level: eight times the most cells a wave takes; 32, 64 or 128 */
+    int spin_block;        /* core_ds sweep level: 16 times the most cells a wave takes; 32, 64 or 128 */
     int sweep_block;       /* core_dTe diffusion: threads of a tile's workgroup (twice as many on meshes of
                               up to 512 tiles); 64, 128 or 256 */
-    int force_block;       /* force/energy: threads (one per atom) per block; 64, 128 or 256 */
+    int force_block;       /* force/energy: threads (four per atom) per block; 64, 128 or 256 */
     int nbuild_cells;      /* neighbour build: link cells (one wave each) per block; 1, 2 or 4 */
-    int temperature_block; /* calculate_temperature: threads (32 per cell) per block; 64, 128 or 256 */
+    int temperature_block; /* calculate_temperature: threads (8 per cell) per block; 64, 128 or 256 */
     int sweep_tail;        /* kept for the layout: every level of a sweep runs inside its tile's workgroup;
                               0, 2048 or 8192 */
-    int spin_lanes;        /* core_ds sweep level: lanes that walk one cell (four times as many where the
-                              wave has them to spare); 1, 2 or 4 */
+    int spin_lanes;        /* core_ds sweep level: the waves it is spread over where it has too few cells, in
+                              units of 512; 1, 2 or 4 */
 } sld_shapes;
 int sld_get_shapes(sld_ctx* ctx, sld_shapes* out);
 /* How sld_step issues its work (no counterpart in the reference): 0 (default)
@@ -316,7 +316,8 @@ int sld_model_nparams(void);
 /* The reference's values of theta. */
 int sld_model_default_params(double* theta);
 /* Builds the model's tables (10^6 samples each, as potential_CPU.cpp:61-170)
- * at theta; about a second on the host. */
+ * at theta, on the device (about 0.1 ms; the first call also prepares the
+ * bridge's theta-independent part on the host). */
 int sld_model_set_params(sld_ctx* ctx, const double* theta);
 int sld_model_get_params(sld_ctx* ctx, double* theta);
 int sld_model_natoms(const sld_ctx* ctx);

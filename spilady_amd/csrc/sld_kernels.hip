@@ -1,9 +1,8 @@
 // HIP kernels of the spin-lattice engine (gfx950, FP64).
 //
-// Work decomposition: one thread per atom for the pair passes (neighbour
-// build + density, force), one thread per link cell for everything that the
-// reference runs as a sequential walk down a cell's list (spin sweeps,
-// Langevin momentum with local collective motion, cell temperatures).
+// Work decomposition: a wave per link cell for the neighbour build and density,
+// four lanes per atom for the force pass, eight lanes per link cell for the
+// Langevin momentum with local collective motion and the cell temperatures.
 // The spin sweeps are launched one dependency level at a time by the host;
 // within a launch no two cells interact. The electron diffusion sweeps run all
 // their levels inside tiles of the mesh.
@@ -377,14 +376,15 @@ __global__ __launch_bounds__(256) void k_fp(Tables T, Dev D) {
 // instruction touches 32 or 16 lines and not 64; the quad then swaps the pieces
 // by register moves (the columns after the interpolation).
 //
-// What bounds it are the rows: 44 M pairs of 2 M atoms read lines of a 64 MB
-// range, 3.1 GB from beyond the L2s. 893 us, where a lane an atom, which loaded
-// all of a pair by itself and had eight pairs in flight to hide it, took 1,340;
-// 64 x 16,000 atoms 655 (910), 250,000 atoms 110 (160), 2,000 14 (40). Smaller
-// rows lose again what they save as soon as a pair needs a second line (J in a
-// table of its own: 970 with rows of 64 bytes, 1,000 with entries of 32 that are
-// not stored twice), loads straight to LDS save the moves but not the lines
-// (970), and 128 registers spill (1,840).
+// What bounds it is the instruction stream, 1,970 a wave of 16 atoms, with three
+// waves a SIMD (158 registers) to hide the rows' latency; 1.5 GB come from beyond
+// the L2s. 2 M atoms 862 us, where a lane an atom, which loaded all of a pair by
+// itself, ten lines, and had eight pairs in flight to hide it, took 1,283 and
+// 3.8 GB; 64 x 16,000 atoms 636 (878), 250,000 atoms 109 (155), 2,000 13 (37).
+// Tried at 2 M atoms against 893 us on the same clock: rows of 64 bytes with J in
+// a table of its own 967, entries of 32 bytes that are not stored twice 1,000,
+// loads straight to LDS instead of register moves 970, no loads ahead 1,021, 128
+// registers with spills 1,840.
 __global__ __launch_bounds__(256) void k_force(Tables T, Phys P, Dev D) {
     const int lb = xcd_block((4 * D.N + blockDim.x - 1) / blockDim.x);
     if (lb < 0) return;
