@@ -89,25 +89,29 @@ __device__ __forceinline__ double dte_relax_steps(double e0, double dE, double g
     return e;
 }
 
+// What A and B take of cell c: h dE and g (see above).
+__device__ __forceinline__ double2 dte_source(const Mesh& M, int c, double h) {
+    double dE = 0.0, G = 0.0;
+    if (M.lattlang) {
+        dE += M.Gel[c] * M.Tl[c];
+        G += M.Gel[c];
+    }
+    if (M.spinlang) {
+        dE += M.Ges[c] * M.TsL[c];
+        G += M.Ges[c];
+    }
+    return make_double2(dE * h, G * (h / kBoltz) * (-1.0 / (3.0 * kCeB)));
+}
+
 // the first sub-step's A(h), B(h), then Ee = E(Te) as C starts
 __global__ __launch_bounds__(256) void k_dte_ab(double h, Mesh M, double* partials) {
     int c = blockIdx.x * blockDim.x + threadIdx.x;
     double acc[1] = {0.0};
     if (c < M.C) {
-        double dE = 0.0, G = 0.0;
-        if (M.lattlang) {
-            dE += M.Gel[c] * M.Tl[c];
-            G += M.Gel[c];
-        }
-        if (M.spinlang) {
-            dE += M.Ges[c] * M.TsL[c];
-            G += M.Ges[c];
-        }
-        dE *= h;
-        const double g = G * (h / kBoltz) * (-1.0 / (3.0 * kCeB));
-        M.src[c] = make_double2(dE, g);
+        const double2 src = dte_source(M, c, h);
+        M.src[c] = src;
         double T;
-        const double ee = dte_relax_steps(te_to_ee(M.Te[c]) + dE, dE, g, 1, T);
+        const double ee = dte_relax_steps(te_to_ee(M.Te[c]) + src.x, src.x, src.y, 1, T);
         M.Te[c] = T;
         M.Ee[c] = ee;
         acc[0] = ee;
@@ -133,6 +137,67 @@ __global__ __launch_bounds__(256) void k_dte_ab(double h, Mesh M, double* partia
 // The energy partials are one per tile: its cells in slot order, 64 at a
 // time, so the sum does not depend on the block size.
 constexpr int kAhead = 4;  // levels
+
+// a thread's first update of level l; bound: in lane l, the first update of level l
+__device__ __forceinline__ uint4 dte_request(const DteTile& T, const uint4* upd, int bound, int l) {
+    return upd[min(__builtin_amdgcn_readlane(bound, min(l, T.nlev)) + (int)threadIdx.x, T.nent - 1)];
+}
+
+// one update (core_dTe_CPU.cpp:161-190)
+__device__ __forceinline__ void dte_update(uint4 d, double* sT, double* sE, double px, double py, double pz) {
+    // keeps the split of the last word here: ahead of the loop's end it
+    // would wait for the requests
+    asm volatile("" : "+v"(d.w));
+    char* q = reinterpret_cast<char*>(sT);
+    auto at = [&](uint32_t o) -> double& { return *reinterpret_cast<double*>(q + o); };
+    const uint32_t self = d.x & 0xffffu;
+    const double txp = at(d.x >> 16), txm = at(d.y & 0xffffu);
+    const double typ = at(d.y >> 16), tym = at(d.z & 0xffffu);
+    const double tzp = at(d.z >> 16), tzm = at(d.w & 0xffffu);
+    const double tc = at(self);
+    double& E = *reinterpret_cast<double*>(reinterpret_cast<char*>(sE) + self);
+    double ee = E;
+    ee = fma(fma(-2.0, tc, txp + txm), px, ee);
+    ee = fma(fma(-2.0, tc, typ + tym), py, ee);
+    ee = fma(fma(-2.0, tc, tzp + tzm), pz, ee);
+    E = ee;
+    double T = ee_to_te_fit(ee);
+    if (__builtin_expect(__ballot(!te_fits(ee)) != 0, 0)) T = ee_to_te(ee);  // without a branch per lane
+    at(self) = T;
+}
+
+// The levels of a tile, a workgroup barrier after each. ring[l]: the thread's
+// first update of level l < kAhead; from there on they are requested kAhead
+// levels ahead (straight-line code, so that the wait before an update leaves
+// the later requests in flight).
+__device__ __forceinline__ void dte_levels(const DteTile& T, const uint4* upd, int bound, uint4 (&ring)[kAhead],
+                                           double* sT, double* sE, double px, double py, double pz) {
+    const int t = threadIdx.x, B = blockDim.x, lane = t & 63;
+    const int after = __shfl_down(bound, 1, 64);
+    if (__ballot(lane < T.nlev && after - bound > B) == 0) {  // a thread has at most one update a level
+        // past the last level nothing is left to update
+        int lo = 0, hi = __builtin_amdgcn_readlane(bound, 1);
+        for (int l0 = 0; l0 < T.nlev; l0 += kAhead) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const uint4 d = ring[u];
+                const bool on = lo + t < hi;
+                lo = hi;
+                hi = __builtin_amdgcn_readlane(bound, min(l0 + u + 2, T.nlev));
+                ring[u] = dte_request(T, upd, bound, l0 + u + kAhead);
+                if (on) dte_update(d, sT, sE, px, py, pz);
+                __syncthreads();
+            }
+        }
+    } else {
+        for (int l = 0; l < T.nlev; ++l) {
+            const int hi = __builtin_amdgcn_readlane(bound, l + 1);
+            for (int k = __builtin_amdgcn_readlane(bound, l) + t; k < hi; k += B)
+                dte_update(upd[k], sT, sE, px, py, pz);
+            __syncthreads();
+        }
+    }
+}
 
 template <int U>
 __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
@@ -168,15 +233,9 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
     int32_t c[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) c[u] = slot[min(t + u * B, T.nslot - 1)];
-    // a thread's first update of a level, requested kAhead levels ahead:
-    // ring[l % kAhead] (straight-line code, so that the wait before an update
-    // leaves the later requests in flight)
-    auto request = [&](int l) {
-        return upd[min(__builtin_amdgcn_readlane(bound, min(l, T.nlev)) + t, T.nent - 1)];
-    };
     uint4 ring[kAhead];
 #pragma unroll
-    for (int l = 0; l < kAhead; ++l) ring[l] = request(l);
+    for (int l = 0; l < kAhead; ++l) ring[l] = dte_request(T, upd, bound, l);
     {
         double a[U], e[U];
 #pragma unroll
@@ -196,52 +255,8 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
         sT[s] = A.Tin[cell];
         if (s < T.nupd) sE[s] = A.Ein[cell];
     }
-    // one update (core_dTe_CPU.cpp:161-190)
-    auto update = [&](uint4 d) {
-        // keeps the split of the last word here: ahead of the loop's end it
-        // would wait for the requests
-        asm volatile("" : "+v"(d.w));
-        char* q = reinterpret_cast<char*>(sT);
-        auto at = [&](uint32_t o) -> double& { return *reinterpret_cast<double*>(q + o); };
-        const uint32_t self = d.x & 0xffffu;
-        const double txp = at(d.x >> 16), txm = at(d.y & 0xffffu);
-        const double typ = at(d.y >> 16), tym = at(d.z & 0xffffu);
-        const double tzp = at(d.z >> 16), tzm = at(d.w & 0xffffu);
-        const double tc = at(self);
-        double& E = *reinterpret_cast<double*>(reinterpret_cast<char*>(sE) + self);
-        double ee = E;
-        ee = fma(fma(-2.0, tc, txp + txm), A.px, ee);
-        ee = fma(fma(-2.0, tc, typ + tym), A.py, ee);
-        ee = fma(fma(-2.0, tc, tzp + tzm), A.pz, ee);
-        E = ee;
-        double T = ee_to_te_fit(ee);
-        if (__builtin_expect(__ballot(!te_fits(ee)) != 0, 0)) T = ee_to_te(ee);  // without a branch per lane
-        at(self) = T;
-    };
     __syncthreads();
-    const int after = __shfl_down(bound, 1, 64);
-    if (__ballot(lane < T.nlev && after - bound > B) == 0) {  // a thread has at most one update a level
-        // past the last level nothing is left to update
-        int lo = 0, hi = __builtin_amdgcn_readlane(bound, 1);
-        for (int l0 = 0; l0 < T.nlev; l0 += kAhead) {
-#pragma unroll
-            for (int u = 0; u < kAhead; ++u) {
-                const uint4 d = ring[u];
-                const bool on = lo + t < hi;
-                lo = hi;
-                hi = __builtin_amdgcn_readlane(bound, min(l0 + u + 2, T.nlev));
-                ring[u] = request(l0 + u + kAhead);
-                if (on) update(d);
-                __syncthreads();
-            }
-        }
-    } else {
-        for (int l = 0; l < T.nlev; ++l) {
-            const int hi = __builtin_amdgcn_readlane(bound, l + 1);
-            for (int k = __builtin_amdgcn_readlane(bound, l) + t; k < hi; k += B) update(upd[k]);
-            __syncthreads();
-        }
-    }
+    dte_levels(T, upd, bound, ring, sT, sE, A.px, A.py, A.pz);
     const int nch = (T.nupd + 63) >> 6;
     auto put = [&](int s, int32_t c) {
         const bool own = s < T.nupd && (c & 1) != 0;
@@ -325,6 +340,77 @@ __global__ __launch_bounds__(256) void k_dte_finish(Mesh M, const double* E, con
     const double ee = dte_relax_steps(E[c] * f, src.x, src.y, 1, T) + src.x;
     M.Ee[c] = ee;
     M.Te[c] = ee_to_te(ee);
+}
+
+// A whole core_dTe call of a small mesh, one tile, in one workgroup: the
+// temperatures, energies and sources stay in LDS for all sub-steps. A sub-step
+// takes its levels (0.29 us each), one relaxation a thread and two sums, and no
+// launch: a call of 7^3 cells 692 us where two launches a sub-step took 970, of
+// 8^3 333 (621), of 10^3 479 (615). From there on the relaxations, two and more a
+// thread, are worth more compute units: 11^3 936 and 942, 12^3 744 and 636, so
+// the line is at kDteSmall cells. (The relaxation as a function of its own, to
+// spare scalar registers, made the levels slower: 885 us at 7^3.)
+__global__ __launch_bounds__(512) void k_dte_small(DteTiles S, Mesh M, double h, double px, double py, double pz,
+                                                   int nloop) {
+    extern __shared__ double sT[];
+    __shared__ double sp[kDteSmall / 64];
+    const int t = threadIdx.x, B = blockDim.x, lane = t & 63;
+    const DteTile T = S.tile[0];
+    const uint4* upd = S.upd + T.upd0;
+    const int32_t* slot = S.slot + T.slot0;
+    const int bound = S.lev[T.lev0 + lane];
+    double* sE = sT + kDteSmall;
+    double2* src = reinterpret_cast<double2*>(sE + kDteSmall);
+    uint4 first[kAhead];
+#pragma unroll
+    for (int l = 0; l < kAhead; ++l) first[l] = dte_request(T, upd, bound, l);
+    // sum of the energies, in chunks of 64 cells
+    const int nch = (M.C + 63) >> 6;
+    auto total = [&]() {
+        for (int q = t >> 6; q < nch; q += B >> 6) {
+            const int s = q * 64 + lane;
+            const double v = wave_sum(s < M.C ? sE[s] : 0.0);
+            if (lane == 0) sp[q] = v;
+        }
+        __syncthreads();
+        return wave_sum(lane < nch ? sp[lane] : 0.0);
+    };
+    for (int s = t; s < M.C; s += B) {
+        const int c = T.origin + (slot[s] >> 1);
+        const double2 a = dte_source(M, c, h);
+        double Tn;
+        sE[s] = dte_relax_steps(te_to_ee(M.Te[c]) + a.x, a.x, a.y, 1, Tn);
+        sT[s] = Tn;
+        src[s] = a;
+    }
+    __syncthreads();
+    for (int it = 0; it < nloop; ++it) {
+        const double start = total();
+        uint4 ring[kAhead];
+#pragma unroll
+        for (int l = 0; l < kAhead; ++l) ring[l] = first[l];
+        dte_levels(T, upd, bound, ring, sT, sE, px, py, pz);
+        const double f = start / total();
+        // renormalise, B(h), A(h), and the next sub-step's A(h), B(h)
+        const bool last = it + 1 == nloop;
+        for (int s = t; s < M.C; s += B) {
+            const double2 a = src[s];
+            double Tn;
+            double ee = dte_relax_steps(sE[s] * f, a.x, a.y, last ? 1 : 2, Tn);
+            if (last) {
+                ee += a.x;
+                Tn = ee_to_te(ee);
+            }
+            sE[s] = ee;
+            sT[s] = Tn;
+        }
+        __syncthreads();
+    }
+    for (int s = t; s < M.C; s += B) {
+        const int c = T.origin + (slot[s] >> 1);
+        M.Ee[c] = sE[s];
+        M.Te[c] = sT[s];
+    }
 }
 
 }  // namespace sld

@@ -79,6 +79,7 @@ struct sld_ctx {
     // electron diffusion: tile schedules of the forward and the backward
     // sweep, or one of both together, and the second copy of the mesh
     int dte_n = 0;
+    bool dte_small = false;  // one tile, one launch a core_dTe call
     DteTiles dte[2] = {};
     size_t dte_lds[2] = {0, 0};
     double *d_te2 = nullptr, *d_ee2 = nullptr;
@@ -524,12 +525,21 @@ int do_dTe_launches(sld_ctx* c, double dt) {
     int nb = nblk(c->D.C, 256);
     const Mesh M{c->D.Te, c->D.Ee, c->D.Gel, c->D.Ges, c->D.Tl, c->D.TsL, c->d_dte_src, c->D.C, c->phys.lattlang,
                  c->phys.spinlang};
+    const double px = pref / h0.dx2, py = pref / h0.dy2, pz = pref / h0.dz2;
+    if (c->dte_small) {
+        hipEvent_t* ev = timing_slot(c, "k_dte_sweep");  // the sweeps' name for all meshes
+        if (ev) (void)hipEventRecord(ev[0], c->stream);
+        hipLaunchKernelGGL(k_dte_small, dim3(1), dim3(2 * c->shapes.sweep_block), 32 * kDteSmall, c->stream, c->dte[0], M,
+                           h, px, py, pz, nloop);
+        HIPCHK(c, hipGetLastError());
+        if (ev) (void)hipEventRecord(ev[1], c->stream);
+        return SLD_OK;
+    }
     LAUNCH(c, k_dte_ab, nb, 256, h, M, c->d_part);
     // block partials: [0, nb) starting energies (k_dte_ab / k_dte_finish_ab),
     // then the final energies of the backward sweep's tiles
     double* start = c->d_scal + 8;
     double* ends = c->d_part + nb;
-    const double px = pref / h0.dx2, py = pref / h0.dy2, pz = pref / h0.dz2;
     for (int it = 0; it < nloop; ++it) {
         // the sub-step's sweeps timed as one span
         hipEvent_t* ev = timing_slot(c, "k_dte_sweep");
@@ -1093,15 +1103,19 @@ int upload_dte_schedules(sld_ctx* c) {
     // Both sweeps in one launch save a launch's latency and a pass over the
     // mesh and compute the larger closure: kept where that is small, on meshes
     // of few levels (40^3 cells, 8 levels: 17.4 us a sub-step against 20.0;
-    // 100^3: 70 against 74) and on small ones (7^3: 22.7 against 25.7;
-    // 33 x 25 x 10: 22.8 against 23.6). 41^3 cells, 36 levels: 31.9 against 28.5.
+    // 100^3: 70 against 74) and on small ones (33 x 25 x 10: 22.8 against 23.6).
+    // 41^3 cells, 36 levels: 31.9 against 28.5. The smallest meshes are one tile
+    // and one launch for the whole call (k_dte_small).
     constexpr int kFewLevels = 16, kSmallMesh = 10000;
     auto make = [&](DteSweeps sw, int e, int most_levels, DteSchedule& S) {
         return dte_schedule(hc.nx, hc.ny, hc.nz, group, sw, e, e, e, most_levels, S) &&
                8 * ((size_t)S.max_slot + S.max_upd) <= kDteLds;
     };
     std::vector<DteSchedule> sch(1);
-    if (!make(kDteBoth, dte_tile_edge(hc, 512), hc.C <= kSmallMesh ? kDteMaxLev : kFewLevels, sch[0])) {
+    c->dte_small = hc.C <= kDteSmall &&
+                   dte_schedule(hc.nx, hc.ny, hc.nz, group, kDteBoth, hc.nx, hc.ny, hc.nz, kDteMaxLev, sch[0]) &&
+                   sch[0].tile.size() == 1;
+    if (!c->dte_small && !make(kDteBoth, dte_tile_edge(hc, 512), hc.C <= kSmallMesh ? kDteMaxLev : kFewLevels, sch[0])) {
         sch.resize(2);
         int e = dte_tile_edge(hc, 768);
         while (!(make(kDteForward, e, kDteMaxLev, sch[0]) && make(kDteBackward, e, kDteMaxLev, sch[1]))) {

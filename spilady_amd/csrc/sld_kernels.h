@@ -144,6 +144,9 @@ struct DteSweepArgs {
     int na;
     double* start;
 };
+// cells of a mesh that one workgroup sweeps on its own: 32 bytes of LDS a cell
+constexpr int kDteSmall = 1024;
+__global__ void k_dte_small(DteTiles S, Mesh M, double h, double px, double py, double pz, int nloop);
 template <int U>
 __global__ void k_dte_sweep(DteTiles S, DteSweepArgs A);
 // E: the energies the sweeps left; start: the sub-step's starting energy;
