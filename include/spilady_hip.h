@@ -33,7 +33,7 @@ extern "C" {
 #define SLD_OK 0
 #define SLD_ERR_ARG 1       /* invalid argument or input state */
 #define SLD_ERR_HIP 2       /* a HIP runtime call failed */
-#define SLD_ERR_CAPACITY 3  /* a fixed per-cell/per-atom capacity was exceeded */
+#define SLD_ERR_CAPACITY 3  /* a fixed per-cell/per-atom capacity or the host's memory was exceeded */
 #define SLD_ERR_STATE 4     /* call not valid in the context's current state */
 #define SLD_ERR_NOGPU 5     /* no usable gfx950 device */
 

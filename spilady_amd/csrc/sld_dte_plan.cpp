@@ -2,8 +2,9 @@
 #include "sld_dte_plan.h"
 
 #include <algorithm>
-#include <thread>
 #include <unordered_map>
+
+#include "sld_threads.h"
 
 namespace sld {
 namespace {
@@ -207,11 +208,7 @@ bool dte_schedule(int nx, int ny, int nz, const std::vector<int>& group, DteSwee
     int nt = (int)std::min(std::max(std::thread::hardware_concurrency(), 1u), 16u);
     nt = std::max(1, std::min(nt, ntile / 8));
     std::vector<Made> made(nt);
-    std::vector<std::thread> th;
-    for (int k = 1; k < nt; ++k)
-        th.emplace_back(work, (int)((long)ntile * k / nt), (int)((long)ntile * (k + 1) / nt), std::ref(made[k]));
-    work(0, (int)((long)ntile / nt), made[0]);
-    for (auto& x : th) x.join();
+    run_parts(nt, [&](int k) { work((int)((long)ntile * k / nt), (int)((long)ntile * (k + 1) / nt), made[k]); });
 
     out = DteSchedule();
     std::vector<Lists> all;

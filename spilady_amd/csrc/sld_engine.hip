@@ -13,7 +13,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -146,6 +148,19 @@ int set_err(sld_ctx* c, int code, const char* fmt, ...) {
     va_end(ap);
     if (c) c->err = buf;
     return code;
+}
+
+// f's code; what the host work in it throws becomes an error code, since no
+// exception may leave a C entry
+template <class F>
+int no_throw(sld_ctx* c, F f) {
+    try {
+        return f();
+    } catch (const std::bad_alloc&) {
+        return set_err(c, SLD_ERR_CAPACITY, "out of host memory");
+    } catch (const std::exception& e) {
+        return set_err(c, SLD_ERR_STATE, "%s", e.what());
+    }
 }
 
 #define HIPCHK(ctx, call)                                                                  \
@@ -1540,10 +1555,10 @@ int sld_create_batch(int nrep, const sld_params* params, const sld_atoms* init, 
                      sld_ctx** out) {
     if (!params || !init || !out) return SLD_ERR_ARG;
     *out = nullptr;
-    sld_ctx* c = new sld_ctx();
-    int rc = create_impl(c, nrep, params, init, compute_initial_forces);
+    sld_ctx* c = new (std::nothrow) sld_ctx();
+    if (!c) return SLD_ERR_CAPACITY;
     *out = c;  // returned even on failure so that sld_last_error can be read
-    return rc;
+    return no_throw(c, [&] { return create_impl(c, nrep, params, init, compute_initial_forces); });
 }
 
 int sld_nreplicas(const sld_ctx* c) { return c ? c->R : 0; }
@@ -2029,7 +2044,10 @@ int sld_model_set_params(sld_ctx* c, const double* theta) {
     auto& m = c->model;
     const int N = c->D.N;
     if (!m.d_r) {
-        m.bridge = model_bridge(c->prm.rcut_max);
+        TRY(no_throw(c, [&] {
+            m.bridge = model_bridge(c->prm.rcut_max);
+            return SLD_OK;
+        }));
         TRY(upload_vec(c, &m.d_bridge, m.bridge->q));
         TRY(dalloc(c, &m.d_r, (size_t)kNInput * kMRStride));
         TRY(dalloc(c, &m.d_f, kNInput)); TRY(dalloc(c, &m.d_df, kNInput));

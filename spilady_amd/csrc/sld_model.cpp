@@ -25,6 +25,7 @@
 #include "sld_common.h"
 #include "sld_model.h"
 #include "sld_tables.h"
+#include "sld_threads.h"
 
 namespace sld {
 namespace {
@@ -75,11 +76,9 @@ void fill_bridge(double rmax, ModelBridge& t) {
                     for (int p = 0; p < 9; ++p) t.q[((size_t)k * 7 + s) * 9 + p] = quintic(q[p], x[s]);
         }
     };
-    unsigned nt = std::min(std::max(std::thread::hardware_concurrency(), 1u), 16u);
-    std::vector<std::thread> th;
-    const int chunk = (t.nrow + (int)nt - 1) / (int)nt;
-    for (int a = 0; a < t.nrow; a += chunk) th.emplace_back(work, a, std::min(a + chunk, t.nrow));
-    for (auto& x : th) x.join();
+    const int nt = (int)std::min(std::max(std::thread::hardware_concurrency(), 1u), 16u);
+    const int chunk = (t.nrow + nt - 1) / nt;
+    run_parts(nt, [&](int k) { work(k * chunk, std::min((k + 1) * chunk, t.nrow)); });
 }
 
 }  // namespace

@@ -13,6 +13,7 @@
 
 #include "sld_common.h"
 #include "sld_tables.h"
+#include "sld_threads.h"
 
 namespace sld {
 namespace {
@@ -224,13 +225,8 @@ void build_tables(double rcut_max, bool magmom, HostTables& t) {
     unsigned nt = std::thread::hardware_concurrency();
     if (nt == 0) nt = 1;
     if (nt > 16) nt = 16;
-    std::vector<std::thread> th;
-    int chunk = (kNInput + nt - 1) / nt;
-    for (unsigned k = 0; k < nt; ++k) {
-        int a = k * chunk, b = a + chunk < kNInput ? a + chunk : kNInput;
-        if (a < b) th.emplace_back(work, a, b);
-    }
-    for (auto& x : th) x.join();
+    const int chunk = (kNInput + (int)nt - 1) / (int)nt;
+    run_parts((int)nt, [&](int k) { work(k * chunk, std::min((k + 1) * chunk, kNInput)); });
 }
 
 std::shared_ptr<const HostTables> shared_tables(double rcut_max, bool magmom) {
