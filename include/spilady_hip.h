@@ -265,11 +265,16 @@ int sld_kernel_timing(sld_ctx* ctx, int* launches, double* total_ms);
  * No counterpart in the reference (its CUDA launches use fixed block sizes).
  * These are the block shapes of the kernels whose results do not depend on
  * them: every reduction inside them sums per wavefront, so a trajectory is
- * bitwise the same under any valid shapes. */
+ * bitwise the same under any valid shapes. spin_block, spin_lanes and
+ * sweep_block once counted other things, and the default sweep_block was 64:
+ * shapes stored then are still accepted, with the same results, but should be
+ * tuned anew (the diffusion of 2,000,000 atoms takes twice as long with 64
+ * threads a tile as with 256). */
 typedef struct {
     int spin_block;        /* core_ds sweep level: 16 times the most cells a wave takes; 32, 64 or 128 */
     int sweep_block;       /* core_dTe diffusion: threads of a tile's workgroup (twice as many on meshes of
-                              up to 512 tiles); 64, 128 or 256 */
+                              up to 512 tiles, always 512 where the mesh is one tile of up to 1,024
+                              cells); 64, 128 or 256 */
     int force_block;       /* force/energy: threads (four per atom) per block; 64, 128 or 256 */
     int nbuild_cells;      /* neighbour build: link cells (one wave each) per block; 1, 2 or 4 */
     int temperature_block; /* calculate_temperature: threads (8 per cell) per block; 64, 128 or 256 */

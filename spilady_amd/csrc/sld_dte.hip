@@ -349,9 +349,11 @@ __global__ __launch_bounds__(256) void k_dte_finish(Mesh M, const double* E, con
 // 8^3 333 (621), of 10^3 479 (615). From there on the relaxations, two and more a
 // thread, are worth more compute units: 11^3 936 and 942, 12^3 744 and 636, so
 // the line is at kDteSmall cells. (The relaxation as a function of its own, to
-// spare scalar registers, made the levels slower: 885 us at 7^3.)
-__global__ __launch_bounds__(512) void k_dte_small(DteTiles S, Mesh M, double h, double px, double py, double pz,
-                                                   int nloop) {
+// spare scalar registers, made the levels slower: 885 us at 7^3.) Always 512
+// threads: 128, which sweep_block = 64 once gave, made a call of 10^3 cells 1,088
+// us where a launch a level had taken 1,045; 256 are as good below 300 cells only.
+__global__ __launch_bounds__(kDteSmallBlock) void k_dte_small(DteTiles S, Mesh M, double h, double px, double py,
+                                                              double pz, int nloop) {
     extern __shared__ double sT[];
     __shared__ double sp[kDteSmall / 64];
     const int t = threadIdx.x, B = blockDim.x, lane = t & 63;

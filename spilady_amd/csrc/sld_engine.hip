@@ -544,8 +544,8 @@ int do_dTe_launches(sld_ctx* c, double dt) {
     if (c->dte_small) {
         hipEvent_t* ev = timing_slot(c, "k_dte_sweep");  // the sweeps' name for all meshes
         if (ev) (void)hipEventRecord(ev[0], c->stream);
-        hipLaunchKernelGGL(k_dte_small, dim3(1), dim3(2 * c->shapes.sweep_block), 32 * kDteSmall, c->stream, c->dte[0], M,
-                           h, px, py, pz, nloop);
+        hipLaunchKernelGGL(k_dte_small, dim3(1), dim3(kDteSmallBlock), 32 * kDteSmall, c->stream, c->dte[0], M, h, px,
+                           py, pz, nloop);
         HIPCHK(c, hipGetLastError());
         if (ev) (void)hipEventRecord(ev[1], c->stream);
         return SLD_OK;

@@ -146,6 +146,7 @@ struct DteSweepArgs {
 };
 // cells of a mesh that one workgroup sweeps on its own: 32 bytes of LDS a cell
 constexpr int kDteSmall = 1024;
+constexpr int kDteSmallBlock = 512;
 __global__ void k_dte_small(DteTiles S, Mesh M, double h, double px, double py, double pz, int nloop);
 template <int U>
 __global__ void k_dte_sweep(DteTiles S, DteSweepArgs A);
