@@ -257,7 +257,11 @@ int sld_last_step_timing(sld_ctx* ctx, double* total_ms);
 /* Bracket every launch of the kernel named `kernel` (e.g. "k_force"; "" or
  * NULL turns it off) with HIP events on the context's stream; after each
  * sld_step, sld_kernel_timing returns the launches seen and their summed
- * device time over that call. */
+ * device time over that call. "k_dte_sweep" takes the sweeps of a core_dTe
+ * sub-step as one span; on an electron mesh of up to 1,024 cells a whole
+ * core_dTe call is one launch, relaxations included, which answers to
+ * "k_dte_sweep" and to its own name, "k_dte_small": the two kinds of span do
+ * not compare. */
 int sld_time_kernel(sld_ctx* ctx, const char* kernel);
 int sld_kernel_timing(sld_ctx* ctx, int* launches, double* total_ms);
 

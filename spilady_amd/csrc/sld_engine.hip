@@ -542,7 +542,9 @@ int do_dTe_launches(sld_ctx* c, double dt) {
                  c->phys.spinlang};
     const double px = pref / h0.dx2, py = pref / h0.dy2, pz = pref / h0.dz2;
     if (c->dte_small) {
-        hipEvent_t* ev = timing_slot(c, "k_dte_sweep");  // the sweeps' name for all meshes
+        // under its own name and the sweeps', which a caller may time on any mesh
+        hipEvent_t* ev = timing_slot(c, "k_dte_small");
+        if (!ev) ev = timing_slot(c, "k_dte_sweep");
         if (ev) (void)hipEventRecord(ev[0], c->stream);
         hipLaunchKernelGGL(k_dte_small, dim3(1), dim3(kDteSmallBlock), 32 * kDteSmall, c->stream, c->dte[0], M, h, px,
                            py, pz, nloop);
