@@ -301,8 +301,10 @@ int sld_set_shapes(sld_ctx* ctx, const sld_shapes* in);
  * call had not been made. best (may be NULL) receives the chosen shapes;
  * us (may be NULL, 21 entries: kernel-major in the order of sld_shapes, three
  * candidates each in ascending order) the device microseconds per step of
- * each candidate, 0 where the kernel did not run. Needs device memory for a
- * copy of the context's state while it runs. */
+ * each candidate, 0 where the kernel did not run. sweep_tail changes no launch:
+ * it is left as it is, and its three entries repeat the time of the chosen
+ * sweep_block. Needs device memory for a copy of the context's state while it
+ * runs. */
 int sld_autotune(sld_ctx* ctx, int steps, sld_shapes* best, double* us);
 
 /* ---- Parametric potential model and its parameter adjoint ----
