@@ -33,7 +33,6 @@ struct LevelSet {
     std::vector<int> cells;   // cells grouped by level
     std::vector<int> off;     // level offsets (size nlev + 1)
     int* d_cells = nullptr;
-    int* d_off = nullptr;
     int nlev() const { return (int)off.size() - 1; }
 };
 
@@ -1101,12 +1100,6 @@ int upload_vec(sld_ctx* c, T** d, const std::vector<T>& h) {
     return SLD_OK;
 }
 
-int upload_levels(sld_ctx* c, LevelSet& L) {
-    TRY(upload_vec(c, &L.d_cells, L.cells));
-    TRY(upload_vec(c, &L.d_off, L.off));
-    return SLD_OK;
-}
-
 // The tile schedules of the electron diffusion (single-system contexts).
 int upload_dte_schedules(sld_ctx* c) {
     const HostCells& hc = c->rh[0].hc;
@@ -1475,8 +1468,8 @@ int create_impl(sld_ctx* c, int nrep, const sld_params* params, const sld_atoms*
     HIPCHK(c, hipStreamSynchronize(c->stream));
     merge_levels(sf, c->reps, c->spin_fwd);
     merge_levels(sb, c->reps, c->spin_bwd);
-    TRY(upload_levels(c, c->spin_fwd));
-    TRY(upload_levels(c, c->spin_bwd));
+    TRY(upload_vec(c, &c->spin_fwd.d_cells, c->spin_fwd.cells));
+    TRY(upload_vec(c, &c->spin_bwd.d_cells, c->spin_bwd.cells));
     if (nrep == 1) TRY(upload_dte_schedules(c));
 
     // electron temperatures (map_cells.cpp:128-159)
