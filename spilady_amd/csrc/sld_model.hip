@@ -202,19 +202,30 @@ __device__ __forceinline__ Basis pair_basis(const ModelTab& M, int l) {
     return B;
 }
 
-// 6-point derivative at r near the knot, where the stencil sees it
-__device__ __forceinline__ double basis_knot(const Basis& B, double r) {
+// value and derivative at r near the knot, where the stencil sees it,
+// interpolated in the entries of the table
+__device__ __forceinline__ double2 basis_knot(const Basis& B, double step, double in_over_rmax, double r) {
     auto at = [&](double x) {
         const double d = fmax(B.R - x, 0.0);
         return d * d * fma(B.alpha, d, B.beta * x);
     };
-    const double dx = 1e-3 * r;
-    double q = __builtin_amdgcn_rcp(r);
-    q = fma(fma(-r, q, 1.0), q, q);
-    q = fma(fma(-r, q, 1.0), q, q);
-    const double s = 45.0 * (at(r + dx) - at(r - dx)) - 9.0 * (at(fma(2.0, dx, r)) - at(fma(-2.0, dx, r))) +
-                     (at(fma(3.0, dx, r)) - at(fma(-3.0, dx, r)));
-    return s * (q * (1000.0 / 60.0));
+    int n;
+    double ratio;
+    interp_index(r, in_over_rmax, n, ratio);
+    double2 out = make_double2(0.0, 0.0);
+#pragma unroll 1
+    for (int e = n - 1; e <= n; ++e) {
+        const double x = step * (double)(e + 1), dx = 1e-3 * x;
+        double q = __builtin_amdgcn_rcp(x);
+        q = fma(fma(-x, q, 1.0), q, q);
+        q = fma(fma(-x, q, 1.0), q, q);
+        const double s = 45.0 * (at(x + dx) - at(x - dx)) - 9.0 * (at(fma(2.0, dx, x)) - at(fma(-2.0, dx, x))) +
+                         (at(fma(3.0, dx, x)) - at(fma(-3.0, dx, x)));
+        const double w = e == n ? 1.0 - ratio : ratio;
+        out.x = fma(w, at(x), out.x);
+        out.y = fma(w, s * (q * (1000.0 / 60.0)), out.y);
+    }
+    return out;
 }
 
 // value and derivative of a pair spline that reaches the quintic bridge below 2,
@@ -225,41 +236,50 @@ __device__ __forceinline__ double2 basis_bridge(const double* bridge, int row0, 
     double ratio;
     interp_index(r, in_over_rmax, n, ratio);
     double2 out = make_double2(0.0, 0.0);
+    // one point after another: the points side by side would cost the whole
+    // kernel registers for this rare pair
+#pragma unroll 1
     for (int e = n - 1; e <= n; ++e) {
         const double x = step * (double)(e + 1);
-        double v[7];
-        for (int s = 0; s < 7; ++s) {
+        const double w = e == n ? 1.0 - ratio : ratio;
+        auto at = [&](int s) {
             const double xs = stencil_x(x, s), d = fmax(R - xs, 0.0);
-            v[s] = xs <= 1.8   ? 0.0
+            return xs <= 1.8   ? 0.0
                    : xs <= 2.0 ? bridge[(size_t)(e - row0) * kModelBridgeRow + 9 * s + 1 + k]
                                : d * d * d;
-        }
-        const double w = e == n ? 1.0 - ratio : ratio;
-        out.x += w * v[0];
-        out.y += w * stencil_deriv(v, x);
+        };
+        double sum = 0.0;
+#pragma unroll 1
+        for (int s = 1; s < 7; s += 2) sum += (s == 1 ? 45e0 : s == 3 ? -9e0 : 1e0) * (at(s) - at(s + 1));
+        out.x += w * at(0);
+        out.y += w * (sum / (60e0 * (x / 1000e0)));
     }
     return out;
 }
 
-// Value and derivative at r as a table of step h interpolates them: g + q g''
-// for a smooth g, with q = (r - x0)(x1 - r) / 2 between the entries x0 and x1.
-// Away from the knots the 6-point derivative of these cubics is their
-// derivative; near one q g'' (1e-11) is below the stencil's own rounding of the
-// knot and left out.
-__device__ __forceinline__ double2 basis_at(const ModelTab& M, const Basis& B, double r, double q) {
+// Value and derivative at r as a table of step h interpolates them. Away from
+// the knots the 6-point derivative of these cubics is their derivative, and the
+// table gives g + q g'' with q = (r - x0)(x1 - r) / 2 between the entries x0 and
+// x1. Near a knot or in the bridge (rest turns true, 0 returned) that is off by
+// 1e-11, and the entries themselves are evaluated: basis_rest.
+__device__ __forceinline__ double2 basis_smooth(const Basis& B, double r, double q, bool& rest) {
     double2 out = make_double2(0.0, 0.0);
+    rest = false;
     if (r * 0.9969 < B.R) {  // else every point of the stencil is past the knot
-        const double d = fmax(B.R - r, 0.0), g = 3.0 * B.alpha;
-        out.x = fma(q, fma(2.0 * g, d, B.beta * fma(-4.0, d, 2.0 * r)), d * d * fma(B.alpha, d, B.beta * r));
-        out.y = fma(q, fma(6.0, B.beta, -2.0 * g), d * fma(-g, d, B.beta * fma(-2.0, r, d)));
-        if (r * 1.0031 >= B.R) {
-            out.x = d * d * fma(B.alpha, d, B.beta * r);
-            out.y = basis_knot(B, r);
+        rest = r * 1.0031 >= B.R || (B.bridge >= 0 && r * 0.9969 <= 2.0);
+        if (!rest) {
+            const double d = B.R - r, g = 3.0 * B.alpha;
+            out.x = fma(q, fma(2.0 * g, d, B.beta * fma(-4.0, d, 2.0 * r)), d * d * fma(B.alpha, d, B.beta * r));
+            out.y = fma(q, fma(6.0, B.beta, -2.0 * g), d * fma(-g, d, B.beta * fma(-2.0, r, d)));
         }
-        if (__builtin_expect(B.bridge >= 0 && r * 0.9969 <= 2.0, 0))
-            out = basis_bridge(M.bridge, M.row0, B.bridge, B.R, M.step, M.in_over_rmax, r);
     }
     return out;
+}
+
+__device__ __forceinline__ double2 basis_rest(const ModelTab& M, const Basis& B, double r) {
+    if (B.bridge >= 0 && r * 0.9969 <= 2.0)
+        return basis_bridge(M.bridge, M.row0, B.bridge, B.R, M.step, M.in_over_rmax, r);
+    return basis_knot(B, M.step, M.in_over_rmax, r);
 }
 
 // adjoint, second pass: the kNParam components of grad_theta, in partial sums
@@ -271,9 +291,11 @@ __device__ __forceinline__ double2 basis_at(const ModelTab& M, const Basis& B, d
 // basis function it evaluates: a table of them has 512 bytes a lookup, 3 GB a
 // call at 262,144 atoms and as much as the memory gives (712 us, and 70 us and
 // 256 MB to build the table at every parameter change), and the arithmetic takes
-// 267 us; of 4,096 atoms 13 (119). A pair near some lane's knot costs its wave
-// the stencil, two of five rounds. 128 registers with seven spilled for four
-// waves a SIMD: 331 us with 145 and three.
+// 252 us; of 4,096 atoms 16 (119). The pairs near a lane's knot, one in 120, wait
+// for the end of the round: some lane of a wave has one in two of five pairs, but
+// a lane has one or two of its 16, and their two stencils in the pairs' order
+// would cost 355 us. Without waves' registers for the rare points in the bridge
+// it is 127 of them and four waves a SIMD.
 constexpr int kAdjWaves = 4;
 
 __global__ __launch_bounds__(64 * kAdjWaves, 4) void k_model_adjoint(ModelTab M, Phys P, Dev D, int per_block,
@@ -353,9 +375,18 @@ __global__ __launch_bounds__(64 * kAdjWaves, 4) void k_model_adjoint(ModelTab M,
             for (int q = 0; q < 6; ++q) sW[wave][q][lane] = w[q];
             wave_fence();
             const int left = min(nn - k0, 16);
+            unsigned later = 0;  // bit p: pair p near this lane's knot
             for (int p = 0; p < left; ++p) {
                 const int at = (lane & 48) + p;
-                const double2 b = basis_at(M, B, sR[wave][at], sQ[wave][at]);
+                bool rest;
+                const double2 b = basis_smooth(B, sR[wave][at], sQ[wave][at], rest);
+                acc += sW[wave][kind][at] * b.y;
+                val += sW[wave][3 + kind][at] * b.x;
+                later |= (unsigned)rest << p;
+            }
+            for (; later; later &= later - 1) {
+                const int at = (lane & 48) + __builtin_ctz(later);
+                const double2 b = basis_rest(M, B, sR[wave][at]);
                 acc += sW[wave][kind][at] * b.y;
                 val += sW[wave][3 + kind][at] * b.x;
             }
