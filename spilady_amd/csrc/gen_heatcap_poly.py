@@ -10,7 +10,8 @@ With x = bT and y = bE/3 = log cosh x:
   acosh(e^y)   = sqrt(2y) * Gy(y)      Gy analytic, nearest singularities y = +-i pi
 Each factor is fitted by Chebyshev interpolation in 60-digit arithmetic
 (mpmath.chebyfit) on [0, S]; the degree is the smallest whose fit is below
-2^-56 relative. The script then evaluates each double-precision Horner form
+2^-56 relative. Gy is also written out in E itself, T(E) = sqrt(E) P(E), its
+first coefficient in two doubles: a rounding of it would be one of every T(E). The script then evaluates each double-precision Horner form
 against mpmath on a dense grid and prints the largest relative error.
 
 Run: python3 spilady_amd/csrc/gen_heatcap_poly.py  (rewrites heatcap_poly.h)
@@ -24,6 +25,7 @@ mp.mp.dps = 60
 X_MAX = 1.25                      # bT <= 1.25, i.e. T <= 6250 K
 Y_MAX = 0.75                      # bE/3 <= 0.75 (log cosh 1.25 = 0.636)
 TARGET = mp.mpf(2) ** -56
+K_BOLTZ = 8.617343e-5             # eV/K, kBoltz of sld_common.h
 
 
 def q_fn(s):                      # log cosh(x) / x^2 at s = x^2
@@ -57,7 +59,7 @@ def fit(f, hi):
     for n in range(4, 40):
         poly, err = mp.chebyfit(f, [0, hi], n + 1, error=True)
         if err / abs(f(hi)) < TARGET and err / abs(f(mp.mpf(0))) < TARGET:
-            return [float(c) for c in reversed(poly)], n   # lowest degree first
+            return list(reversed(poly)), n   # lowest degree first
     raise RuntimeError("no fit")
 
 
@@ -78,11 +80,19 @@ def check(name, c, f_full, arg, hi):
     print(f"{name}: degree {len(c) - 1}, max relative error {worst:.2e} on (0, {hi}]")
 
 
+def doubles(c):
+    return [float(v) for v in c]
+
+
 def main():
     cq, nq = fit(q_fn, mp.mpf(X_MAX) ** 2)
     cr, nr = fit(r_fn, mp.mpf(X_MAX) ** 2)
     ck, nk = fit(k_fn, mp.mpf(X_MAX) ** 2)
     cg, ng = fit(g_fn, mp.mpf(Y_MAX))
+    b = mp.mpf(2e-4 / K_BOLTZ)       # kCeB, as the kernels hold it
+    cp = [c * mp.sqrt(2 * b / 3) / b * (b / 3) ** k for k, c in enumerate(cg)]
+    lo = float(cp[0] - mp.mpf(float(cp[0])))
+    cq, cr, ck, cg, cp = map(doubles, (cq, cr, ck, cg, cp))
     check("log cosh x", cq, lambda c, x: x * x * horner(c, x * x), lambda x: mp.log(mp.cosh(x)), X_MAX)
     check("tanh x", cr, lambda c, x: x * horner(c, x * x), mp.tanh, X_MAX)
     check("x coth x", ck, lambda c, x: horner(c, x * x), lambda x: x * mp.coth(x), X_MAX)
@@ -96,10 +106,12 @@ def main():
     with open(out, "w") as fh:
         fh.write("// Generated by gen_heatcap_poly.py: Chebyshev fits (lowest degree first) of\n"
                  "// log cosh(x)/x^2, tanh(x)/x and x coth(x) in s = x^2 on [0, %r], and of\n"
-                 "// acosh(e^y)/sqrt(2y) in y on [0, %r], each below 2^-56 relative.\n"
+                 "// acosh(e^y)/sqrt(2y) in y on [0, %r], each below 2^-56 relative; kEeToTe: the\n"
+                 "// last as T(E)/sqrt(E) in E, kEeToTeLo what its first coefficient lacks.\n"
                  "#pragma once\n\nnamespace sld {\n\n" % (X_MAX * X_MAX, Y_MAX))
         fh.write(f"constexpr double kPolyXMax = {X_MAX!r};\nconstexpr double kPolyYMax = {Y_MAX!r};\n")
-        fh.write(arr("kLogCoshQ", cq) + arr("kTanhR", cr) + arr("kXCothX", ck) + arr("kAcoshExpG", cg))
+        fh.write(arr("kLogCoshQ", cq) + arr("kTanhR", cr) + arr("kXCothX", ck) + arr("kAcoshExpG", cg)
+                 + arr("kEeToTe", cp) + f"constexpr double kEeToTeLo = {lo!r};\n")
         fh.write("\n}  // namespace sld\n")
     print("wrote", out)
 

@@ -23,7 +23,6 @@ namespace sld {
 // ok turns false outside the fitted temperatures or for |u| > 1/4 (NaN
 // included).
 constexpr Poly<13> kRelaxK = scaled(kXCothX, 1.0, kCeB* kCeB);     // K(x^2) in T^2
-constexpr Poly<18> kTeToEe = scaled(kLogCoshQ, 3.0 * kCeB, kCeB* kCeB);  // E(T) / T^2 in T^2
 constexpr double kPolyT2Max = kPolyXMax * kPolyXMax / (kCeB * kCeB);
 // (e^u - 1) / u for |u| <= 1/4: the next term is 2^-24 / 13! = 1e-17
 constexpr double kExpm1[12] = {1.0,           1.0 / 2.0,      1.0 / 6.0,       1.0 / 24.0,
@@ -71,11 +70,11 @@ __device__ __forceinline__ double dte_relax_steps(double e0, double dE, double g
     for (int k = 0; k < n; ++k) {
         if (k > 0) e = (e + dE) + dE;
         ok = ok && e <= kPolyEMax && e >= 1e-200;
-        T = sqrt_normal(e) * horner2(kEeToTe.c, e);
+        T = ee_to_te_fit(e);
         T = rk4(T, [&](double x) { return relax_fast(g, x, ok); });
         const double t = T * T;
         ok = ok && t <= kPolyT2Max;
-        e = t * horner2(kTeToEe.c, t);
+        e = te_to_ee_fit(t);
     }
     if (__builtin_expect(!ok, 0)) {
         e = e0;
