@@ -378,13 +378,15 @@ __global__ __launch_bounds__(256) void k_fp(Tables T, Dev D) {
 //
 // What bounds it is the instruction stream, 1,970 a wave of 16 atoms, with three
 // waves a SIMD (158 registers) to hide the rows' latency; 1.5 GB come from beyond
-// the L2s. 2 M atoms 862 us, where a lane an atom, which loaded all of a pair by
+// the L2s. 2 M atoms 870 us, where a lane an atom, which loaded all of a pair by
 // itself, ten lines, and had eight pairs in flight to hide it, took 1,283 and
 // 3.8 GB; 64 x 16,000 atoms 636 (878), 250,000 atoms 109 (155), 2,000 13 (37).
 // Tried at 2 M atoms against 893 us on the same clock: rows of 64 bytes with J in
 // a table of its own 967, entries of 32 bytes that are not stored twice 1,000,
 // loads straight to LDS instead of register moves 970, no loads ahead 1,021, 128
-// registers with spills 1,840.
+// registers with spills 1,840. |s_i| |s_j| is the root of the squares' product, as
+// the one-body terms' squares: the rounded lengths' product (862 us) carries a
+// common rounding of them into every pair's energy.
 __global__ __launch_bounds__(256) void k_force(Tables T, Phys P, Dev D) {
     const int lb = xcd_block((4 * D.N + blockDim.x - 1) / blockDim.x);
     if (lb < 0) return;
@@ -396,8 +398,8 @@ __global__ __launch_bounds__(256) void k_force(Tables T, Phys P, Dev D) {
     const Box b = R.box;
     const double4 ri4 = D.r[i];
     const double3 ri = d3(ri4);
-    const double4 si4 = D.s[i];
-    const double3 si = d3(si4);
+    const double3 si = d3(D.s[i]);
+    const double si_sq = sq3(si);
     const double fpi = ri4.w;
     double3 f = make_double3(0.0, 0.0, 0.0);
     double pe = 0.0, me = 0.0, me0 = 0.0;
@@ -426,7 +428,7 @@ __global__ __launch_bounds__(256) void k_force(Tables T, Phys P, Dev D) {
         quad_transpose(x, j);
         quad_transpose(y, j);
         const double3 sj = make_double3(x[2], y[2], x[3]);
-        const double fpj = y[1], sj_len = y[3];
+        const double fpj = y[1];
         double rsq, inv, ratio;
         int n0;
         const double3 rij = min_image_sq(b, sub3(ri, make_double3(x[0], y[0], x[1])), rsq);
@@ -457,7 +459,7 @@ __global__ __launch_bounds__(256) void k_force(Tables T, Phys P, Dev D) {
             pe += 0.5 * c[2];
         }
         if (mag) {
-            const double sdot = dot3(si, sj), stimes = si4.w * sj_len;
+            const double sdot = dot3(si, sj), stimes = sqrt_any(si_sq * sq3(sj));
             const double Jh = lerp(qJ, ratio) / 2.0;
             dudr += -c[3] * (sdot - stimes);
             me0 += Jh * stimes;
@@ -483,7 +485,6 @@ __global__ __launch_bounds__(256) void k_force(Tables T, Phys P, Dev D) {
         m1 = quad_sum(m1);
         m2 = quad_sum(m2);
     }
-    const double si_sq = sq3(si);
     // one-body terms (calculate_force_energy_CPU.cpp:196-215)
     int n0;
     double ratio;
