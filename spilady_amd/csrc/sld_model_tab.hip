@@ -9,10 +9,10 @@
 //
 // Every value is evaluated in the order of the forms' definition with no
 // contraction, so a table entry is the host's to the rounding of exp and log
-// (the ZBL core and F(rho)) and of a cube. The quintic bridge (1.8 < r <= 2)
-// cancels terms of 1e5 down to 1, so there the powers' last bit would show:
-// its theta-independent polynomials come from the host (ModelBridge), one
-// value for each of a row's seven stencil points.
+// (the ZBL core and F(rho)). The quintic bridge (1.8 < r <= 2) cancels terms of
+// 1e5 down to 1, so there the powers' last bit would show: its theta-independent
+// polynomials come from the host (ModelBridge), one value for each of a row's
+// seven stencil points.
 #include <hip/hip_runtime.h>
 
 #include "sld_kernels.h"
@@ -23,15 +23,16 @@
 
 namespace sld {
 
-__device__ __forceinline__ double cube_knot(double R, double r) {
-    const double d = R - r;
-    return r < R ? d * d * d : 0e0;
+// d^3 rounded once, as pow(d, 3) is: the splines' terms cancel to a hundredth of
+// the largest, and the stencil divides what is left by 1e-3
+__device__ __forceinline__ double cube(double d) {
+    const double p = d * d;
+    return fma(p, d, fma(d, d, -p) * d);
 }
 
-__device__ __forceinline__ double cube_j(double r, double rc) {
-    const double q = 1.0 - r / rc;
-    return r < rc ? q * q * q : 0e0;
-}
+__device__ __forceinline__ double cube_knot(double R, double r) { return r < R ? cube(R - r) : 0e0; }
+
+__device__ __forceinline__ double cube_j(double r, double rc) { return r < rc ? cube(1.0 - r / rc) : 0e0; }
 
 // DD05.cpp:45-62
 __device__ __forceinline__ double zbl(double r, double as) {
