@@ -85,14 +85,17 @@ void fill_bridge(double rmax, ModelBridge& t) {
 
 std::shared_ptr<const ModelBridge> model_bridge(double rcut_max) {
     static std::mutex mu;
-    static std::vector<std::pair<double, std::shared_ptr<const ModelBridge>>> cache;
+    static std::vector<std::pair<double, std::shared_ptr<const ModelBridge>>> cache;  // the last used first
     std::lock_guard<std::mutex> lock(mu);
-    for (auto& e : cache)
-        if (e.first == rcut_max) return e.second;
-    auto t = std::make_shared<ModelBridge>();
-    fill_bridge(rcut_max, *t);
-    cache.emplace_back(rcut_max, t);
-    return t;
+    auto it = std::find_if(cache.begin(), cache.end(), [&](const auto& e) { return e.first == rcut_max; });
+    if (it == cache.end()) {
+        auto t = std::make_shared<ModelBridge>();
+        fill_bridge(rcut_max, *t);
+        if ((int)cache.size() == kModelBridges) cache.pop_back();
+        it = cache.emplace(cache.end(), rcut_max, std::move(t));
+    }
+    std::rotate(cache.begin(), it, it + 1);
+    return cache.front().second;
 }
 
 void model_default_params(double* th) {

@@ -37,7 +37,9 @@ struct ModelBridge {
     int row0 = 0, nrow = 0;
     std::vector<double> q;  // [nrow][7][9]
 };
-// Built on the host (16 threads) once per cutoff and process.
+// Built on the host (up to 16 threads, about 50 ms on 8 and 26 MB); the last
+// kModelBridges cutoffs stay with the process, older ones with their contexts.
+constexpr int kModelBridges = 4;
 std::shared_ptr<const ModelBridge> model_bridge(double rcut_max);
 
 // What the device needs to fill the tables at theta.
