@@ -127,12 +127,14 @@ __global__ __launch_bounds__(256) void k_dte_ab(double h, Mesh M, double* partia
 // last update is that value up to one rounding.
 //
 // A sweep is a chain of up to 20 dependent cell updates whatever the mesh
-// size. A launch per level cost 3.5 us each; here a level costs one LDS round
-// trip, the update's FP64 chain and a barrier, 600 cycles or 0.25 us, of which
-// neither the number of waves nor the lists' loads are a part any more (7^3
-// cells, 33 levels of both sweeps: 14.2 us a launch, 15.7 with the lists
-// requested one level ahead, whose hand-over waited for them, and a branch per
-// lane for temperatures outside the fit; 33 x 25 x 10 cells 12.6 and 14.2).
+// size, and the tile with the longest chain ends the launch: at 69^3 and 23^3
+// cells most tiles have 8 levels, the last few 18, in either sweep. A launch per
+// level cost 3.5 us each; here a level costs one LDS round trip, the update's FP64
+// chain and a barrier, 600 cycles or 0.25 us, of which neither the number of waves
+// nor the lists' loads are a part any more (33 x 25 x 10 cells, 28 levels of both
+// sweeps: 12.6 us a launch, 14.2 with the lists requested one level ahead, whose
+// hand-over waited for them, and a branch per lane for temperatures outside the
+// fit; 7^3 cells, 40 levels, in a launch of their own 14.2 and 15.7).
 // The energy partials are one per tile: its cells in slot order, 64 at a
 // time, so the sum does not depend on the block size.
 constexpr int kAhead = 4;  // levels
@@ -228,7 +230,7 @@ __global__ __launch_bounds__(512) void k_dte_sweep(DteTiles S, DteSweepArgs A) {
     // a thread's first U slots t, t + B, ... are in flight together, and their
     // cells stay in registers until the results go out: 8 where a thread has
     // that many (69^3 cells: 11.1 us a launch instead of 12.2), 4 where the
-    // other four would be loads for nothing (7^3: 14.1 and 14.8; 40^3 8.2 and 9.3)
+    // other four would be loads for nothing (40^3: 8.2 and 9.3)
     int32_t c[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) c[u] = slot[min(t + u * B, T.nslot - 1)];
@@ -343,9 +345,9 @@ __global__ __launch_bounds__(256) void k_dte_finish(Mesh M, const double* E, con
 
 // A whole core_dTe call of a small mesh, one tile, in one workgroup: the
 // temperatures, energies and sources stay in LDS for all sub-steps. A sub-step
-// takes its levels (0.29 us each), one relaxation a thread and two sums, and no
-// launch: a call of 7^3 cells 692 us where two launches a sub-step took 970, of
-// 8^3 333 (621), of 10^3 479 (615). From there on the relaxations, two and more a
+// takes its levels (0.25 us each, 40 at 7^3 and 8 at even sides), one relaxation a thread and two sums, and no
+// launch: a call of 7^3 cells 680 us where two launches a sub-step took 970, of
+// 8^3 297 (621), of 10^3 442 (615). From there on the relaxations, two and more a
 // thread, are worth more compute units: 11^3 936 and 942, 12^3 744 and 636, so
 // the line is at kDteSmall cells. (The relaxation as a function of its own, to
 // spare scalar registers, made the levels slower: 885 us at 7^3.) Always 512

@@ -34,7 +34,7 @@ __global__ __launch_bounds__(256) void k_reduce(const double* partials, int nblk
 // Per-replica sums: block r of the grid (1,024 threads) reduces partial rows
 // [seg[r], seg[r+1]) into out[r * kScal + out_off + k], in an order fixed by
 // the row count alone: thread t adds rows t, t + 1024, ... in turn, each wave
-// sums by shuffles, thread 0 adds the 16 wave sums in order.
+// sums its lanes (wave_sum), thread 0 adds the 16 wave sums in order.
 __global__ __launch_bounds__(1024) void k_reduce_seg(const double* partials, const int* seg, int nk, double* out,
                                                      int out_off) {
     constexpr int KG = 4;  // components summed together
@@ -621,7 +621,8 @@ __device__ __forceinline__ LanRows landau_rows(const Tables& T, double rho) {
     int n0;
     double ratio;
     interp_index(rho, T.in_over_rhomax, n0, ratio);
-    // columns A..D sit 16-byte aligned in 128-byte rows
+    // rows of 80 bytes: columns A..D are 16-byte aligned, in one line or two
+    static_assert(kRhoStride % 2 == 0 && H_A % 2 == 0, "double2 loads");
     const double2* lo = reinterpret_cast<const double2*>(T.rhotab + (size_t)(n0 - 1) * kRhoStride + H_A);
     const double2* hi = reinterpret_cast<const double2*>(T.rhotab + (size_t)n0 * kRhoStride + H_A);
     const double2 l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
@@ -636,8 +637,8 @@ __device__ __forceinline__ LanRows landau_rows(const Tables& T, double rho) {
 // (calculate_spin_CPU.cpp:118-121), interpolated as the reference does. The
 // density changes once a step (calculate_rho); the four spin sweeps, the
 // force pass and the temperature and energy observables in between read the
-// coefficients from here, 32 contiguous bytes per atom, instead of two
-// 128-byte table rows each.
+// coefficients from here, 32 contiguous bytes per atom, instead of two table
+// rows of 80 bytes each.
 __global__ __launch_bounds__(256) void k_landau(Tables T, Dev D) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= D.N || D.arep[i] < 0) return;

@@ -30,7 +30,7 @@
 namespace sld {
 namespace {
 
-// knots of the density and pair splines (DD05.cpp:26-37,70-85), as in sld_model_tab.hip
+// knots of the density and pair splines (DD05.cpp:26-37,70-85), as in sld_model_device.h
 const double kFR[6] = {3.0, 2.8666666666666666, 2.7333333333333333, 2.6, 2.4, 2.3};
 const double kVR[8] = {4.1, 3.8, 3.5, 3.2, 2.9, 2.6, 2.4, 2.3};
 

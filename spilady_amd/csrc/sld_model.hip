@@ -294,8 +294,8 @@ __device__ __forceinline__ double2 basis_rest(const ModelTab& M, const Basis& B,
 // 252 us; of 4,096 atoms 16 (119). The pairs near a lane's knot, one in 120, wait
 // for the end of the round: some lane of a wave has one in two of five pairs, but
 // a lane has one or two of its 16, and their two stencils in the pairs' order
-// would cost 355 us. Without waves' registers for the rare points in the bridge
-// it is 127 of them and four waves a SIMD.
+// would cost 355 us. 127 registers for four waves a SIMD, with the points in the
+// bridge one after another (side by side 12 spilled, 275 us).
 constexpr int kAdjWaves = 4;
 
 __global__ __launch_bounds__(64 * kAdjWaves, 4) void k_model_adjoint(ModelTab M, Phys P, Dev D, int per_block,

@@ -4,8 +4,8 @@
 // stencil behind every second one, 16 threads) took about 250 ms of every
 // parameter change, against 2 ms for the whole loss gradient of 262,144
 // atoms. The rows are independent, so one thread makes one row and the rows
-// leave through LDS as contiguous lines: 192 MB in 83
-// us (the r values 64, the rho table 19).
+// leave through LDS as contiguous lines: 192 MB in 85
+// us (the r values 66, the rho table 19).
 //
 // Every value is evaluated in the order of the forms' definition with no
 // contraction, so a table entry is the host's to the rounding of exp and log
