@@ -376,11 +376,11 @@ __global__ __launch_bounds__(256) void k_fp(Tables T, Dev D) {
 // instruction touches 32 or 16 lines and not 64; the quad then swaps the pieces
 // by register moves (the columns after the interpolation).
 //
-// What bounds it is the instruction stream, 1,970 a wave of 16 atoms, with three
-// waves a SIMD (158 registers) to hide the rows' latency; 1.5 GB come from beyond
+// What bounds it is the instruction stream, 2,044 a wave of 16 atoms, with three
+// waves a SIMD (160 registers) to hide the rows' latency; 1.5 GB come from beyond
 // the L2s. 2 M atoms 870 us, where a lane an atom, which loaded all of a pair by
 // itself, ten lines, and had eight pairs in flight to hide it, took 1,283 and
-// 3.8 GB; 64 x 16,000 atoms 636 (878), 250,000 atoms 109 (155), 2,000 13 (37).
+// 3.8 GB; 64 x 16,000 atoms 640 (878), 250,000 atoms 108 (155), 2,000 13 (37).
 // Tried at 2 M atoms against 893 us on the same clock: rows of 64 bytes with J in
 // a table of its own 967, entries of 32 bytes that are not stored twice 1,000,
 // loads straight to LDS instead of register moves 970, no loads ahead 1,021, 128

@@ -124,12 +124,12 @@ __device__ __forceinline__ unsigned quad_or(unsigned v) {
 //
 // A walk that loads as it goes waits for memory once an atom and fetches a
 // neighbour's line again for every atom that reads it; here a launch waits
-// about four times in all. The update is a chain of 240 instructions, about 0.7
+// about four times in all. The update is a chain of 250 instructions, about 0.7
 // us for a wave on its own, so rounds count: cells of 9.3 atoms on average and
 // 16 at most need 6.1 and 9 of them, cells of 6.5 and 10 need 4.9 and 6.
 // At 27 cells a launch that leaves 3 us of launch, 2 of first loads, 1 of
-// gathering and 4 of rounds: 9.7 us where the walk atom by atom took 16.5. Of
-// 2 M atoms a level moves 108 MB in 31.1 us (39.5); registers are kept to 128 for
+// gathering and 4 of rounds: 10.0 us where the walk atom by atom took 16.5. Of
+// 2 M atoms a level moves 104 MB in 31.5 us (39.5); registers are kept to 128 for
 // four waves a SIMD, the atoms' own values loaded after the gathering (before
 // it: 150 registers, 1 us more at 64 x 16,000 atoms, 0.2 less at 2,000).
 
