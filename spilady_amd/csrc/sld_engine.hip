@@ -1976,6 +1976,31 @@ int autotune_body(sld_ctx* c, int steps, double* us) {
     }
     return read_flags(c);
 }
+
+// the parametric model's buffers and what of it does not depend on theta
+int model_buffers(sld_ctx* c, sld_ctx::Model& m) {
+    const int N = c->D.N;
+    m.bridge = model_bridge(c->prm.rcut_max);
+    TRY(upload_vec(c, &m.d_bridge, m.bridge->q));
+    TRY(dalloc(c, &m.d_r, (size_t)kNInput * kMRStride));
+    TRY(dalloc(c, &m.d_f, kNInput)); TRY(dalloc(c, &m.d_df, kNInput));
+    TRY(dalloc(c, &m.d_h, (size_t)kNInput * kMHStride));
+    std::vector<int> coff(c->R);
+    int tot = 0;
+    for (int r = 0; r < c->R; ++r) {
+        coff[r] = tot;
+        tot += c->reps[r].natom;
+    }
+    m.ntot = tot;
+    TRY(upload_vec(c, &m.d_coff, coff));
+    TRY(dalloc(c, &m.d_rho, N)); TRY(dalloc(c, &m.d_fp, N)); TRY(dalloc(c, &m.d_Q, N));
+    TRY(dalloc(c, &m.d_F, (size_t)3 * tot)); TRY(dalloc(c, &m.d_H, (size_t)3 * tot));
+    TRY(dalloc(c, &m.d_gF, (size_t)3 * tot)); TRY(dalloc(c, &m.d_gH, (size_t)3 * tot));
+    TRY(dalloc(c, &m.d_gE, c->R)); TRY(dalloc(c, &m.d_E, (size_t)kScal * c->R));
+    TRY(dalloc(c, &m.d_grad, kNParam));
+    TRY(dalloc(c, &m.d_part, std::max((size_t)nblk(N, 256), (size_t)kNParam * kAdjBlocks)));
+    return SLD_OK;
+}
 }  // namespace
 
 extern "C" {
@@ -2044,30 +2069,18 @@ int sld_model_set_params(sld_ctx* c, const double* theta) {
         if (!std::isfinite(theta[k])) return set_err(c, SLD_ERR_ARG, "parameter %d is not finite", k);
     if (!(theta[P_JRC] > 0.0)) return set_err(c, SLD_ERR_ARG, "exchange cutoff must be positive");
     auto& m = c->model;
-    const int N = c->D.N;
     if (!m.d_r) {
-        TRY(no_throw(c, [&] {
-            m.bridge = model_bridge(c->prm.rcut_max);
-            return SLD_OK;
-        }));
-        TRY(upload_vec(c, &m.d_bridge, m.bridge->q));
-        TRY(dalloc(c, &m.d_r, (size_t)kNInput * kMRStride));
-        TRY(dalloc(c, &m.d_f, kNInput)); TRY(dalloc(c, &m.d_df, kNInput));
-        TRY(dalloc(c, &m.d_h, (size_t)kNInput * kMHStride));
-        std::vector<int> coff(c->R);
-        int tot = 0;
-        for (int r = 0; r < c->R; ++r) {
-            coff[r] = tot;
-            tot += c->reps[r].natom;
+        // all of it or nothing: what a failed call has got goes back, and the next starts anew
+        const size_t mark = c->allocs.size();
+        sld_ctx::Model made = m;
+        const int rc = no_throw(c, [&] { return model_buffers(c, made); });
+        if (rc != SLD_OK) {
+            for (; c->allocs.size() > mark; c->allocs.pop_back(), c->alloc_bytes.pop_back())
+                (void)hipFree(c->allocs.back());
+            (void)hipGetLastError();
+            return rc;
         }
-        m.ntot = tot;
-        TRY(upload_vec(c, &m.d_coff, coff));
-        TRY(dalloc(c, &m.d_rho, N)); TRY(dalloc(c, &m.d_fp, N)); TRY(dalloc(c, &m.d_Q, N));
-        TRY(dalloc(c, &m.d_F, (size_t)3 * tot)); TRY(dalloc(c, &m.d_H, (size_t)3 * tot));
-        TRY(dalloc(c, &m.d_gF, (size_t)3 * tot)); TRY(dalloc(c, &m.d_gH, (size_t)3 * tot));
-        TRY(dalloc(c, &m.d_gE, c->R)); TRY(dalloc(c, &m.d_E, (size_t)kScal * c->R));
-        TRY(dalloc(c, &m.d_grad, kNParam));
-        TRY(dalloc(c, &m.d_part, std::max((size_t)nblk(N, 256), (size_t)kNParam * kAdjBlocks)));
+        m = made;
     }
     const ModelCoef mc = model_coef(theta, c->prm.rcut_max, *m.bridge);
     LAUNCH(c, k_model_tab_r, nblk(kNInput - 1, 255), 256, mc, (const double*)m.d_bridge, m.d_r, m.d_f, m.d_df);
