@@ -27,7 +27,7 @@ def test_no_thread_to_be_had(check):
     assert a.stdout.count("\n") == 3 and b.stdout == a.stdout
 
 
-@pytest.mark.skipif((os.cpu_count() or 1) < 2, reason="one processor: no thread is made")
+@pytest.mark.skipif(len(os.sched_getaffinity(0)) < 2, reason="one processor: no thread is made")
 def test_no_memory_inside_a_thread(check):
     r = check("memory")
     assert r.returncode == 0 and r.stdout == "bad_alloc in the caller\n", (r.returncode, r.stdout, r.stderr)
